@@ -11,6 +11,8 @@
 #include <atomic>
 #include <chrono>
 #include <functional>
+#include <map>
+#include <mutex>
 #include <thread>
 #include <cmath>
 #include <cstdio>
@@ -62,6 +64,54 @@ using Mask = std::array<uint64_t, kMaxTPL>;
 
 static std::vector<Chunk> make_chunks(int nsusp, const std::vector<int64_t> &susp_sph_off,
                                       const std::vector<int64_t> &off, std::vector<int> *seg_off);
+
+// A rows x cols matrix in the layout the transform GEMMs read (transforms.hip):
+// [48-row block][its three 16-row blocks rb][group of 16 columns][lane][4], lane
+// i + 16 k holding columns 4k .. 4k + 3 of the group in row 3 (16 w + i) + rb
+// (points: matrices on grid values) or 48 w + 16 rb + i; zero outside.
+template <typename T, typename F>
+static std::vector<T> pack_gemm(int rows, int cols, bool points, F at) {
+    const int nblk = (rows + 47) / 48, ngrp = (cols + 15) / 16;
+    std::vector<T> m(size_t(nblk) * 3 * ngrp * 256, T(0));
+    size_t o = 0;
+    for (int w = 0; w < nblk; w++)
+        for (int rb = 0; rb < 3; rb++)
+            for (int g = 0; g < ngrp; g++)
+                for (int lane = 0; lane < 64; lane++) {
+                    const int i = lane & 15, c0 = 16 * g + 4 * (lane >> 4);
+                    const int r = points ? 3 * (16 * w + i) + rb : 48 * w + 16 * rb + i;
+                    for (int q = 0; q < 4; q++, o++)
+                        if (r < rows && c0 + q < cols) m[o] = (T)at(r, c0 + q);
+                }
+    return m;
+}
+
+// Those matrices depend on the orders alone: kept per process, like the tables
+// they are made from, so that a handle per time step does not lay them out again.
+template <typename T, typename F>
+static const std::vector<T> &packed_gemm(const std::vector<int> &key, F make) {
+    static std::mutex mu;
+    static std::map<std::vector<int>, std::unique_ptr<std::vector<T>>> cache;
+    std::lock_guard<std::mutex> lock(mu);
+    auto &e = cache[key];
+    if (!e) e = std::make_unique<std::vector<T>>(make());
+    return *e;
+}
+
+static void gemm_view(GemmTables &g, int p, const void *tab, int rows, int cols) {
+    g.view.tab[p] = tab;
+    g.view.nblk[p] = (rows + 47) / 48;
+    g.view.ngrp[p] = (cols + 15) / 16;
+    g.view.max_blk = std::max(g.view.max_blk, g.view.nblk[p]);
+}
+static void upload_gemm(GemmTables &g, int p, int rows, int cols, const std::vector<double> &m) {
+    g.d[p].upload(m);
+    gemm_view(g, p, g.d[p].p, rows, cols);
+}
+static void upload_gemm(GemmTables &g, int p, int rows, int cols, const std::vector<float> &m) {
+    g.f[p].upload(m);
+    gemm_view(g, p, g.f[p].p, rows, cols);
+}
 
 // ---------------------------------------------------------------------------
 // Operator set-up: SphereSTKSHOperator::setupDOF / setupFMM / setupNearEval
@@ -253,6 +303,13 @@ Operator::Operator(int nsusp, const int *counts, const double *pos, const double
             tl.push_back(SphTile{order_[ts[i]], i, j - i, 0});
             i = j;
         }
+        std::vector<int64_t> bo(tl.size() + 1, 0);
+        for (size_t i = 0; i < tl.size(); i++)
+            bo[i + 1] = bo[i] + (int64_t)kTileSph * body_cols(grid_points(tl[i].p));
+        d_body_off_.upload(bo);
+        geom_.body_off = d_body_off_.p;
+        body64_.alloc(std::max<int64_t>(bo.back(), 1));
+        tiles_ = tl;
         d_tile_sph_.upload(ts);
         d_tiles_.upload(tl);
         geom_.ntiles = (int)tl.size();
@@ -263,8 +320,13 @@ Operator::Operator(int nsusp, const int *counts, const double *pos, const double
     for (int p : order_) used[p] = true;
     for (int p = 0; p <= kMaxOrder; p++)
         if (used[p]) {
-            d_anal_[p].upload(sh_tables(p).anal);
-            geom_.anal[p] = d_anal_[p].p;
+            const ShTables &t = sh_tables(p);
+            const int rows = 6 * t.Q;
+            upload_gemm(anal_, p, rows, 3 * t.npts, packed_gemm<double>(std::vector<int>{p, -1}, [&] {
+                            return pack_gemm<double>(rows, 3 * t.npts, false,
+                                                     [&](int r, int c) { return t.anal[size_t(c) * rows + r]; });
+                        }));
+            max_pts_ = std::max(max_pts_, t.npts);
         }
 
     // segmented-vector chunks (one segment per suspension)
@@ -352,15 +414,17 @@ Operator::Operator(int nsusp, const int *counts, const double *pos, const double
                 po0(pt_off_.begin(), pt_off_.begin() + s0 + 1);
             const std::vector<Runs> r0(runs_fine_.begin(), runs_fine_.begin() + s0);
             build_far_lists(lists_fine_, b0, so0, po0, po0, r0, 1, split, kWantItems);
-            if (lists_fine_.split > 1) lists_fine_.part.alloc(size_t(lists_fine_.split) * 3 * npts_);
+            if (lists_fine_.pairs > 0.0) lists_fine_.part.alloc(size_t(lists_fine_.split) * 3 * npts_);
             srcm_.alloc(std::max<int64_t>(4 * (std::min(ncopy_, kMultiCols) + 1) * pt_off_[s0], 8));
         } else {
             build_far_lists(lists_fine_, nsusp_, susp_sph_off_, pt_off_, pt_off_, runs_fine_, tpl, split, kWantItems);
+            lists_fine_.slots();
         }
     }
     ls32_.tpl = ls64_.tpl = lsc_.tpl = tpl;
 
     src64_.alloc(std::max<int64_t>(8 * npts_, 8));
+    launch_pack_src_f64(npts_, d_coords_.p, d_w_.p, nullptr, src64_.p, stream_);
     coef_.alloc(std::max<int64_t>(coef_off_[nsph_], 1));
     rec_.alloc(std::max<int64_t>(rec_off_[nsph_], 1));
     tmp_.alloc(std::max<int64_t>(3 * npts_, 1));
@@ -379,13 +443,13 @@ Operator::Operator(int nsusp, const int *counts, const double *pos, const double
 // warms caches and code), within a time budget so that very large problems
 // keep the default shapes instead of spending minutes tuning.
 double Operator::time_far_pass(FarLists &L, int prec, const void *src, const double *tcoords, const double *tnorms,
-                               const float *trg32, const Chunk *chunks, int nchunks, double *out) {
+                               const float *trg32) {
     hipEvent_t a, b;
     SPHSTK_HIP(hipEventCreate(&a));
     SPHSTK_HIP(hipEventCreate(&b));
-    far_run(L, 0, prec, src, tcoords, tnorms, trg32, chunks, nchunks, 1.0, out, nullptr);
+    far_slots(L, 0, prec, src, tcoords, tnorms, trg32, 1.0, nullptr);
     SPHSTK_HIP(hipEventRecord(a, stream_));
-    far_run(L, 0, prec, src, tcoords, tnorms, trg32, chunks, nchunks, 1.0, out, nullptr);
+    far_slots(L, 0, prec, src, tcoords, tnorms, trg32, 1.0, nullptr);
     SPHSTK_HIP(hipEventRecord(b, stream_));
     SPHSTK_HIP(hipEventSynchronize(b));
     float ms = 0.f;
@@ -399,11 +463,9 @@ void Operator::autotune_fine(double &budget_s) {
     if (nsph_ == 0) return;
     launch_fill(3 * npts_, 1.0, tmp_.p, stream_);
     launch_pack_src_f64(npts_, d_coords_.p, d_w_.p, tmp_.p, src64_.p, stream_);
-    DevBuf<double> out;
-    out.alloc(std::max<int64_t>(3 * npts_, 1));
     auto timed = [&](FarLists &L) {
-        const double ms = time_far_pass(L, 0, src64_.p, d_coords_.p, d_norms_.p, nullptr, chunks_.p,
-                                        (int)chunks_.n, out.p);
+        L.slots();
+        const double ms = time_far_pass(L, 0, src64_.p, d_coords_.p, d_norms_.p, nullptr);
         budget_s -= 2e-3 * ms;
         return ms;
     };
@@ -435,29 +497,18 @@ void Operator::autotune_fine(double &budget_s) {
 
 // FP32 inner operator: targets per lane of all its level lists, timed as one
 // multi-level pass.
-void Operator::far_levels_pass(LevelSet &S, const double *in, double *out) {
-    launch_pack_src_f32(npts_, d_coords_.p, d_w_.p, in, src32_.p, stream_);
-    far_levels(S, 0, 1.0, in, out, nullptr, nullptr, nullptr);
-}
-
 void Operator::autotune_inner(double &budget_s) {
     if (nsph_ == 0 || !multi_level_) return;
-    if (!trg32_.p) {
-        trg32_.alloc(8 * std::max<int64_t>(npts_, 1));
-        src32_.alloc(8 * std::max<int64_t>(npts_, 1));
-        launch_pack_trg_f32(npts_, d_coords_.p, d_norms_.p, trg32_.p, stream_);
-    }
     launch_fill(3 * npts_, 1.0, tmp_.p, stream_);
-    DevBuf<double> out;
-    out.alloc(std::max<int64_t>(3 * npts_, 1));
+    pack(tmp_.p, 1);
     auto timed = [&]() {
         auto t0 = std::chrono::steady_clock::now();
-        far_levels_pass(ls32_, tmp_.p, out.p);
+        far_levels(ls32_, 0, 1.0, nullptr, nullptr, nullptr);
         hipEvent_t a, b;
         SPHSTK_HIP(hipEventCreate(&a));
         SPHSTK_HIP(hipEventCreate(&b));
         SPHSTK_HIP(hipEventRecord(a, stream_));
-        far_levels_pass(ls32_, tmp_.p, out.p);
+        far_levels(ls32_, 0, 1.0, nullptr, nullptr, nullptr);
         SPHSTK_HIP(hipEventRecord(b, stream_));
         SPHSTK_HIP(hipEventSynchronize(b));
         float ms = 0.f;
@@ -1046,6 +1097,7 @@ void Operator::ensure_levels(LevelSet &S) {
     {
         PhaseTimer pm("  mid-range lists");
         build_far_lists(S.mid, nsusp_, susp_sph_off_, pt_off_, pt_off_, mid, S.tpl, 0, kWantItems);
+        S.mid.slots();
     }
     S.levels.clear();
     std::vector<std::vector<int64_t>> level_off(nlev);
@@ -1054,13 +1106,11 @@ void Operator::ensure_levels(LevelSet &S) {
         std::vector<int64_t> &off = level_off[l];
         off.assign(nsph_ + 1, 0);
         std::vector<int64_t> off_by_sph(nsph_);
-        int maxpts = 0;
         for (int r = 0; r < nsph_; r++) {
             const int s = perm[r];
             const int p = order_[s], pc = lorder(l, p);
             off[r + 1] = off[r] + grid_points(pc);
             off_by_sph[s] = off[r];
-            maxpts = std::max(maxpts, std::max(grid_points(p), grid_points(pc)));
         }
         const int64_t nc = off[nsph_];
         std::vector<double> cc(3 * nc), cn(3 * nc), cw(nc);
@@ -1078,47 +1128,25 @@ void Operator::ensure_levels(LevelSet &S) {
             }
         }
         L->npts = nc;
-        L->max_pts = maxpts;
         L->d_off_by_sph.upload(off_by_sph);
         L->coords.upload(cc);
         L->norms.upload(cn);
         L->w.upload(cw);
-        std::vector<bool> used(kMaxOrder + 1, false);
-        for (int p : order_) used[p] = true;
-        for (int p = 0; p <= kMaxOrder; p++)
-            if (used[p]) {
-                const Resample &rs = resample_tables(p, lorder(l, p));
-                L->d_down[p].upload(rs.down);
-                L->d_up[p].upload(rs.up);
-                L->down.M[p] = L->d_down[p].p;
-                L->down.nin[p] = rs.n;
-                L->down.nout[p] = rs.nc;
-                L->up.M[p] = L->d_up[p].p;
-                L->up.nin[p] = rs.nc;
-                L->up.nout[p] = rs.n;
-                if (!S.fp64) {
-                    L->d_down32[p].upload(std::vector<float>(rs.down.begin(), rs.down.end()));
-                    L->d_up32[p].upload(std::vector<float>(rs.up.begin(), rs.up.end()));
-                    L->down.M32[p] = L->d_down32[p].p;
-                    L->up.M32[p] = L->d_up32[p].p;
-                }
-            }
-        L->down.fp32 = L->up.fp32 = !S.fp64;
         PhaseTimer pl("  level lists");
         build_far_lists(L->lists, nsusp_, susp_sph_off_, off, off, lvl[l], S.tpl, 0, kWantItems);
-        std::vector<int> dummy;
-        L->chunks.upload(make_chunks(nsusp_, susp_sph_off_, off, &dummy));
-        L->sv.alloc(std::max<int64_t>(3 * nc, 1));
-        L->tv.alloc(std::max<int64_t>(3 * nc, 1));
+        L->lists.slots();
         if (S.fp64) {
             L->src64.alloc(std::max<int64_t>(8 * nc, 8));
+            launch_pack_src_f64(nc, L->coords.p, L->w.p, nullptr, L->src64.p, stream_);
         } else {
             L->src32.alloc(std::max<int64_t>(8 * nc, 8));
             L->trg32.alloc(std::max<int64_t>(8 * nc, 8));
+            launch_pack_src_f32(nc, L->coords.p, L->w.p, nullptr, L->src32.p, stream_);
             launch_pack_trg_f32(nc, L->coords.p, L->norms.p, L->trg32.p, stream_);
         }
         S.levels.push_back(std::move(L));
     }
+    level_transforms(S);
     S.agg.reset();
     // keep the cells some target uses, renumbered in order (runs stay sorted)
     std::vector<int> cell_new(ncell, -1);
@@ -1185,7 +1213,6 @@ void Operator::ensure_levels(LevelSet &S) {
         A->P.upload(Pcm);
         A->rho.upload(crho);
         A->susp.upload(csusp);
-        A->chk_u.alloc((size_t)ncell * m);
         // check points of cell c x the fine grids of its members (sphere index space)
         std::vector<int64_t> chk_off(ncell + 1), eq_off(ncell + 1);
         std::vector<Runs> chk_runs(ncell);
@@ -1200,18 +1227,91 @@ void Operator::ensure_levels(LevelSet &S) {
         }
         build_far_lists(A->chk_lists, nsusp_, susp_cell_off, chk_off, pt_off_, chk_runs, 1, 0, kWantItems, nullptr,
                         &susp_sph_off_);
-        A->chk_chunks.upload(make_chunks(nsusp_, susp_cell_off, chk_off, nullptr));
+        A->chk_lists.slots();
         A->check_pairs = A->chk_lists.pairs;
         for (int i = 0; i < 2; i++) {
             std::vector<Runs> runs(nsph_);
             for (int r = 0; r < nsph_; r++) runs[r] = crun[r][i];
             build_far_lists(A->lists[i], nsusp_, susp_sph_off_, level_off[2 + i], eq_off, runs, S.tpl, 0, kWantItems,
                             nullptr, &susp_cell_off);
+            A->lists[i].slots();
             A->pairs += A->lists[i].pairs;
         }
         S.agg = std::move(A);
     }
+    for (int l = 0; l < nlev; l++) {
+        FarLevel &L = *S.levels[l];
+        LevelViews &V = S.views;
+        V.off[l] = L.d_off_by_sph.p;
+        V.w[l] = L.w.p;
+        V.src[l] = S.fp64 ? (void *)L.src64.p : (void *)L.src32.p;
+        V.stride[l] = 3 * L.npts;
+        V.part[l][0] = L.lists.part.p;
+        V.nslot[l][0] = L.lists.nslot();
+        const FarLists *C = S.agg && l >= 2 ? &S.agg->lists[l - 2] : nullptr;
+        V.part[l][1] = C ? C->part.p : nullptr;
+        V.nslot[l][1] = C ? C->nslot() : 0;
+    }
     S.ready = true;
+}
+
+// The resampling matrices between the fine grids and all levels of a set as one
+// matrix per order: levels stacked by rows (down) and by columns (up), so that
+// each direction is one launch (four or six levels had one launch each way per
+// level, each too small to fill the GPU: 1024 spheres p=12, FP32 set, 8
+// launches of 138 us per apply).
+void Operator::level_transforms(LevelSet &S) {
+    std::vector<bool> used(kMaxOrder + 1, false);
+    for (int p : order_) used[p] = true;
+    LevelViews &V = S.views;
+    V.nlev = S.nlev;
+    S.max_lev_pts = 0;
+    for (int p = 0; p <= kMaxOrder; p++) {
+        if (!used[p]) continue;
+        std::vector<const Resample *> rs;
+        std::vector<int> key{p};
+        for (int l = 0; l < S.nlev; l++) {
+            const int pc = S.order[l] < 0 ? level_order(l, p) : std::min(p, S.order[l]);
+            rs.push_back(&resample_tables(p, pc));
+            key.push_back(pc);
+            V.first[p][l + 1] = V.first[p][l] + rs[l]->nc;
+        }
+        const int n = rs[0]->n, nl = V.first[p][S.nlev];
+        S.max_lev_pts = std::max(S.max_lev_pts, nl);
+        std::vector<int> lev_of(nl);
+        for (int l = 0; l < S.nlev; l++) std::fill(lev_of.begin() + V.first[p][l], lev_of.begin() + V.first[p][l + 1], l);
+        auto down = [&](int r, int c) {
+            const int l = lev_of[r / 3];
+            return rs[l]->down[size_t(c) * 3 * rs[l]->nc + r - 3 * V.first[p][l]];
+        };
+        auto up = [&](int r, int c) {
+            const int l = lev_of[c / 3];
+            return rs[l]->up[size_t(c - 3 * V.first[p][l]) * 3 * n + r];
+        };
+        std::vector<int> kd = key, ku = key;
+        kd.push_back(-1);
+        ku.push_back(-2);
+        auto put = [&](auto zero) {
+            using T = decltype(zero);
+            upload_gemm(S.down, p, 3 * nl, 3 * n,
+                        packed_gemm<T>(kd, [&] { return pack_gemm<T>(3 * nl, 3 * n, true, down); }));
+            upload_gemm(S.up, p, 3 * n, 3 * nl,
+                        packed_gemm<T>(ku, [&] { return pack_gemm<T>(3 * n, 3 * nl, true, up); }));
+        };
+        if (S.fp64)
+            put(0.0);
+        else
+            put(0.f);
+    }
+    std::vector<int64_t> bo(tiles_.size() + 1, 0);
+    for (size_t i = 0; i < tiles_.size(); i++)
+        bo[i + 1] = bo[i] + (int64_t)kTileSph * body_cols(V.first[tiles_[i].p][S.nlev]);
+    S.d_body_off.upload(bo);
+    V.body_off = S.d_body_off.p;
+    if (S.fp64)
+        S.body64.alloc(std::max<int64_t>(bo.back(), 1));
+    else
+        S.body32.alloc(std::max<int64_t>(bo.back(), 1));
 }
 
 void Operator::harvest_events() {
@@ -1237,69 +1337,64 @@ void Operator::far_run(FarLists &L, int kind, int prec, const void *src, const d
     if (L.split > 1) launch_slot_reduce(out, L.part.p, L.split, 3 * L.ntrg, chunks, nchunks, active, stream_);
 }
 
-// Multi-level far field (the packed fine-grid sources of `in` are already in
-// src64_ or src32_): each level resamples `in` to its grid, sums its shell of
-// sphere pairs there and interpolates the result back onto the fine grid; the
-// pairs closer than the first level are summed on the fine grid.  ev_a and
-// ev_b bracket the pair sums only.
-void Operator::far_levels(LevelSet &S, int kind, double coef, const double *in, double *out, const int *active,
-                          hipEvent_t ev_a, hipEvent_t ev_b) {
+// The pair sums of one list into its partial-sum slots.
+void Operator::far_slots(FarLists &L, int kind, int prec, const void *src, const double *tcoords, const double *tnorms,
+                         const float *trg32, double coef, const int *active) {
+    if (L.pairs == 0.0) return; // e.g. a level that no sphere pair reaches
+    launch_far(kind, prec, L.tpl, src, tcoords, tnorms, trg32, L.ntrg, L.ngroups, L.order.p, L.groups.p, L.iv.p,
+               active, L.part.p, coef, 0, stream_, &L != &lists_fine_);
+}
+
+// Multi-level far field of the densities that pack() left in body64_ or body32_
+// and src64_ or src32_: the sources are resampled to all levels, each list sums
+// its shell of sphere pairs into its slots; the pairs closer than the first
+// level are summed on the fine grid.  levels_up interpolates the level fields
+// back.  ev_a and ev_b bracket the pair sums only.
+void Operator::far_levels(LevelSet &S, int kind, double coef, const int *active, hipEvent_t ev_a, hipEvent_t ev_b) {
     ensure_levels(S);
-    const int prec = S.fp64 ? 0 : 1;
-    for (auto &L : S.levels) {
-        launch_resample(geom_, L->down, d_pt_off_.p, L->d_off_by_sph.p, in, L->sv.p, 0, active, stream_, L->max_pts);
-        if (S.fp64)
-            launch_pack_src_f64(L->npts, L->coords.p, L->w.p, L->sv.p, L->src64.p, stream_);
-        else
-            launch_pack_src_f32(L->npts, L->coords.p, L->w.p, L->sv.p, L->src32.p, stream_);
-        launch_fill(3 * L->npts, 0.0, L->tv.p, stream_);
-    }
+    launch_levels_down(geom_, S.down.view, S.fp64, S.fp64 ? (const void *)body64_.p : (const void *)body32_.p, S.views,
+                       active, stream_);
     CellAgg *A = S.agg.get();
     if (A) {
         // check velocities of each cell's raw fine-grid sources (single layer,
         // FP32 pairs, FP64 sums), then the equivalent point forces
-        launch_fill((int64_t)A->ncell * 3 * A->E->Kc, 0.0, A->chk_u.p, stream_);
-        far_run(A->chk_lists, 1, 1, src32_.p, nullptr, nullptr, A->chk32.p, A->chk_chunks.p, (int)A->chk_chunks.n,
-                1.0 / (8.0 * kPi), A->chk_u.p, active);
-        launch_equiv_forces(A->ncell, A->E->K, A->E->Kc, A->P.p, A->chk_u.p, A->rho.p, A->susp.p,
-                            active, A->eq32.p, stream_);
+        far_slots(A->chk_lists, 1, 1, src32_.p, nullptr, nullptr, A->chk32.p, 1.0 / (8.0 * kPi), active);
+        launch_equiv_forces(A->ncell, A->E->K, A->E->Kc, A->P.p, A->chk_lists.part.p, A->chk_lists.nslot(),
+                            3 * A->chk_lists.ntrg, A->rho.p, A->susp.p, active, A->eq32.p, stream_);
     }
     if (ev_a) SPHSTK_HIP(hipEventRecord(ev_a, stream_));
     if (A)
-        for (int i = 0; i < 2; i++) {
-            FarLevel &L = *S.levels[2 + i];
-            far_run(A->lists[i], kind, 1, A->eq32.p, nullptr, nullptr, L.trg32.p, L.chunks.p, (int)L.chunks.n, coef,
-                    L.tv.p, active);
-        }
+        for (int i = 0; i < 2; i++)
+            far_slots(A->lists[i], kind, 1, A->eq32.p, nullptr, nullptr, S.levels[2 + i]->trg32.p, coef, active);
     for (auto &L : S.levels) {
         if (S.fp64)
-            far_run(L->lists, kind, 0, L->src64.p, L->coords.p, L->norms.p, nullptr, L->chunks.p, (int)L->chunks.n,
-                    coef, L->tv.p, active);
+            far_slots(L->lists, kind, 0, L->src64.p, L->coords.p, L->norms.p, nullptr, coef, active);
         else
-            far_run(L->lists, kind, 1, L->src32.p, nullptr, nullptr, L->trg32.p, L->chunks.p, (int)L->chunks.n, coef,
-                    L->tv.p, active);
+            far_slots(L->lists, kind, 1, L->src32.p, nullptr, nullptr, L->trg32.p, coef, active);
     }
     if (S.fp64)
-        far_run(S.mid, kind, prec, src64_.p, d_coords_.p, d_norms_.p, nullptr, chunks_.p, (int)chunks_.n, coef, out,
-                active);
+        far_slots(S.mid, kind, 0, src64_.p, d_coords_.p, d_norms_.p, nullptr, coef, active);
     else
-        far_run(S.mid, kind, prec, src32_.p, nullptr, nullptr, trg32_.p, chunks_.p, (int)chunks_.n, coef, out,
-                active);
+        far_slots(S.mid, kind, 1, src32_.p, nullptr, nullptr, trg32_.p, coef, active);
     if (ev_b) SPHSTK_HIP(hipEventRecord(ev_b, stream_));
-    for (auto &L : S.levels)
-        launch_resample(geom_, L->up, L->d_off_by_sph.p, d_pt_off_.p, L->tv.p, out, 1, active, stream_, L->max_pts);
+    launch_pack_levels(geom_, S.fp64, S.views, S.fp64 ? (void *)S.body64.p : (void *)S.body32.p, S.max_lev_pts, stream_);
+}
+
+// out += the level fields of the last far_levels of this set, on the fine grids
+void Operator::levels_up(LevelSet &S, double *out, const int *active) {
+    launch_levels_up(geom_, S.up.view, S.fp64, S.fp64 ? (const void *)S.body64.p : (const void *)S.body32.p, S.views, out,
+                     active, stream_);
 }
 
 // FP64 far field of ncopy identical copies of a set of suspensions (several
 // right-hand sides on one geometry), with the first copy's work lists.  The
 // traction sum is computed once per pair for blocks of up to 8 copies
 // (k_far_trac_multi_f64); the single layer one copy at a time on the first
-// copy's geometry.
-void Operator::far_copies(int kind, double coef, const double *in, double *out, const int *active, hipEvent_t ev_a) {
+// copy's geometry.  All copies' sums go to the slots of the list.
+void Operator::far_copies(int kind, double coef, const double *in, const int *active, hipEvent_t ev_a) {
     FarLists &L = lists_fine_;
     const int b0 = nsusp_ / ncopy_;
     const int64_t n0 = npts_ / ncopy_, col = 3 * n0;
-    const bool split = L.split > 1;
     if (ev_a) SPHSTK_HIP(hipEventRecord(ev_a, stream_));
     if (L.pairs == 0.0) return;
     if (kind == 0) {
@@ -1307,18 +1402,15 @@ void Operator::far_copies(int kind, double coef, const double *in, double *out, 
             const int nc = std::min(kMultiCols, ncopy_ - c0);
             launch_far_trac_multi(nc, n0, d_coords_.p, d_norms_.p, d_w_.p, in + c0 * col, col, srcm_.p, L.ngroups,
                                   L.order.p, L.groups.p, L.iv.p, active ? active + c0 * b0 : nullptr, b0,
-                                  (split ? L.part.p : out) + c0 * col, coef, split ? 0 : 1, 3 * npts_, stream_);
+                                  L.part.p + c0 * col, coef, 0, 3 * npts_, stream_);
         }
-        if (split) launch_slot_reduce(out, L.part.p, L.split, 3 * npts_, chunks_.p, (int)chunks_.n, active, stream_);
         return;
     }
-    const int nch0 = seg_chunk_off_host_[b0];
     for (int c = 0; c < ncopy_; c++) {
         const int *act = active ? active + c * b0 : nullptr;
         launch_pack_src_f64(n0, d_coords_.p, d_w_.p, in + c * col, src64_.p, stream_);
-        launch_far(kind, 0, L.tpl, src64_.p, d_coords_.p, d_norms_.p, nullptr, L.ntrg, L.ngroups, L.order.p,
-                   L.groups.p, L.iv.p, act, split ? L.part.p : out + c * col, coef, split ? 0 : 1, stream_);
-        if (split) launch_slot_reduce(out + c * col, L.part.p, L.split, 3 * L.ntrg, chunks_.p, nch0, act, stream_);
+        launch_far(kind, 0, L.tpl, src64_.p, d_coords_.p, d_norms_.p, nullptr, npts_, L.ngroups, L.order.p,
+                   L.groups.p, L.iv.p, act, L.part.p + c * col, coef, 0, stream_);
     }
 }
 
@@ -1343,10 +1435,27 @@ bool Operator::outer_levels_pay() {
     return outer_pay_ == 1;
 }
 
-// Far field of `in` into out (accumulating).  FP64: fine grid, direct sum over
-// all far pairs.  FP32: multi-level (fine for mid-range pairs, coarser grids
-// with distance) unless disabled, in which case the FP32 direct sum.
-void Operator::far(int kind, int prec, double coef, const double *in, double *out, const int *active) {
+void Operator::ensure_fp32_grid() {
+    if (trg32_.p) return;
+    trg32_.alloc(8 * std::max<int64_t>(npts_, 1));
+    src32_.alloc(8 * std::max<int64_t>(npts_, 1));
+    body32_.alloc(body64_.n);
+    launch_pack_trg_f32(npts_, d_coords_.p, d_norms_.p, trg32_.p, stream_);
+    launch_pack_src_f32(npts_, d_coords_.p, d_w_.p, nullptr, src32_.p, stream_);
+}
+
+void Operator::pack(const double *in, int prec) {
+    const bool f32 = prec == 1 || prec == 3;
+    if (f32) ensure_fp32_grid();
+    launch_pack_body(geom_, in, body64_.p, f32 && multi_level_ ? body32_.p : nullptr,
+                     (prec == 0 || prec == 2) && ncopy_ == 1 ? src64_.p : nullptr, f32 ? src32_.p : nullptr, max_pts_,
+                     stream_);
+}
+
+// FP64: fine grid, direct sum over all far pairs.  FP32: multi-level (fine for
+// mid-range pairs, coarser grids with distance) unless disabled, in which case
+// the FP32 direct sum.
+FarSum Operator::far(int kind, int prec, double coef, const double *in, const int *active, LevelSet **levels) {
     const bool timing = (flags_ & 1) != 0 && !capturing_;
     EvPair ev{};
     if (timing) {
@@ -1360,97 +1469,76 @@ void Operator::far(int kind, int prec, double coef, const double *in, double *ou
         ev.kind = kind;
         ev.prec = prec;
     }
-    if (ncopy_ > 1) {
+    LevelSet *S = nullptr;
+    if (ncopy_ > 1)
         SPHSTK_REQUIRE(prec == 0, "several right-hand sides on one geometry are solved in FP64 only");
-        far_copies(kind, coef, in, out, active, timing ? ev.a : nullptr);
-    } else if (prec == 0) {
-        launch_pack_src_f64(npts_, d_coords_.p, d_w_.p, in, src64_.p, stream_);
-        if (timing) SPHSTK_HIP(hipEventRecord(ev.a, stream_));
-        far_run(lists_fine_, kind, 0, src64_.p, d_coords_.p, d_norms_.p, nullptr, chunks_.p, (int)chunks_.n, coef,
-                out, active);
-    } else if (prec == 2 && !outer_levels_pay()) {
-        // the coarse levels would save too few pair evaluations: direct FP64 sum
-        launch_pack_src_f64(npts_, d_coords_.p, d_w_.p, in, src64_.p, stream_);
-        if (timing) SPHSTK_HIP(hipEventRecord(ev.a, stream_));
-        far_run(lists_fine_, kind, 0, src64_.p, d_coords_.p, d_norms_.p, nullptr, chunks_.p, (int)chunks_.n, coef,
-                out, active);
-    } else if (prec == 2) {
-        launch_pack_src_f64(npts_, d_coords_.p, d_w_.p, in, src64_.p, stream_);
-        far_levels(ls64_, kind, coef, in, out, active, timing ? ev.a : nullptr, timing ? ev.b : nullptr);
-        if (timing) {
-            pending_.push_back(ev);
-            timing_done_ = true;
-        }
-    } else {
+    else if (prec == 2)
+        S = outer_levels_pay() ? &ls64_ : nullptr; // else too few pair evaluations saved: direct FP64 sum
+    else if (prec != 0 && multi_level_) {
         if (prec == 1) wait_inner_levels();
-        if (!trg32_.p) {
-            trg32_.alloc(8 * std::max<int64_t>(npts_, 1));
-            src32_.alloc(8 * std::max<int64_t>(npts_, 1));
-            launch_pack_trg_f32(npts_, d_coords_.p, d_norms_.p, trg32_.p, stream_);
-        }
-        launch_pack_src_f32(npts_, d_coords_.p, d_w_.p, in, src32_.p, stream_);
-        if (multi_level_) {
-            far_levels(prec == 3 ? lsc_ : ls32_, kind, coef, in, out, active, timing ? ev.a : nullptr,
-                       timing ? ev.b : nullptr);
-            if (timing) {
-                pending_.push_back(ev);
-                timing_done_ = true;
-            }
-        } else {
-            if (timing) SPHSTK_HIP(hipEventRecord(ev.a, stream_));
-            far_run(lists_fine_, kind, 1, src32_.p, nullptr, nullptr, trg32_.p, chunks_.p, (int)chunks_.n, coef, out,
-                    active);
-        }
+        S = prec == 3 ? &lsc_ : &ls32_;
+    }
+    *levels = S;
+    FarLists &L = S ? S->mid : lists_fine_;
+    if (S) {
+        far_levels(*S, kind, coef, active, timing ? ev.a : nullptr, timing ? ev.b : nullptr);
+    } else if (ncopy_ > 1) {
+        far_copies(kind, coef, in, active, timing ? ev.a : nullptr);
+    } else {
+        if (timing) SPHSTK_HIP(hipEventRecord(ev.a, stream_));
+        if (prec == 0 || prec == 2)
+            far_slots(L, kind, 0, src64_.p, d_coords_.p, d_norms_.p, nullptr, coef, active);
+        else
+            far_slots(L, kind, 1, src32_.p, nullptr, nullptr, trg32_.p, coef, active);
     }
     SPHSTK_HIP(hipGetLastError());
-    if (timing && !timing_done_) {
-        SPHSTK_HIP(hipEventRecord(ev.b, stream_));
+    if (timing) {
+        if (!S) SPHSTK_HIP(hipEventRecord(ev.b, stream_));
         pending_.push_back(ev);
+        if (pending_.size() > 64) harvest_events();
     }
-    timing_done_ = false;
-    if (timing && pending_.size() > 64) harvest_events();
+    return FarSum{L.part.p, L.nslot(), 3 * npts_};
 }
 
-// applyP2POP (cpp:262-485), accumulating into out.
-void Operator::p2p(const double *in, double *out, double cId, double cSL, double cTrac, int prec, const int *active) {
-    const bool doSL = std::fabs(cSL) > 1e-9, doT = std::fabs(cTrac) > 1e-9;
-    double cid = std::fabs(cId) > 1e-9 ? cId : 0.0;
-    if (!doSL && !doT) {
+// applyP2POP (cpp:262-485), accumulating into out (or, overwrite, the whole
+// operator with cLOP L).  Per kernel (traction, single layer): the self and near
+// terms (SH analysis, expansion, evaluation into scratch) run on the second
+// stream while the far field runs on the first; the gather into out waits for
+// both.
+void Operator::p2p(const double *in, double *out, double cId, double cSL, double cTrac, int prec, const int *active,
+                   bool overwrite, double cLOP) {
+    const bool on[2] = {std::fabs(cTrac) > 1e-9, std::fabs(cSL) > 1e-9};
+    double cid = std::fabs(cId) > 1e-9 ? cId : 0.0, clop = std::fabs(cLOP) > 1e-9 ? cLOP : 0.0;
+    if (nsph_ == 0) return;
+    if (!on[0] && !on[1]) {
+        if (overwrite) launch_fill(3 * npts_, 0.0, out, stream_);
         if (cid != 0.0) launch_identity(geom_, in, out, cid, active, stream_);
+        if (clop != 0.0) launch_lop(geom_, in, out, clop, active, stream_);
         return;
     }
-    if (nsph_ == 0) return;
-    if (doT && !capturing_) {
-        // the self and near terms (SH analysis, expansion, evaluation into
-        // scratch) on the second stream while the far field runs on the first;
-        // the gather into out waits for both
-        SPHSTK_HIP(hipEventRecord(ev_fork_, stream_));
-        SPHSTK_HIP(hipStreamWaitEvent(aux_, ev_fork_, 0));
-        launch_analysis(geom_, in, coef_.p, active, aux_, max_order_);
-        launch_expand(geom_, 1, coef_.p, rec_.p, active, aux_, max_order_);
-        launch_sheval_items(geom_, 1, rec_.p, items_.p, (int)items_.n, evscratch_.p, 0.0, cTrac, active, aux_,
+    const hipStream_t side = capturing_ ? stream_ : aux_;
+    pack(in, prec);
+    bool first = true;
+    for (int kind = 0; kind < 2; kind++) {
+        if (!on[kind]) continue;
+        if (side != stream_) {
+            SPHSTK_HIP(hipEventRecord(ev_fork_, stream_));
+            SPHSTK_HIP(hipStreamWaitEvent(side, ev_fork_, 0));
+        }
+        if (first) analyse(active, side);
+        const int mode = kind == 0 ? 1 : 0;
+        launch_expand(geom_, mode, coef_.p, rec_.p, active, side, max_order_);
+        launch_sheval_items(geom_, mode, rec_.p, items_.p, (int)items_.n, evscratch_.p, cSL, cTrac, active, side,
                             &src_items_);
-        SPHSTK_HIP(hipEventRecord(ev_join_, aux_));
-        far(0, prec, -3.0 / (4.0 * kPi) * cTrac, in, out, active);
-        SPHSTK_HIP(hipStreamWaitEvent(stream_, ev_join_, 0));
-        launch_sheval_gather(geom_, (int)items_.n, d_trg_slot_off_.p, d_trg_nsrc_.p, evscratch_.p, in, out, cid,
-                             active, stream_);
-        cid = 0.0;
-    } else {
-        launch_analysis(geom_, in, coef_.p, active, stream_, max_order_);
-    }
-    if (doT && capturing_) {
-        far(0, prec, -3.0 / (4.0 * kPi) * cTrac, in, out, active);
-        launch_expand(geom_, 1, coef_.p, rec_.p, active, stream_, max_order_);
-        launch_sheval(geom_, 1, rec_.p, items_.p, (int)items_.n, d_trg_slot_off_.p, d_trg_nsrc_.p, evscratch_.p, in,
-                      out, 0.0, cTrac, cid, active, stream_, &src_items_);
-        cid = 0.0;
-    }
-    if (doSL) {
-        far(1, prec, cSL / (8.0 * kPi), in, out, active);
-        launch_expand(geom_, 0, coef_.p, rec_.p, active, stream_, max_order_);
-        launch_sheval(geom_, 0, rec_.p, items_.p, (int)items_.n, d_trg_slot_off_.p, d_trg_nsrc_.p, evscratch_.p, in,
-                      out, cSL, 0.0, cid, active, stream_);
+        if (side != stream_) SPHSTK_HIP(hipEventRecord(ev_join_, side));
+        LevelSet *S = nullptr;
+        const FarSum f = far(kind, prec, kind == 0 ? -3.0 / (4.0 * kPi) * cTrac : cSL / (8.0 * kPi), in, active, &S);
+        if (side != stream_) SPHSTK_HIP(hipStreamWaitEvent(stream_, ev_join_, 0));
+        launch_sheval_gather(geom_, d_trg_slot_off_.p, d_trg_nsrc_.p, evscratch_.p, f, in, out, cid, clop,
+                             overwrite && first, active, stream_);
+        if (S) levels_up(*S, out, active);
+        cid = clop = 0.0;
+        first = false;
     }
     SPHSTK_HIP(hipGetLastError());
 }
@@ -1582,27 +1670,29 @@ void Operator::prepare_mixed(bool outer_levels, bool coarse) {
 void Operator::rigid_p2p(const double *force, const double *rho0, double *out, double cId, double cTrac) {
     if (nsph_ == 0) return;
     ensure_centre();
-    launch_analysis(geom_, rho0, coef_.p, nullptr, stream_, max_order_);
-    launch_pack_src_f64(npts_, d_coords_.p, d_w_.p, rho0, src64_.p, stream_);
+    pack(rho0, 0);
+    analyse(nullptr, stream_);
     far_run(lists_rv_mid_, 0, 0, src64_.p, d_coords_.p, d_norms_.p, nullptr, chunks_.p, (int)chunks_.n,
             -3.0 / (4.0 * kPi) * cTrac, out, nullptr);
     launch_far_rigid(d_coords_.p, d_norms_.p, d_pos_.p, force, d_rad_.p, npts_, lists_rigid_.ngroups,
                      lists_rigid_.order.p, lists_rigid_.groups.p, lists_rigid_.iv.p, out, cTrac, 1, stream_);
     launch_expand(geom_, 1, coef_.p, rec_.p, nullptr, stream_, max_order_);
-    launch_sheval(geom_, 1, rec_.p, items_.p, (int)items_.n, d_trg_slot_off_.p, d_trg_nsrc_.p, evscratch_.p, rho0, out,
-                  0.0, cTrac, cId, nullptr, stream_, &src_items_);
+    launch_sheval_items(geom_, 1, rec_.p, items_.p, (int)items_.n, evscratch_.p, 0.0, cTrac, nullptr, stream_,
+                        &src_items_);
+    launch_sheval_gather(geom_, d_trg_slot_off_.p, d_trg_nsrc_.p, evscratch_.p, FarSum{}, rho0, out, cId, 0.0, false,
+                         nullptr, stream_);
     SPHSTK_HIP(hipGetLastError());
 }
 
 void Operator::rigid_velocity(const double *rho, double inv_mu, double *vel) {
     if (nsph_ == 0) return;
     ensure_centre();
-    launch_analysis(geom_, rho, coef_.p, nullptr, stream_, max_order_);
+    pack(rho, 0);
+    analyse(nullptr, stream_);
     launch_expand(geom_, 0, coef_.p, rec_.p, nullptr, stream_, max_order_);
-    launch_fill(3 * npts_, 0.0, u_ns_.p, stream_);
-    launch_sheval(geom_, 0, rec_.p, items_.p, (int)items_.n, d_trg_slot_off_.p, d_trg_nsrc_.p, evscratch_.p, rho,
-                  u_ns_.p, 1.0, 0.0, 0.0, nullptr, stream_);
-    launch_pack_src_f64(npts_, d_coords_.p, d_w_.p, rho, src64_.p, stream_);
+    launch_sheval_items(geom_, 0, rec_.p, items_.p, (int)items_.n, evscratch_.p, 1.0, 0.0, nullptr, stream_);
+    launch_sheval_gather(geom_, d_trg_slot_off_.p, d_trg_nsrc_.p, evscratch_.p, FarSum{}, rho, u_ns_.p, 0.0, 0.0, true,
+                         nullptr, stream_);
     far_run(lists_rv_mid_, 1, 0, src64_.p, d_coords_.p, d_norms_.p, nullptr, chunks_.p, (int)chunks_.n,
             1.0 / (8.0 * kPi), u_ns_.p, nullptr);
     launch_rigid_avg(geom_, u_ns_.p, inv_mu, vel_ns_.p, stream_);
@@ -1617,9 +1707,7 @@ void Operator::lop(const double *in, double *out, double cLOP, const int *active
 }
 
 void Operator::apply_into(const double *in, double *out, int prec, const int *active) {
-    launch_fill(3 * npts_, 0.0, out, stream_);
-    p2p(in, out, c_[0], c_[1], c_[2], prec, active);
-    lop(in, out, c_[3], active);
+    p2p(in, out, c_[0], c_[1], c_[2], prec, active, true, c_[3]);
 }
 
 // The inner operator's apply as one HIP graph: captured on the first call (or
@@ -1684,7 +1772,8 @@ void Operator::apply(const double *X, double *Y, double alpha, double beta, int 
 // on the host.
 void Operator::pole_values(const double *in, double *out) {
     if (nsph_ == 0) return;
-    launch_analysis(geom_, in, coef_.p, nullptr, stream_, max_order_);
+    pack(in, -1);
+    analyse(nullptr, stream_);
     std::vector<double> coef(std::max<int64_t>(coef_off_[nsph_], 1));
     SPHSTK_HIP(hipMemcpyAsync(coef.data(), coef_.p, sizeof(double) * coef_off_[nsph_], hipMemcpyDeviceToHost,
                               stream_));
@@ -1709,7 +1798,8 @@ void Operator::pole_values(const double *in, double *out) {
 
 void Operator::project(double *inout) {
     if (nsph_ == 0) return;
-    launch_analysis(geom_, inout, coef_.p, nullptr, stream_, max_order_);
+    pack(inout, -1);
+    analyse(nullptr, stream_);
     launch_expand(geom_, 1, coef_.p, rec_.p, nullptr, stream_, max_order_);
     launch_synthesis(geom_, rec_.p, self_items_.p, (int)self_items_.n, inout, stream_);
     SPHSTK_HIP(hipGetLastError());
@@ -1756,7 +1846,8 @@ static std::vector<double> self_inverse_blocks() {
 void Operator::precondition(const double *in, double *out, const int *active) {
     if (nsph_ == 0) return;
     if (!self_inv_.p) self_inv_.upload(self_inverse_blocks());
-    launch_analysis(geom_, in, coef_.p, active, stream_, max_order_);
+    pack(in, -1);
+    analyse(active, stream_);
     launch_degree_blocks(geom_, coef_.p, self_inv_.p, active, stream_);
     launch_expand(geom_, 1, coef_.p, rec_.p, active, stream_, max_order_);
     launch_fill(3 * npts_, 0.0, out, stream_);

@@ -79,6 +79,11 @@ struct FarLists {
     int ngroups = 0, tpl = 1, split = 1;
     double pairs = 0.0; // algorithmic pairs per launch
     int64_t ntrg = 0;
+    // the slots as the consumers of the sum read them (a list without pairs has none)
+    void slots() {
+        if (pairs > 0.0) part.alloc(size_t(split) * 3 * ntrg);
+    }
+    int nslot() const { return pairs > 0.0 ? split : 0; }
 };
 
 // Half-open ranges [a, b) of sphere indices, sorted and disjoint.
@@ -102,16 +107,18 @@ void build_far_lists(FarLists &L, int nsusp, const std::vector<int64_t> &susp_sp
 // order, their geometry, resampling tables and work lists.
 struct FarLevel {
     int64_t npts = 0;
-    int max_pts = 0;
     DevBuf<int64_t> d_off_by_sph; // first level point of each sphere
-    DevBuf<double> coords, norms, w, sv, tv;
+    DevBuf<double> coords, norms, w;
     DevBuf<float> src32, trg32;
     DevBuf<double> src64;
-    DevBuf<Chunk> chunks;
-    DevBuf<double> d_down[kMaxOrder + 1], d_up[kMaxOrder + 1];
-    DevBuf<float> d_down32[kMaxOrder + 1], d_up32[kMaxOrder + 1]; // FP32 copies (FP32 level sets)
-    ResampleTabs down, up;
     FarLists lists;
+};
+
+// Device copies of one matrix per order in the layout of the transform GEMMs.
+struct GemmTables {
+    DevBuf<double> d[kMaxOrder + 1];
+    DevBuf<float> f[kMaxOrder + 1];
+    ShGemm view;
 };
 
 // Source-cell aggregation of the two coarsest FP32 levels (the treecode part
@@ -131,19 +138,17 @@ struct CellAgg {
     std::vector<int64_t> susp_cell_off; // first cell of each suspension
     DevBuf<float> chk32;              // check points as FP32 target records (zero normals)
     DevBuf<float> eq32;               // equivalent points as FP32 source records (forces per apply)
-    DevBuf<double> chk_u;             // check velocities, 3 Kc per cell
     DevBuf<double> P;                 // template fit, column-major (3K x 3Kc)
     DevBuf<double> rho;               // cell radius
     DevBuf<int> susp;                 // cell suspension
-    DevBuf<Chunk> chk_chunks;
     FarLists chk_lists;               // check points of a cell x the fine grids of its members
+                                      // (its slots: the check velocities, 3 Kc per cell)
     FarLists lists[2];                // level-2 / level-3 target grids x equivalent points
 };
 
 // A multi-level far field: fine-grid sums for the pairs closer than the first
 // level's separation (mid), then one coarser grid per separation shell.
 constexpr int kNumLevels = 4; // levels of the FP32 sets (source cells on their last two)
-constexpr int kMaxLevels = 6;
 struct LevelSet {
     int nlev = kNumLevels;   // levels in use
     double alo[kMaxLevels];  // separations (in units of R_s + R_t) where levels 0..nlev-1 start
@@ -152,6 +157,12 @@ struct LevelSet {
     int tpl = 1;             // targets per lane of its work lists
     std::vector<std::unique_ptr<FarLevel>> levels;
     FarLists mid;
+    GemmTables down, up;              // resampling to all levels at once, and back
+    LevelViews views;
+    int max_lev_pts = 0;              // most stacked level points of a sphere
+    DevBuf<int64_t> d_body_off;       // per tile: body-frame values of its level points
+    DevBuf<double> body64;            // those values (FP64 set, FP32 sets)
+    DevBuf<float> body32;
     bool cells = false;               // aggregate sources over cells on levels 2-3
     double cell_theta = kCellTheta;   // cells serve targets beyond cell_theta cell radii
     int equiv_k = kEquivK;            // equivalent point forces per cell
@@ -202,7 +213,9 @@ class Operator {
     // out += cId in + cSL S[in] + cTrac K'[in].  Far field: prec 0 FP64 direct
     // sum, 1 FP32 (multi-level unless disabled), 2 FP64 multi-level.
     static constexpr int kNumPrec = 4;
-    void p2p(const double *in, double *out, double cId, double cSL, double cTrac, int prec, const int *active);
+    // overwrite: out = that + cLOP L[in] instead (zero on inactive suspensions).
+    void p2p(const double *in, double *out, double cId, double cSL, double cTrac, int prec, const int *active,
+             bool overwrite = false, double cLOP = 0.0);
     // out += cLOP L[in]
     void lop(const double *in, double *out, double cLOP, const int *active);
     // out = A in with the stored coefficients (overwrites out)
@@ -248,24 +261,34 @@ class Operator {
     double *scratch_partial() { return partial_.p; }
 
   private:
-    void far(int kind, int prec, double coef, const double *in, double *out, const int *active);
+    // far field of the densities packed by pack() (FP64 direct sum of copies: of
+    // `in`): the fine-grid part as slots; *levels: the level set whose level
+    // fields are still to be added by levels_up (NULL: none)
+    FarSum far(int kind, int prec, double coef, const double *in, const int *active, LevelSet **levels);
+    // body-frame values and far-field sources of `in` for an apply of precision
+    // prec (-1: the values alone)
+    void pack(const double *in, int prec);
+    void analyse(const int *active, hipStream_t s) { launch_analysis(geom_, anal_.view, body64_.p, coef_.p, active, s); }
+    void far_slots(FarLists &L, int kind, int prec, const void *src, const double *tcoords, const double *tnorms,
+                   const float *trg32, double coef, const int *active);
+    void levels_up(LevelSet &S, double *out, const int *active);
+    void ensure_fp32_grid();
     void far_run(FarLists &L, int kind, int prec, const void *src, const double *tcoords, const double *tnorms,
                  const float *trg32, const Chunk *chunks, int nchunks, double coef, double *out, const int *active);
     void ensure_levels(LevelSet &S);
-    void far_copies(int kind, double coef, const double *in, double *out, const int *active, hipEvent_t ev_a);
+    void level_transforms(LevelSet &S);
+    void far_copies(int kind, double coef, const double *in, const int *active, hipEvent_t ev_a);
     // tile-shape autotuner: times candidate work-list shapes on this problem
     void autotune_fine(double &budget_s);
     void autotune_inner(double &budget_s);
     double time_far_pass(FarLists &L, int prec, const void *src, const double *tcoords, const double *tnorms,
-                         const float *trg32, const Chunk *chunks, int nchunks, double *out);
-    void far_levels_pass(LevelSet &S, const double *in, double *out);
+                         const float *trg32);
     std::vector<std::vector<int>> neighbours_within(double amax) const;
     bool outer_levels_pay();
     void ensure_centre();
-    // multi-level far field of `in` into out; ev_a and ev_b (if set) bracket
-    // the pair-sum launches
-    void far_levels(LevelSet &S, int kind, double coef, const double *in, double *out, const int *active,
-                    hipEvent_t ev_a, hipEvent_t ev_b);
+    // multi-level far field of the packed densities into the slots of the set's
+    // lists; ev_a and ev_b (if set) bracket the pair-sum launches
+    void far_levels(LevelSet &S, int kind, double coef, const int *active, hipEvent_t ev_a, hipEvent_t ev_b);
 
     StreamOwner stream_owner_; // declared before every buffer, so destroyed after them
     StreamOwner aux_owner_;    // second stream: self/near terms beside the far field
@@ -293,7 +316,12 @@ class Operator {
     DevBuf<int> d_order_, d_sph_susp_, d_near_src_, d_tile_sph_;
     DevBuf<SphTile> d_tiles_;
     DevBuf<int64_t> d_pt_off_, d_coef_off_, d_rec_off_, d_near_off_;
-    DevBuf<double> d_anal_[kMaxOrder + 1];
+    GemmTables anal_;               // analysis matrices
+    DevBuf<int64_t> d_body_off_;
+    DevBuf<double> body64_;         // body-frame values of the density being applied
+    DevBuf<float> body32_;
+    std::vector<SphTile> tiles_;
+    int max_pts_ = 0;               // most grid points of a sphere
     DevGeom geom_;
 
     // far-field work lists: fine grid (FP64 and direct FP32); the multi-level
@@ -303,7 +331,7 @@ class Operator {
     std::string tune_log_;         // autotuner decisions
     LevelSet ls32_, ls64_;
     LevelSet lsc_; // coarse FP32 operator (prec 3): the preconditioning solves of the mixed form
-    bool multi_level_ = true, timing_done_ = false;
+    bool multi_level_ = true;
     int outer_pay_ = -1; // FP64 multi-level outer far field in use: -1 undecided, 0 no, 1 yes
     std::future<void> ls64_build_; // ls64_ being built on a host thread (prepare_mixed)
     void wait_outer_levels();      // joins that build, rethrowing its error

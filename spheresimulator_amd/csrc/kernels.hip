@@ -9,9 +9,6 @@
 //                            through scalar loads (no LDS staging).
 // Centre sums k_far_centre   Faxen sphere-centre sums of the final velocities;
 //             k_far_rigid    closed-form traction of distant rigid-body densities.
-// SH matrices k_tiled_apply  grid values -> vector-SH coefficients per sphere
-//                            (Shexp::calcSpectralCoeff, Sphere/Shexp.cpp:408-447)
-//                            and resampling between grids, 16 spheres per tile.
 // Expansion   k_expand       coefficients -> exterior solid-harmonic expansion
 //                            records (the flow of SCTL StokesEvalSL/KL/KSelf).
 // Near/self   k_sheval_src,  self (SphereSTKSHOperator.cpp:305-351, :375-456)
@@ -66,6 +63,27 @@ __device__ __forceinline__ T block_sum(T v, T *sh) {
     return r;
 }
 
+// A and B of the rigid-body projector of the density `in` on the points [b, e)
+// of one sphere, by one workgroup (every thread gets both)
+__device__ __forceinline__ void rigid_part(const DevGeom &g, const double *__restrict__ in, int64_t b, int64_t e,
+                                           double R, double *sh, double A[3], double B[3]) {
+    double a[6] = {0, 0, 0, 0, 0, 0};
+    for (int64_t i = b + threadIdx.x; i < e; i += blockDim.x) {
+        const double w = g.w[i];
+        const double v[3] = {in[3 * i], in[3 * i + 1], in[3 * i + 2]};
+        const double nv[3] = {g.norms[3 * i], g.norms[3 * i + 1], g.norms[3 * i + 2]};
+        a[0] += w * v[0];
+        a[1] += w * v[1];
+        a[2] += w * v[2];
+        a[3] += w * R * (nv[1] * v[2] - nv[2] * v[1]);
+        a[4] += w * R * (nv[2] * v[0] - nv[0] * v[2]);
+        a[5] += w * R * (nv[0] * v[1] - nv[1] * v[0]);
+    }
+    const double ca = 1.0 / (4.0 * kPi * R * R), cb = 3.0 / (8.0 * kPi * R * R * R * R);
+    for (int c = 0; c < 3; c++) A[c] = block_sum(a[c], sh) * ca;
+    for (int c = 0; c < 3; c++) B[c] = block_sum(a[3 + c], sh) * cb;
+}
+
 // ---------------------------------------------------------------------------
 // source / target packing
 
@@ -75,12 +93,10 @@ __global__ void k_pack_src_f64(int64_t n, const double *__restrict__ coords, con
     if (i >= n) return;
     const double wi = w[i];
     double *o = src + 8 * i;
-    o[0] = coords[3 * i];
-    o[1] = coords[3 * i + 1];
-    o[2] = coords[3 * i + 2];
-    o[3] = wi * in[3 * i];
-    o[4] = wi * in[3 * i + 1];
-    o[5] = wi * in[3 * i + 2];
+    for (int c = 0; c < 3; c++) {
+        o[c] = coords[3 * i + c];
+        o[3 + c] = in ? wi * in[3 * i + c] : 0.0;
+    }
     o[6] = 0.0;
     o[7] = 0.0;
 }
@@ -91,12 +107,10 @@ __global__ void k_pack_src_f32(int64_t n, const double *__restrict__ coords, con
     if (i >= n) return;
     const double wi = w[i];
     float *o = src + 8 * i;
-    o[0] = (float)coords[3 * i];
-    o[1] = (float)coords[3 * i + 1];
-    o[2] = (float)coords[3 * i + 2];
-    o[3] = (float)(wi * in[3 * i]);
-    o[4] = (float)(wi * in[3 * i + 1]);
-    o[5] = (float)(wi * in[3 * i + 2]);
+    for (int c = 0; c < 3; c++) {
+        o[c] = (float)coords[3 * i + c];
+        o[3 + c] = in ? (float)(wi * in[3 * i + c]) : 0.f;
+    }
     o[6] = 0.f;
     o[7] = 0.f;
 }
@@ -435,8 +449,8 @@ void launch_far(int kind, int prec, int tpl, const void *src, const double *tcoo
 constexpr int kEqCells = 4;
 constexpr int kEqThreads = 256;
 __global__ __launch_bounds__(kEqThreads) void k_equiv_forces(int ncell, int K, int Kc, const double *__restrict__ P,
-                                                             const double *__restrict__ u,
-                                                             const double *__restrict__ rho,
+                                                             const double *__restrict__ u, int nslot,
+                                                             int64_t stride, const double *__restrict__ rho,
                                                              const int *__restrict__ susp,
                                                              const int *__restrict__ active, float *__restrict__ eq) {
     extern __shared__ double su[]; // kEqCells x 3Kc
@@ -444,7 +458,11 @@ __global__ __launch_bounds__(kEqThreads) void k_equiv_forces(int ncell, int K, i
     const int nc = min(kEqCells, ncell - c0);
     const int m = 3 * Kc, n = 3 * K;
     for (int k = 0; k < nc; k++)
-        for (int j = threadIdx.x; j < m; j += blockDim.x) su[k * m + j] = u[(int64_t)(c0 + k) * m + j];
+        for (int j = threadIdx.x; j < m; j += blockDim.x) {
+            double v = 0.0;
+            for (int q = 0; q < nslot; q++) v += u[q * stride + (int64_t)(c0 + k) * m + j];
+            su[k * m + j] = v;
+        }
     __syncthreads();
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
         double acc[kEqCells] = {};
@@ -461,183 +479,12 @@ __global__ __launch_bounds__(kEqThreads) void k_equiv_forces(int ncell, int K, i
     }
 }
 
-void launch_equiv_forces(int ncell, int K, int Kc, const double *P, const double *u, const double *rho,
-                         const int *susp, const int *active, float *eq, hipStream_t s) {
+void launch_equiv_forces(int ncell, int K, int Kc, const double *P, const double *u, int nslot, int64_t stride,
+                         const double *rho, const int *susp, const int *active, float *eq, hipStream_t s) {
     if (ncell <= 0) return;
     const size_t lds = sizeof(double) * kEqCells * 3 * Kc;
-    k_equiv_forces<<<dim3((ncell + kEqCells - 1) / kEqCells), dim3(kEqThreads), lds, s>>>(ncell, K, Kc, P, u, rho,
-                                                                                          susp, active, eq);
-}
-
-// ---------------------------------------------------------------------------
-// Per-sphere matrices applied to body-frame values, one tile of up to kTileSph
-// = 16 spheres of the same order per workgroup, as a GEMM on the matrix cores
-// (the tables are up to 12.7 MB at p = 16; each element is read once per tile):
-//   analysis:  coef[S] = A_p (q_S^-1 in_S)                (A_p: 6Q x 3n)
-//   resample:  out_S (+)= q_S M_p (q_S^-1 in_S)            (M_p: 3 nout x 3 nin)
-// A workgroup owns kRowBlock = 192 matrix rows (64 points): each of its four
-// waves three blocks of 16 rows, accumulated by v_mfma_f64_16x16x4f64 over the
-// columns (16 rows x 4 columns of the matrix, read from global memory, times
-// 4 columns x 16 spheres of the rotated input).  The input is staged through
-// LDS in chunks of kChunkPts points, stored [column][sphere].  Operand layout
-// of the instruction: A[i][k] in lane i + 16k, B[k][j] in lane j + 16k,
-// D[i][j] in lane j + 16 (i % 4), element i / 4.
-// The FP32 inner operator's level resampling runs the same GEMM with FP32
-// tables, FP32 staging and v_mfma_f32_16x16x4f32 (same A and B layout, D[i][j]
-// in lane j + 16 (i / 4), element i % 4; FP32 accumulation: about 1e-7
-// relative against the FP64 resampling, far below that operator's own 4e-6).
-constexpr int kRowBlock = 192;
-constexpr int kWaveRowBlocks = 3;
-constexpr int kChunkPts = 64;
-typedef double dbl4 __attribute__((ext_vector_type(4)));
-typedef float flt4 __attribute__((ext_vector_type(4)));
-
-template <typename T>
-struct MatTabsT {
-    const T *M[kMaxOrder + 1] = {};
-    int rows[kMaxOrder + 1] = {};
-    int nin[kMaxOrder + 1] = {};
-};
-using MatTabs = MatTabsT<double>;
-
-__device__ __forceinline__ dbl4 mfma16x16x4(double a, double b, dbl4 c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ flt4 mfma16x16x4(float a, float b, flt4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-template <bool RESAMPLE, typename T>
-__global__ __launch_bounds__(256) void k_tiled_apply(DevGeom g, MatTabsT<T> tab, const int64_t *__restrict__ in_off,
-                                                     const int64_t *__restrict__ out_off,
-                                                     const double *__restrict__ in, double *__restrict__ out,
-                                                     int accumulate, const int *__restrict__ active) {
-    typedef T T4 __attribute__((ext_vector_type(4)));
-    __shared__ T V[3 * kChunkPts * kTileSph];
-    __shared__ T P[kRowBlock * kTileSph];
-    const SphTile Ti = g.tiles[blockIdx.x];
-    const int p = Ti.p, rows = tab.rows[p], nin = tab.nin[p];
-    const int r0 = blockIdx.y * kRowBlock;
-    if (r0 >= rows) return;
-    const T *__restrict__ M = tab.M[p];
-    const int *sph = g.tile_sph + Ti.first;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int li = lane & 15, kq = lane >> 4;
-    const int rw = r0 + wv * 16 * kWaveRowBlocks; // this wave's first row
-    T4 acc[kWaveRowBlocks];
-#pragma unroll
-    for (int rb = 0; rb < kWaveRowBlocks; rb++) acc[rb] = T4{T(0), T(0), T(0), T(0)};
-    for (int k0 = 0; k0 < nin; k0 += kChunkPts) {
-        const int kc = min(kChunkPts, nin - k0);
-        __syncthreads();
-        for (int e = tid; e < kChunkPts * kTileSph; e += blockDim.x) {
-            const int t = e / kChunkPts, i = e % kChunkPts;
-            double o[3] = {0.0, 0.0, 0.0};
-            if (t < Ti.count && i < kc) {
-                const int S = sph[t];
-                const double *v = in + 3 * (in_off[S] + k0 + i);
-                const double vv[3] = {v[0], v[1], v[2]};
-                qrot(g.quat + 4 * S, vv, o, true);
-            }
-            V[(3 * i) * kTileSph + t] = (T)o[0];
-            V[(3 * i + 1) * kTileSph + t] = (T)o[1];
-            V[(3 * i + 2) * kTileSph + t] = (T)o[2];
-        }
-        __syncthreads();
-        const int nc = 3 * kc;
-        const T *Mc = M + (int64_t)(3 * k0) * rows;
-        for (int c = 0; c < nc; c += 4) {
-            const int col = c + kq;
-            const bool cin = col < nc;
-            const T b = cin ? V[col * kTileSph + li] : T(0);
-#pragma unroll
-            for (int rb = 0; rb < kWaveRowBlocks; rb++) {
-                const int r = rw + 16 * rb + li;
-                const T a = (cin && r < rows) ? Mc[(int64_t)col * rows + r] : T(0);
-                acc[rb] = mfma16x16x4(a, b, acc[rb]);
-            }
-        }
-    }
-    // row of element q of this lane's accumulator within its 16-row block:
-    // FP32 instruction 4 (lane / 16) + q, FP64 instruction (lane / 16) + 4 q
-#pragma unroll
-    for (int rb = 0; rb < kWaveRowBlocks; rb++)
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int i = sizeof(T) == 8 ? kq + 4 * q : 4 * kq + q;
-            P[(wv * 16 * kWaveRowBlocks + 16 * rb + i) * kTileSph + li] = acc[rb][q];
-        }
-    __syncthreads();
-    if (!RESAMPLE) {
-        const int nr = min(rows, r0 + kRowBlock) - r0;
-        for (int e = tid; e < nr * Ti.count; e += blockDim.x) {
-            const int t = e / nr, i = e % nr;
-            const int S = sph[t];
-            if (active && !active[g.sph_susp[S]]) continue;
-            out[g.coef_off[S] + r0 + i] = P[i * kTileSph + t];
-        }
-        return;
-    }
-    // resample: rotate each output point back to the lab frame
-    const int npt = (min(rows, r0 + kRowBlock) - r0) / 3;
-    for (int e = tid; e < npt * Ti.count; e += blockDim.x) {
-        const int t = e / npt, i = e % npt;
-        const int S = sph[t];
-        if (active && !active[g.sph_susp[S]]) continue;
-        const double vb[3] = {(double)P[(3 * i) * kTileSph + t], (double)P[(3 * i + 1) * kTileSph + t],
-                              (double)P[(3 * i + 2) * kTileSph + t]};
-        double o[3];
-        qrot(g.quat + 4 * S, vb, o, false);
-        double *dst = out + 3 * (out_off[S] + r0 / 3 + i);
-        if (accumulate) {
-            dst[0] += o[0];
-            dst[1] += o[1];
-            dst[2] += o[2];
-        } else {
-            dst[0] = o[0];
-            dst[1] = o[1];
-            dst[2] = o[2];
-        }
-    }
-}
-
-void launch_resample(const DevGeom &g, const ResampleTabs &tab, const int64_t *in_off, const int64_t *out_off,
-                     const double *in, double *out, int accumulate, const int *active, hipStream_t s,
-                     int max_points) {
-    if (!g.nsph || !g.ntiles) return;
-    const int rb = (3 * max_points + kRowBlock - 1) / kRowBlock;
-    if (tab.fp32) {
-        MatTabsT<float> mt;
-        for (int p = 0; p <= kMaxOrder; p++) {
-            mt.M[p] = tab.M32[p];
-            mt.rows[p] = 3 * tab.nout[p];
-            mt.nin[p] = tab.nin[p];
-        }
-        k_tiled_apply<true, float><<<dim3(g.ntiles, rb), dim3(256), 0, s>>>(g, mt, in_off, out_off, in, out,
-                                                                           accumulate, active);
-        return;
-    }
-    MatTabs mt;
-    for (int p = 0; p <= kMaxOrder; p++) {
-        mt.M[p] = tab.M[p];
-        mt.rows[p] = 3 * tab.nout[p];
-        mt.nin[p] = tab.nin[p];
-    }
-    k_tiled_apply<true, double><<<dim3(g.ntiles, rb), dim3(256), 0, s>>>(g, mt, in_off, out_off, in, out, accumulate,
-                                                                        active);
-}
-void launch_analysis(const DevGeom &g, const double *in, double *coef, const int *active, hipStream_t s,
-                     int max_order) {
-    if (!g.nsph || !g.ntiles) return;
-    MatTabs mt;
-    for (int p = 0; p <= kMaxOrder; p++) {
-        mt.M[p] = g.anal[p];
-        mt.rows[p] = 3 * (p + 1) * (p + 2);
-        mt.nin[p] = (p + 1) * (2 * p + 2);
-    }
-    const int rb = (3 * (max_order + 1) * (max_order + 2) + kRowBlock - 1) / kRowBlock;
-    k_tiled_apply<false, double><<<dim3(g.ntiles, rb), dim3(256), 0, s>>>(g, mt, g.pt_off, nullptr, in, coef, 0,
-                                                                         active);
+    k_equiv_forces<<<dim3((ncell + kEqCells - 1) / kEqCells), dim3(kEqThreads), lds, s>>>(
+        ncell, K, Kc, P, u, nslot, stride, rho, susp, active, eq);
 }
 
 // ---------------------------------------------------------------------------
@@ -1062,22 +909,49 @@ __global__ __launch_bounds__(64 * kSrcWaves) __attribute__((amdgpu_waves_per_eu(
     }
 }
 
-// out[T's points] += sum over T's items (self first, then near pairs in list
-// order) of their scratch contributions + cId in
+// out[T's points] (+)= far-field slots + sum over T's items (self first, then
+// near pairs in list order) of their scratch contributions + cId in + cLOP L[in],
+// L the rigid-body projector (SphereSTKSHOperator.cpp:487-521):
+//   A = sum w sigma / (4 pi R^2),  B = 3/(8 pi R^4) sum w R n x sigma,  L[sigma] = A + B x R n.
+// One pass over the output ends an apply: the slots of the far field (35 us at
+// 1024 spheres p=12 in a launch of its own), the near terms, the identity and L
+// each had a launch and a read-modify-write of the vector before.
 __global__ __launch_bounds__(256) void k_sheval_gather(DevGeom g, const int64_t *__restrict__ trg_slot_off,
                                                        const int *__restrict__ trg_nsrc, const double *__restrict__ scratch,
-                                                       const double *__restrict__ in, double *__restrict__ out, double cId,
+                                                       FarSum far, const double *__restrict__ in,
+                                                       double *__restrict__ out, double cId, double cLOP, int overwrite,
                                                        const int *__restrict__ active) {
+    __shared__ double sh[8];
     const int T = blockIdx.x;
-    if (active && !active[g.sph_susp[T]]) return;
     const int64_t off = g.pt_off[T];
     const int nT = (int)(g.pt_off[T + 1] - off);
+    if (active && !active[g.sph_susp[T]]) {
+        if (overwrite)
+            for (int i = threadIdx.x; i < 3 * nT; i += blockDim.x) out[3 * off + i] = 0.0;
+        return;
+    }
+    double A[3] = {0.0, 0.0, 0.0}, B[3] = {0.0, 0.0, 0.0};
+    const double R = g.rad[T];
+    if (cLOP != 0.0) rigid_part(g, in, off, off + nT, R, sh, A, B);
     const int64_t base = trg_slot_off[T];
     const int ns = trg_nsrc[T];
     for (int i = threadIdx.x; i < 3 * nT; i += blockDim.x) {
+        const int64_t j = 3 * off + i;
         double s = 0.0;
-        for (int k = 0; k < ns; k++) s += scratch[base + (int64_t)k * 3 * nT + i];
-        out[3 * off + i] += s + cId * in[3 * off + i];
+        for (int k = 0; k < far.nslot; k++) s += far.part[k * far.stride + j];
+        double v = 0.0;
+        for (int k = 0; k < ns; k++) v += scratch[base + (int64_t)k * 3 * nT + i];
+        s += v + cId * in[j];
+        if (cLOP != 0.0) {
+            const int c = i % 3;
+            const double *nv = g.norms + (j - c);
+            const double rn1 = R * nv[c == 0 ? 2 : c - 1], rn2 = R * nv[c == 2 ? 0 : c + 1];
+            // (B x R n)_c = B_{c+1} R n_{c+2} - B_{c+2} R n_{c+1}
+            const double b1 = c == 0 ? B[1] : c == 1 ? B[2] : B[0], b2 = c == 0 ? B[2] : c == 1 ? B[0] : B[1];
+            const double a = c == 0 ? A[0] : c == 1 ? A[1] : A[2];
+            s += cLOP * (a + b1 * rn1 - b2 * rn2);
+        }
+        out[j] = overwrite ? s : out[j] + s;
     }
 }
 
@@ -1109,18 +983,12 @@ void launch_sheval_items(const DevGeom &g, int mode, const double *rec, const Ev
                                                                    cTrac, active);
 }
 
-void launch_sheval_gather(const DevGeom &g, int nitems, const int64_t *trg_slot_off, const int *trg_nsrc,
-                          const double *scratch, const double *in, double *out, double cId, const int *active,
-                          hipStream_t s) {
-    if (!g.nsph || nitems <= 0) return;
-    k_sheval_gather<<<dim3(g.nsph), dim3(256), 0, s>>>(g, trg_slot_off, trg_nsrc, scratch, in, out, cId, active);
-}
-
-void launch_sheval(const DevGeom &g, int mode, const double *rec, const EvalItem *items, int nitems,
-                   const int64_t *trg_slot_off, const int *trg_nsrc, double *scratch, const double *in, double *out,
-                   double cSL, double cTrac, double cId, const int *active, hipStream_t s, const SrcItems *by_src) {
-    launch_sheval_items(g, mode, rec, items, nitems, scratch, cSL, cTrac, active, s, by_src);
-    launch_sheval_gather(g, nitems, trg_slot_off, trg_nsrc, scratch, in, out, cId, active, s);
+void launch_sheval_gather(const DevGeom &g, const int64_t *trg_slot_off, const int *trg_nsrc, const double *scratch,
+                          const FarSum &far, const double *in, double *out, double cId, double cLOP, bool overwrite,
+                          const int *active, hipStream_t s) {
+    if (!g.nsph) return;
+    k_sheval_gather<<<dim3(g.nsph), dim3(256), 0, s>>>(g, trg_slot_off, trg_nsrc, scratch, far, in, out, cId, cLOP,
+                                                      overwrite ? 1 : 0, active);
 }
 
 void launch_synthesis(const DevGeom &g, const double *rec, const EvalItem *self_items, int nitems, double *out,
@@ -1155,23 +1023,8 @@ __global__ __launch_bounds__(256) void k_lop(DevGeom g, const double *__restrict
     if (active && !active[g.sph_susp[S]]) return;
     const int64_t b = g.pt_off[S], e = g.pt_off[S + 1];
     const double R = g.rad[S];
-    double a[6] = {0, 0, 0, 0, 0, 0};
-    for (int64_t i = b + threadIdx.x; i < e; i += blockDim.x) {
-        const double w = g.w[i];
-        const double v[3] = {in[3 * i], in[3 * i + 1], in[3 * i + 2]};
-        const double nv[3] = {g.norms[3 * i], g.norms[3 * i + 1], g.norms[3 * i + 2]};
-        a[0] += w * v[0];
-        a[1] += w * v[1];
-        a[2] += w * v[2];
-        a[3] += w * R * (nv[1] * v[2] - nv[2] * v[1]);
-        a[4] += w * R * (nv[2] * v[0] - nv[0] * v[2]);
-        a[5] += w * R * (nv[0] * v[1] - nv[1] * v[0]);
-    }
-    double tot[6];
-    for (int c = 0; c < 6; c++) tot[c] = block_sum(a[c], sh);
-    const double ca = 1.0 / (4.0 * kPi * R * R), cb = 3.0 / (8.0 * kPi * R * R * R * R);
-    const double A[3] = {tot[0] * ca, tot[1] * ca, tot[2] * ca};
-    const double B[3] = {tot[3] * cb, tot[4] * cb, tot[5] * cb};
+    double A[3], B[3];
+    rigid_part(g, in, b, e, R, sh, A, B);
     for (int64_t i = b + threadIdx.x; i < e; i += blockDim.x) {
         const double rn[3] = {R * g.norms[3 * i], R * g.norms[3 * i + 1], R * g.norms[3 * i + 2]};
         out[3 * i] += cLOP * (A[0] + B[1] * rn[2] - B[2] * rn[1]);

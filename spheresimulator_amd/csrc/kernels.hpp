@@ -6,6 +6,7 @@
 namespace sphstk {
 
 constexpr int kMaxOrder = 32;
+constexpr int kMaxLevels = 6; // levels of a multi-level far field
 
 // Read-only device view of one (possibly batched) operator's geometry.
 // Spheres of one order, at most kTileSph of them (indices tile_sph[first ..
@@ -34,7 +35,7 @@ struct DevGeom {
     const double *w = nullptr;         // P
     const int64_t *near_off = nullptr; // N+1
     const int *near_src = nullptr;
-    const double *anal[kMaxOrder + 1] = {}; // analysis matrix per order (column-major)
+    const int64_t *body_off = nullptr; // per tile: first element of its body-frame grid values (see body_cols)
 };
 
 // Chunks of the DOF vector used by the segmented BLAS-1 kernels.
@@ -43,19 +44,34 @@ struct Chunk {
     int32_t seg, pad;
 };
 
-// Per-order resampling matrices on device (see Resample in common.hpp).
-// per-order resampling matrices (column-major, 3 nout x 3 nin); M32: the same
-// in FP32 (set for the FP32 inner operator's levels, whose resampling then runs
-// on FP32 matrix cores with FP32 accumulation), else NULL
-struct ResampleTabs {
-    bool fp32 = false;
-    const double *M[kMaxOrder + 1] = {};
-    const float *M32[kMaxOrder + 1] = {};
-    int nin[kMaxOrder + 1] = {};
-    int nout[kMaxOrder + 1] = {};
+// Body-frame values of a tile: 3 values per point as matrix columns, padded to
+// groups of 16, times 16 spheres (layout: transforms.hip).
+__host__ __device__ inline int body_cols(int points) { return (3 * points + 15) & ~15; }
+
+// A matrix per order in the layout of the transform GEMMs: nblk row blocks of
+// 48 rows, ngrp groups of 16 columns (pack_gemm in engine.hip).
+struct ShGemm {
+    const void *tab[kMaxOrder + 1] = {}; // FP64, or FP32 (FP32 level sets)
+    int nblk[kMaxOrder + 1] = {}, ngrp[kMaxOrder + 1] = {};
+    int max_blk = 0;
 };
 
-// source records (x, y, z, w*in, 0, 0) and FP32 target records (x, n, 0, 0) of n points
+// The levels of a multi-level far field as the transforms see them.  A sphere
+// of order p has the points first[p][l] .. first[p][l + 1] - 1 of its stacked
+// level points on level l, stored from off[l][S] on.
+struct LevelViews {
+    int nlev = 0;
+    int first[kMaxOrder + 1][kMaxLevels + 1] = {};
+    const int64_t *off[kMaxLevels] = {};
+    const double *w[kMaxLevels] = {};
+    void *src[kMaxLevels] = {};              // source records (force words written per apply)
+    const double *part[kMaxLevels][2] = {};  // partial-sum slots of the level's lists (level, source cells)
+    int nslot[kMaxLevels][2] = {};
+    int64_t stride[kMaxLevels] = {};         // between slots
+    const int64_t *body_off = nullptr;       // per tile: body-frame values of the stacked level points
+};
+
+// source records (x, y, z, w*in, 0, 0) (in NULL: zero forces) and FP32 target records (x, n, 0, 0) of n points
 void launch_pack_src_f64(int64_t n, const double *coords, const double *w, const double *in, double *src,
                          hipStream_t s);
 void launch_pack_src_f32(int64_t n, const double *coords, const double *w, const double *in, float *src,
@@ -71,18 +87,25 @@ void launch_far(int kind, int prec, int tpl, const void *src, const double *tcoo
                 bool levels = false);
 
 // Equivalent point forces of the far-field cells: the force words of eq
-// (FP32 source records, K per cell) = rho_c P u_c (P 3K x 3Kc column-major, u
-// 3Kc check velocities per cell); cells of inactive suspensions are skipped.
-void launch_equiv_forces(int ncell, int K, int Kc, const double *P, const double *u, const double *rho,
-                         const int *susp, const int *active, float *eq, hipStream_t s);
+// (FP32 source records, K per cell) = rho_c P u_c (P 3K x 3Kc column-major, u_c
+// the sum of nslot partial-sum slots of 3Kc check velocities per cell); cells
+// of inactive suspensions are skipped.
+void launch_equiv_forces(int ncell, int K, int Kc, const double *P, const double *u, int nslot, int64_t stride,
+                         const double *rho, const int *susp, const int *active, float *eq, hipStream_t s);
 
-// out_S (+)= R_S M_p R_S^-1 in_S between two point sets with per-sphere offsets
-void launch_resample(const DevGeom &g, const ResampleTabs &tab, const int64_t *in_off, const int64_t *out_off,
-                     const double *in, double *out, int accumulate, const int *active, hipStream_t s,
-                     int max_points);
-
-void launch_analysis(const DevGeom &g, const double *in, double *coef, const int *active, hipStream_t s,
-                     int max_order);
+// Transforms between grids and coefficients (transforms.hip).  pack_body: the
+// body-frame values bd (FP64) and/or bf (FP32) of `in`, and the force words of
+// the source records src64 / src32 (NULL: not wanted).
+void launch_pack_body(const DevGeom &g, const double *in, double *bd, float *bf, double *src64, float *src32,
+                      int max_points, hipStream_t s);
+void launch_analysis(const DevGeom &g, const ShGemm &M, const double *body, double *coef, const int *active,
+                     hipStream_t s);
+void launch_levels_down(const DevGeom &g, const ShGemm &M, bool fp64, const void *body, const LevelViews &L,
+                        const int *active, hipStream_t s);
+void launch_pack_levels(const DevGeom &g, bool fp64, const LevelViews &L, void *body, int max_points, hipStream_t s);
+// out += the level fields on the fine grids
+void launch_levels_up(const DevGeom &g, const ShGemm &M, bool fp64, const void *body, const LevelViews &L, double *out,
+                      const int *active, hipStream_t s);
 // per sphere and degree n: (F_r, F_s) <- 2x2 block tab[5n..5n+3], F_t <- tab[5n+4] F_t (in place)
 void launch_degree_blocks(const DevGeom &g, double *coef, const double *tab, const int *active, hipStream_t s);
 // mode 0: single-layer record (kRecSL arrays), 1: traction record (kRecTrac arrays)
@@ -109,19 +132,22 @@ struct SrcItems {
     int order_off[kMaxOrder + 2] = {};
 };
 
-// out += cSL*S_self/near + cTrac*K_self/near + cId*in   (mode 0: single layer, 1: traction)
-void launch_sheval(const DevGeom &g, int mode, const double *rec, const EvalItem *items, int nitems,
-                   const int64_t *trg_slot_off, const int *trg_nsrc, double *scratch, const double *in, double *out,
-                   double cSL, double cTrac, double cId, const int *active, hipStream_t s,
-                   const SrcItems *by_src = nullptr);
-// the two halves of launch_sheval: the per-item evaluations into scratch, and
-// the per-target gather (out += sum of the target's items + cId in)
+// Far-field sum on the fine grids as nslot partial-sum slots, stride apart.
+struct FarSum {
+    const double *part = nullptr;
+    int nslot = 0;
+    int64_t stride = 0;
+};
+
+// per-item self/near evaluations (mode 0: cSL single layer, 1: cTrac traction) into scratch
 void launch_sheval_items(const DevGeom &g, int mode, const double *rec, const EvalItem *items, int nitems,
                          double *scratch, double cSL, double cTrac, const int *active, hipStream_t s,
                          const SrcItems *by_src = nullptr);
-void launch_sheval_gather(const DevGeom &g, int nitems, const int64_t *trg_slot_off, const int *trg_nsrc,
-                          const double *scratch, const double *in, double *out, double cId, const int *active,
-                          hipStream_t s);
+// per-target gather: out (+)= far sum + the target's items + cId in + cLOP L[in]
+// (overwrite: out = ..., zero on inactive suspensions)
+void launch_sheval_gather(const DevGeom &g, const int64_t *trg_slot_off, const int *trg_nsrc, const double *scratch,
+                          const FarSum &far, const double *in, double *out, double cId, double cLOP, bool overwrite,
+                          const int *active, hipStream_t s);
 void launch_identity(const DevGeom &g, const double *in, double *out, double cId, const int *active,
                      hipStream_t s);
 void launch_lop(const DevGeom &g, const double *in, double *out, double cLOP, const int *active, hipStream_t s);
