@@ -57,8 +57,7 @@ struct FarGroup {
 
 // Number of complex arrays in the per-sphere expansion records.
 constexpr int kRecSL = 10;   // grad H1, grad H2, H3, grad H4
-constexpr int kRecTrac = 33; // 26 traction arrays + 7 self-synthesis arrays
-constexpr int kRecTracNear = 26;
+constexpr int kRecTrac = 23; // Hess H1, grad H2, Hess H2, H3, grad H3, Hess H4, P (Hessians without zz)
 
 // Host-side spherical-harmonic tables for one order p.
 struct ShTables {
@@ -76,6 +75,10 @@ const ShTables &sh_tables(int p);
 // The synthesis rows at the body-frame poles +z and -z: 6 rows (north x, y, z,
 // south x, y, z) of 6Q coefficients each, row-major.
 std::vector<double> pole_rows(int p);
+
+// out = synthesis(B_n coef) per SH degree n, (F_r, F_s) <- the 2x2 block
+// blocks[5n..5n+3], F_t <- blocks[5n+4] F_t: 3 npts x 6Q, column-major.
+std::vector<double> synthesis_of_blocks(int p, const std::vector<double> &blocks);
 
 // Per-order resampling matrices between the order-p grid and a coarser grid of
 // order pc <= p, both acting on body-frame values (3 per point), column-major:

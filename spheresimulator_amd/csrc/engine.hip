@@ -171,7 +171,6 @@ Operator::Operator(int nsusp, const int *counts, const double *pos, const double
         const int p = order_[i];
         pt_off_[i + 1] = pt_off_[i] + grid_points(p);
         coef_off_[i + 1] = coef_off_[i] + 3 * (p + 1) * (p + 2);
-        rec_off_[i + 1] = rec_off_[i] + 2 * kRecTrac * tri_size(p + 2);
     }
     npts_ = pt_off_[nsph_];
     coords_.resize(3 * npts_);
@@ -211,11 +210,14 @@ Operator::Operator(int nsusp, const int *counts, const double *pos, const double
                              near_src_);
     }
 
-    // self/near evaluation work items: per target sphere its own expansion first,
-    // then its near sources in list order, each cut into chunks of 64 targets;
-    // the same items grouped by source for the traction evaluation
+    for (int i = 0; i < nsph_; i++)
+        rec_off_[i + 1] = rec_off_[i] + (near_off_[i + 1] > near_off_[i] ? 2 * kRecTrac * tri_size(order_[i] + 2) : 0);
+
+    // slots of the self and near terms: per target sphere its own first, then its
+    // near sources in list order; near evaluation work items in chunks of 128
+    // targets, the same items grouped by source for the traction evaluation
     {
-        std::vector<EvalItem> items, selfi;
+        std::vector<EvalItem> items;
         std::vector<std::vector<EvalItem>> by_src(nsph_);
         std::vector<int64_t> tso(nsph_ + 1, 0);
         std::vector<int> tns(nsph_, 0);
@@ -224,20 +226,19 @@ Operator::Operator(int nsusp, const int *counts, const double *pos, const double
             const int nT = (int)(pt_off_[t + 1] - pt_off_[t]);
             tso[t] = slot;
             tns[t] = 1 + (int)(near_off_[t + 1] - near_off_[t]);
-            for (int k = 0; k < tns[t]; k++) {
-                const int s = (k == 0) ? t : near_src_[near_off_[t] + k - 1];
-                for (int j = 0; j < nT; j += 64) {
-                    EvalItem it{t, s, j, std::min(64, nT - j), slot + 3 * (int64_t)j};
+            slot += 3 * (int64_t)nT;
+            for (int k = 1; k < tns[t]; k++) {
+                const int s = near_src_[near_off_[t] + k - 1];
+                for (int j = 0; j < nT; j += 128) {
+                    EvalItem it{t, s, j, std::min(128, nT - j), slot + 3 * (int64_t)j};
                     items.push_back(it);
                     by_src[s].push_back(it);
-                    if (k == 0) selfi.push_back(it);
                 }
                 slot += 3 * (int64_t)nT;
             }
         }
         tso[nsph_] = slot;
         items_.upload(items);
-        self_items_.upload(selfi);
         std::vector<EvalItem> si;
         std::vector<int64_t> soff(nsph_ + 1, 0);
         si.reserve(items.size());
@@ -250,7 +251,7 @@ Operator::Operator(int nsusp, const int *counts, const double *pos, const double
         for (int p = 0; p <= kMaxOrder; p++) {
             src_items_.order_off[p] = (int)sl.size();
             for (int q = 0; q < nsph_; q++)
-                if (order_[q] == p) sl.push_back(q);
+                if (order_[q] == p && !by_src[q].empty()) sl.push_back(q);
         }
         src_items_.order_off[kMaxOrder + 1] = (int)sl.size();
         d_src_items_.upload(si);
@@ -309,6 +310,12 @@ Operator::Operator(int nsusp, const int *counts, const double *pos, const double
         d_body_off_.upload(bo);
         geom_.body_off = d_body_off_.p;
         body64_.alloc(std::max<int64_t>(bo.back(), 1));
+        for (size_t i = 0; i < tl.size(); i++)
+            bo[i + 1] = bo[i] + (int64_t)kTileSph * ((3 * (tl[i].p + 1) * (tl[i].p + 2) + 15) & ~15);
+        d_coef_body_off_.upload(bo);
+        geom_.coef_body_off = d_coef_body_off_.p;
+        cbody_.alloc(std::max<int64_t>(bo.back(), 1));
+        launch_fill((int64_t)cbody_.n, 0.0, cbody_.p, stream_); // padding columns stay zero
         tiles_ = tl;
         d_tile_sph_.upload(ts);
         d_tiles_.upload(tl);
@@ -1526,10 +1533,7 @@ void Operator::p2p(const double *in, double *out, double cId, double cSL, double
             SPHSTK_HIP(hipStreamWaitEvent(side, ev_fork_, 0));
         }
         if (first) analyse(active, side);
-        const int mode = kind == 0 ? 1 : 0;
-        launch_expand(geom_, mode, coef_.p, rec_.p, active, side, max_order_);
-        launch_sheval_items(geom_, mode, rec_.p, items_.p, (int)items_.n, evscratch_.p, cSL, cTrac, active, side,
-                            &src_items_);
+        near_terms(kind, cSL, cTrac, active, side);
         if (side != stream_) SPHSTK_HIP(hipEventRecord(ev_join_, side));
         LevelSet *S = nullptr;
         const FarSum f = far(kind, prec, kind == 0 ? -3.0 / (4.0 * kPi) * cTrac : cSL / (8.0 * kPi), in, active, &S);
@@ -1676,9 +1680,7 @@ void Operator::rigid_p2p(const double *force, const double *rho0, double *out, d
             -3.0 / (4.0 * kPi) * cTrac, out, nullptr);
     launch_far_rigid(d_coords_.p, d_norms_.p, d_pos_.p, force, d_rad_.p, npts_, lists_rigid_.ngroups,
                      lists_rigid_.order.p, lists_rigid_.groups.p, lists_rigid_.iv.p, out, cTrac, 1, stream_);
-    launch_expand(geom_, 1, coef_.p, rec_.p, nullptr, stream_, max_order_);
-    launch_sheval_items(geom_, 1, rec_.p, items_.p, (int)items_.n, evscratch_.p, 0.0, cTrac, nullptr, stream_,
-                        &src_items_);
+    near_terms(0, 0.0, cTrac, nullptr, stream_);
     launch_sheval_gather(geom_, d_trg_slot_off_.p, d_trg_nsrc_.p, evscratch_.p, FarSum{}, rho0, out, cId, 0.0, false,
                          nullptr, stream_);
     SPHSTK_HIP(hipGetLastError());
@@ -1689,8 +1691,7 @@ void Operator::rigid_velocity(const double *rho, double inv_mu, double *vel) {
     ensure_centre();
     pack(rho, 0);
     analyse(nullptr, stream_);
-    launch_expand(geom_, 0, coef_.p, rec_.p, nullptr, stream_, max_order_);
-    launch_sheval_items(geom_, 0, rec_.p, items_.p, (int)items_.n, evscratch_.p, 1.0, 0.0, nullptr, stream_);
+    near_terms(1, 1.0, 0.0, nullptr, stream_);
     launch_sheval_gather(geom_, d_trg_slot_off_.p, d_trg_nsrc_.p, evscratch_.p, FarSum{}, rho, u_ns_.p, 0.0, 0.0, true,
                          nullptr, stream_);
     far_run(lists_rv_mid_, 1, 0, src64_.p, d_coords_.p, d_norms_.p, nullptr, chunks_.p, (int)chunks_.n,
@@ -1800,8 +1801,7 @@ void Operator::project(double *inout) {
     if (nsph_ == 0) return;
     pack(inout, -1);
     analyse(nullptr, stream_);
-    launch_expand(geom_, 1, coef_.p, rec_.p, nullptr, stream_, max_order_);
-    launch_synthesis(geom_, rec_.p, self_items_.p, (int)self_items_.n, inout, stream_);
+    launch_synthesis(geom_, surface(kSurfValue), cbody_.p, d_pt_off_.p, 3, 1.0, 0, inout, nullptr, stream_);
     SPHSTK_HIP(hipGetLastError());
 }
 
@@ -1840,18 +1840,80 @@ static std::vector<double> self_inverse_blocks() {
     return t;
 }
 
+// Per-degree blocks of a sphere's own operators: K_ext above plus half of the
+// projection (the principal value (K_ext + K_int) / 2), and the single layer
+//   S: (F_r, F_s) -> (2 n(n+1) F_r + 3 n(n+1) F_s, 3 F_r + (2n^2+2n+3) F_s) / D_n, F_t -> F_t / (2n+1)
+// of the unit sphere (R S for radius R); both vanish at degree 0 but for the
+// half.  A sphere's own surface is thereby one more matrix on its coefficients.
+// Before, its expansion was evaluated point by point like a near neighbour's,
+// 33 arrays over (p+3)(p+4)/2 terms for each of its points.
+static std::vector<double> surface_blocks(bool traction) {
+    std::vector<double> t(5 * (kMaxOrder + 1), 0.0);
+    for (int n = 0; n <= kMaxOrder; n++) {
+        const double nn = n, D = (2 * nn - 1) * (2 * nn + 1) * (2 * nn + 3);
+        double *b = &t[5 * n];
+        if (traction) {
+            if (n > 0) {
+                b[0] = -nn * (4 * nn * nn + 6 * nn - 1) / D;
+                b[1] = -3.0 * nn * (nn + 1) / D;
+                b[2] = -3.0 / D;
+                b[3] = -(4 * nn * nn * nn + 6 * nn * nn - nn + 3) / D;
+                b[4] = -(nn + 2) / (2 * nn + 1);
+            }
+            b[0] += 0.5;
+            b[3] += 0.5;
+            b[4] += 0.5;
+        } else if (n > 0) {
+            b[0] = 2 * nn * (nn + 1) / D;
+            b[1] = 3 * nn * (nn + 1) / D;
+            b[2] = 3.0 / D;
+            b[3] = (2 * nn * nn + 2 * nn + 3) / D;
+            b[4] = 1.0 / (2 * nn + 1);
+        }
+    }
+    return t;
+}
+
+const ShGemm &Operator::surface(SurfaceOp k) {
+    GemmTables &G = surf_[k];
+    if (G.view.max_blk) return G.view;
+    std::vector<double> blocks(5 * (kMaxOrder + 1), 0.0);
+    if (k == kSurfTrac || k == kSurfSL) {
+        blocks = surface_blocks(k == kSurfTrac);
+    } else if (k == kSurfInverse) {
+        blocks = self_inverse_blocks();
+    } else {
+        for (int n = 0; n <= kMaxOrder; n++) blocks[5 * n] = blocks[5 * n + 3] = blocks[5 * n + 4] = 1.0;
+    }
+    for (int p = 0; p <= kMaxOrder; p++) {
+        if (!anal_.d[p].p) continue;
+        const int rows = 3 * grid_points(p), cols = 6 * tri_size(p);
+        upload_gemm(G, p, rows, cols, packed_gemm<double>(std::vector<int>{p, -3 - (int)k}, [&] {
+                        const std::vector<double> m = synthesis_of_blocks(p, blocks);
+                        return pack_gemm<double>(rows, cols, true, [&](int r, int c) { return m[size_t(c) * rows + r]; });
+                    }));
+    }
+    return G.view;
+}
+
+// The self (slot 0 of every target) and near terms into scratch, from the coefficients.
+void Operator::near_terms(int kind, double cSL, double cTrac, const int *active, hipStream_t s) {
+    launch_synthesis(geom_, surface(kind == 0 ? kSurfTrac : kSurfSL), cbody_.p, d_trg_slot_off_.p, 1,
+                     kind == 0 ? cTrac : cSL, kind == 0 ? 0 : 1, evscratch_.p, active, s);
+    const int mode = kind == 0 ? 1 : 0;
+    launch_expand(geom_, mode, src_items_.srcs, (int)d_src_list_.n, coef_.p, rec_.p, active, s, max_order_);
+    launch_sheval_items(geom_, mode, rec_.p, items_.p, (int)items_.n, evscratch_.p, cSL, cTrac, active, s, &src_items_);
+}
+
 // out = M^-1 in, M the block-diagonal (one block per sphere) part of the
 // operator: the exact inverse of each sphere's self operator (isolated-sphere
 // preconditioner).  Suspensions not active keep out = 2 in.
 void Operator::precondition(const double *in, double *out, const int *active) {
     if (nsph_ == 0) return;
-    if (!self_inv_.p) self_inv_.upload(self_inverse_blocks());
     pack(in, -1);
     analyse(active, stream_);
-    launch_degree_blocks(geom_, coef_.p, self_inv_.p, active, stream_);
-    launch_expand(geom_, 1, coef_.p, rec_.p, active, stream_, max_order_);
     launch_fill(3 * npts_, 0.0, out, stream_);
-    launch_synthesis(geom_, rec_.p, self_items_.p, (int)self_items_.n, out, stream_, active);
+    launch_synthesis(geom_, surface(kSurfInverse), cbody_.p, d_pt_off_.p, 3, 1.0, 0, out, active, stream_);
     launch_axpby(3 * npts_, 2.0, in, 1.0, out, stream_);
 }
 

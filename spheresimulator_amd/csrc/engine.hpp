@@ -268,7 +268,15 @@ class Operator {
     // body-frame values and far-field sources of `in` for an apply of precision
     // prec (-1: the values alone)
     void pack(const double *in, int prec);
-    void analyse(const int *active, hipStream_t s) { launch_analysis(geom_, anal_.view, body64_.p, coef_.p, active, s); }
+    void analyse(const int *active, hipStream_t s) {
+        launch_analysis(geom_, anal_.view, body64_.p, coef_.p, cbody_.p, active, s);
+    }
+    // matrices from coefficients to a sphere's own grid: its traction
+    // (principal value) and single-layer operators, the plain synthesis, and
+    // that of M^-1 - 2 I (precondition); laid out on first use
+    enum SurfaceOp { kSurfTrac, kSurfSL, kSurfValue, kSurfInverse, kNumSurf };
+    const ShGemm &surface(SurfaceOp k);
+    void near_terms(int kind, double cSL, double cTrac, const int *active, hipStream_t s);
     void far_slots(FarLists &L, int kind, int prec, const void *src, const double *tcoords, const double *tnorms,
                    const float *trg32, double coef, const int *active);
     void levels_up(LevelSet &S, double *out, const int *active);
@@ -297,7 +305,6 @@ class Operator {
     static constexpr int kMultiCols = 8; // right-hand sides per shared far-field launch
     int ncopy_ = 1;         // identical copies of one set of suspensions (several right-hand sides)
     DevBuf<double> srcm_;   // source records of the shared far field of the copies
-    DevBuf<double> self_inv_; // per-degree blocks of the isolated-sphere inverse
     double c_[4];
     int flags_;
     int max_order_ = 0;
@@ -317,6 +324,9 @@ class Operator {
     DevBuf<SphTile> d_tiles_;
     DevBuf<int64_t> d_pt_off_, d_coef_off_, d_rec_off_, d_near_off_;
     GemmTables anal_;               // analysis matrices
+    GemmTables surf_[kNumSurf];
+    DevBuf<int64_t> d_coef_body_off_;
+    DevBuf<double> cbody_;          // the coefficients as GEMM columns
     DevBuf<int64_t> d_body_off_;
     DevBuf<double> body64_;         // body-frame values of the density being applied
     DevBuf<float> body32_;
@@ -351,11 +361,11 @@ class Operator {
     bool centre_ready_ = false;
     DevBuf<double> centre_part_, vel_ns_, u_ns_;
 
-    // self/near evaluation work items and their scratch
-    DevBuf<EvalItem> items_, self_items_;
+    // near evaluation work items and the scratch of the self and near terms
+    DevBuf<EvalItem> items_;
     DevBuf<EvalItem> d_src_items_;    // items_ grouped by source sphere
     DevBuf<int64_t> d_src_off_;
-    DevBuf<int> d_src_list_;          // spheres by order
+    DevBuf<int> d_src_list_;          // spheres with near neighbours by order
     SrcItems src_items_;
     DevBuf<int64_t> d_trg_slot_off_;
     DevBuf<int> d_trg_nsrc_;

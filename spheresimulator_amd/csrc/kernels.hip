@@ -11,8 +11,8 @@
 //             k_far_rigid    closed-form traction of distant rigid-body densities.
 // Expansion   k_expand       coefficients -> exterior solid-harmonic expansion
 //                            records (the flow of SCTL StokesEvalSL/KL/KSelf).
-// Near/self   k_sheval_src,  self (SphereSTKSHOperator.cpp:305-351, :375-456)
-//             k_sheval       and near-pair (:575-695) SH evaluations.
+// Near        k_sheval_src,  near-pair SH evaluations
+//             k_sheval       (SphereSTKSHOperator.cpp:575-695).
 // LOP         k_lop          rigid-body projector (:487-521).
 // BLAS-1      k_seg_*        segmented (one segment per suspension) GMRES
 //                            vector kernels.
@@ -499,10 +499,10 @@ void launch_equiv_forces(int ncell, int K, int Kc, const double *P, const double
 //   H1 = a, H2 = A_n b, H3 = B_n b, H4 = alpha, P = b,
 //   A_n = (2-n)/(2n(2n-1)), B_n = (n+1)/(n(2n-1))
 //   u = grad H1 + r^2 grad H2 + x H3 + x cross grad H4,  pressure P.
-// Self synthesis of the projected density at r=1:
-//   P sigma = Qr x + grad Qs + x cross grad Qt,  Qr = F_r + (n+1) F_s, Qs = F_s, Qt = F_t.
-// Records store, per (n,m) with n <= p+2, the K arrays' coefficients interleaved
+// Records store, per (n,m) with n <= p+2 and in order of m, then n, the K arrays' coefficients interleaved
 // as (eps_m Re c, -eps_m Im c) so that eps_m Re(c D) = c0 D.re + c1 D.im.
+
+__device__ __forceinline__ int rec_term(int P, int n, int m) { return m * (2 * P + 3 - m) / 2 + n - m; }
 
 __device__ __forceinline__ double2 hget(const double2 *h, int P, int n, int k) {
     if (k < 0 || k > n || n > P || n < 0) return make_double2(0.0, 0.0);
@@ -538,22 +538,32 @@ __device__ __forceinline__ double2 dcoef(const double2 *h, int P, int n1, int k,
     return r;
 }
 
-__global__ __launch_bounds__(256) void k_expand(DevGeom g, int mode, const double *__restrict__ coef,
-                                                double *__restrict__ rec, const int *__restrict__ active) {
+// degree n of entry k = n (n + 1) / 2 + m of a triangular array
+__device__ __forceinline__ int tri_row(int k) {
+    int n = (int)((sqrtf(8.f * k + 1.f) - 1.f) * 0.5f);
+    while ((n + 1) * (n + 2) / 2 <= k) n++;
+    while (n * (n + 1) / 2 > k) n--;
+    return n;
+}
+
+// One workgroup per sphere with near neighbours (the others need no record: a
+// sphere's own surface goes through launch_synthesis).
+__global__ __launch_bounds__(256) void k_expand(DevGeom g, int mode, const int *__restrict__ list,
+                                                const double *__restrict__ coef, double *__restrict__ rec,
+                                                const int *__restrict__ active) {
     extern __shared__ double2 lds[];
-    const int S = blockIdx.x;
+    const int S = list[blockIdx.x];
     if (active && !active[g.sph_susp[S]]) return;
     const int p = g.order[S];
     const int Q = (p + 1) * (p + 2) / 2, P1 = p + 1, Q1 = (P1 + 1) * (P1 + 2) / 2, P2 = p + 2,
               Q2 = (P2 + 1) * (P2 + 2) / 2;
-    const int nb = (mode == 0) ? 4 : 8;
-    double2 *base = lds;           // nb arrays of Q
-    double2 *grad = lds + nb * Q;  // (mode 0: H1,H2,H4; mode 1: H1,H2,H3,H4,Qs,Qt) x 3 arrays of Q1
+    const int nb = (mode == 0) ? 4 : 5;
+    double2 *base = lds;          // nb arrays of Q: H1, H2, H3, H4, P
+    double2 *grad = lds + nb * Q; // (mode 0: H1,H2,H4; mode 1: H1,H2,H3,H4) x 3 arrays of Q1
     const double2 *F = reinterpret_cast<const double2 *>(coef + g.coef_off[S]);
     // base arrays
     for (int k = threadIdx.x; k < Q; k += blockDim.x) {
-        int n = 0;
-        while ((n + 1) * (n + 2) / 2 <= k) n++;
+        const int n = tri_row(k);
         const double2 fr = F[k], fs = F[Q + k], ft = F[2 * Q + k];
         double2 h1 = make_double2(0, 0), h2 = h1, h3 = h1, h4 = h1, hp = h1;
         if (n >= 1) {
@@ -574,36 +584,25 @@ __global__ __launch_bounds__(256) void k_expand(DevGeom g, int mode, const doubl
         base[Q + k] = h2;
         base[2 * Q + k] = h3;
         base[3 * Q + k] = h4;
-        if (mode == 1) {
-            base[4 * Q + k] = hp;
-            base[5 * Q + k] = make_double2(fr.x + (n + 1.0) * fs.x, fr.y + (n + 1.0) * fs.y);
-            base[6 * Q + k] = fs;
-            base[7 * Q + k] = ft;
-        }
+        if (mode == 1) base[4 * Q + k] = hp;
     }
     __syncthreads();
     // gradient arrays
-    const int ng = (mode == 0) ? 3 : 6;
-    const int gsrc0[3] = {0, 1, 3};
-    const int gsrc1[6] = {0, 1, 2, 3, 6, 7};
+    const int ng = (mode == 0) ? 3 : 4;
     for (int idx = threadIdx.x; idx < ng * 3 * Q1; idx += blockDim.x) {
         const int a = idx / (3 * Q1), rem = idx % (3 * Q1), dir = rem / Q1, k1 = rem % Q1;
-        int n1 = 0;
-        while ((n1 + 1) * (n1 + 2) / 2 <= k1) n1++;
-        const int kk = k1 - n1 * (n1 + 1) / 2;
-        const int f = (mode == 0) ? gsrc0[a] : gsrc1[a];
+        const int n1 = tri_row(k1), kk = k1 - n1 * (n1 + 1) / 2;
+        const int f = (mode == 0 && a == 2) ? 3 : a;
         grad[(a * 3 + dir) * Q1 + k1] = dcoef(base + f * Q, p, n1, kk, dir);
     }
     __syncthreads();
     // record
     const int K = (mode == 0) ? kRecSL : kRecTrac;
-    double *R = rec + g.rec_off[S];
-    const int hd0[6] = {0, 0, 0, 1, 1, 2}, hd1[6] = {0, 1, 2, 1, 2, 2};
+    double2 *R = reinterpret_cast<double2 *>(rec + g.rec_off[S]);
+    const int hd0[5] = {0, 0, 0, 1, 1}, hd1[5] = {0, 1, 2, 1, 2};
     for (int idx = threadIdx.x; idx < K * Q2; idx += blockDim.x) {
         const int k2 = idx / K, a = idx % K;
-        int n2 = 0;
-        while ((n2 + 1) * (n2 + 2) / 2 <= k2) n2++;
-        const int m = k2 - n2 * (n2 + 1) / 2;
+        const int n2 = tri_row(k2), m = k2 - n2 * (n2 + 1) / 2;
         double2 c = make_double2(0, 0);
         if (mode == 0) {
             // 0-2 grad H1, 3-5 grad H2, 6 H3, 7-9 grad H4
@@ -616,67 +615,32 @@ __global__ __launch_bounds__(256) void k_expand(DevGeom g, int mode, const doubl
                 c = hget(grad + (2 * 3 + (a - 7)) * Q1, P1, n2, m);
             }
         } else {
-            // 0-5 Hess H1, 6-8 grad H2, 9-14 Hess H2, 15 H3, 16-18 grad H3, 19-24 Hess H4, 25 P,
-            // 26 Qr, 27-29 grad Qs, 30-32 grad Qt
-            if (a < 6) {
+            // 0-4 Hess H1, 5-7 grad H2, 8-12 Hess H2, 13 H3, 14-16 grad H3, 17-21 Hess H4, 22 P
+            if (a < 5)
                 c = dcoef(grad + (0 * 3 + hd0[a]) * Q1, P1, n2, m, hd1[a]);
-            } else if (a < 9) {
-                c = hget(grad + (1 * 3 + (a - 6)) * Q1, P1, n2, m);
-            } else if (a < 15) {
-                c = dcoef(grad + (1 * 3 + hd0[a - 9]) * Q1, P1, n2, m, hd1[a - 9]);
-            } else if (a == 15) {
+            else if (a < 8)
+                c = hget(grad + (1 * 3 + (a - 5)) * Q1, P1, n2, m);
+            else if (a < 13)
+                c = dcoef(grad + (1 * 3 + hd0[a - 8]) * Q1, P1, n2, m, hd1[a - 8]);
+            else if (a == 13)
                 c = hget(base + 2 * Q, p, n2, m);
-            } else if (a < 19) {
-                c = hget(grad + (2 * 3 + (a - 16)) * Q1, P1, n2, m);
-            } else if (a < 25) {
-                c = dcoef(grad + (3 * 3 + hd0[a - 19]) * Q1, P1, n2, m, hd1[a - 19]);
-            } else if (a == 25) {
+            else if (a < 17)
+                c = hget(grad + (2 * 3 + (a - 14)) * Q1, P1, n2, m);
+            else if (a < 22)
+                c = dcoef(grad + (3 * 3 + hd0[a - 17]) * Q1, P1, n2, m, hd1[a - 17]);
+            else
                 c = hget(base + 4 * Q, p, n2, m);
-            } else if (a == 26) {
-                c = hget(base + 5 * Q, p, n2, m);
-            } else if (a < 30) {
-                c = hget(grad + (4 * 3 + (a - 27)) * Q1, P1, n2, m);
-            } else {
-                c = hget(grad + (5 * 3 + (a - 30)) * Q1, P1, n2, m);
-            }
         }
         const double eps = m ? 2.0 : 1.0;
-        R[2 * (k2 * K + a)] = eps * c.x;
-        R[2 * (k2 * K + a) + 1] = -eps * c.y;
+        R[K * rec_term(P2, n2, m) + a] = make_double2(eps * c.x, -eps * c.y);
     }
 }
 
-// Per-degree blocks on the SH coefficients of each sphere, in place:
-// (F_r, F_s) <- M_n (F_r, F_s) (real 2x2, tab[5n..5n+3] row-major),
-// F_t <- tab[5n+4] F_t.  Used for the inverse of the single-sphere operator.
-__global__ __launch_bounds__(256) void k_degree_blocks(DevGeom g, double *__restrict__ coef,
-                                                       const double *__restrict__ tab,
-                                                       const int *__restrict__ active) {
-    const int S = blockIdx.x;
-    if (active && !active[g.sph_susp[S]]) return;
-    const int p = g.order[S];
-    const int Q = (p + 1) * (p + 2) / 2;
-    double2 *F = reinterpret_cast<double2 *>(coef + g.coef_off[S]);
-    for (int k = threadIdx.x; k < Q; k += blockDim.x) {
-        int n = 0;
-        while ((n + 1) * (n + 2) / 2 <= k) n++;
-        const double *t = tab + 5 * n;
-        const double2 r = F[k], s = F[Q + k], u = F[2 * Q + k];
-        F[k] = make_double2(t[0] * r.x + t[1] * s.x, t[0] * r.y + t[1] * s.y);
-        F[Q + k] = make_double2(t[2] * r.x + t[3] * s.x, t[2] * r.y + t[3] * s.y);
-        F[2 * Q + k] = make_double2(t[4] * u.x, t[4] * u.y);
-    }
-}
-
-void launch_degree_blocks(const DevGeom &g, double *coef, const double *tab, const int *active, hipStream_t s) {
-    if (g.nsph) k_degree_blocks<<<dim3(g.nsph), dim3(256), 0, s>>>(g, coef, tab, active);
-}
-
-void launch_expand(const DevGeom &g, int mode, const double *coef, double *rec, const int *active, hipStream_t s,
-                   int max_order) {
-    if (!g.nsph) return;
+void launch_expand(const DevGeom &g, int mode, const int *list, int n, const double *coef, double *rec,
+                   const int *active, hipStream_t s, int max_order) {
+    if (!n) return;
     const int Q = tri_size(max_order), Q1 = tri_size(max_order + 1);
-    const size_t lds = sizeof(double) * 2 * ((mode == 0 ? 4 : 8) * Q + (mode == 0 ? 9 : 18) * Q1);
+    const size_t lds = sizeof(double) * 2 * ((mode == 0 ? 4 : 5) * Q + (mode == 0 ? 9 : 12) * Q1);
     static size_t lds_set = 0;
     if (lds > 65536 && lds > lds_set) {
         if (hipFuncSetAttribute((const void *)k_expand, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=
@@ -684,14 +648,14 @@ void launch_expand(const DevGeom &g, int mode, const double *coef, double *rec, 
             throw Error(-2, "cannot raise the LDS limit of the expansion kernel to " + std::to_string(lds));
         lds_set = lds;
     }
-    k_expand<<<dim3(g.nsph), dim3(256), lds, s>>>(g, mode, coef, rec, active);
+    k_expand<<<dim3(n), dim3(256), lds, s>>>(g, mode, list, coef, rec, active);
 }
 
 // ---------------------------------------------------------------------------
-// Expansion evaluation: acc[a] = sum_{n<=P, m<=n} (c0 D.re + c1 D.im) for arrays
-// a in [KBEG, KBEG+KCNT) of a record with KTOT arrays, D_n^m by recurrence.
+// Expansion evaluation: acc[a] = sum_{n<=P, m<=n} (c0 D.re + c1 D.im) for the
+// KCNT arrays of a record, D_n^m by recurrence.
 
-template <int KTOT, int KBEG, int KCNT>
+template <int KCNT>
 __device__ __forceinline__ void eval_record(const double *__restrict__ rec, int P, double x, double y, double z,
                                             double *acc) {
 #pragma unroll
@@ -709,7 +673,7 @@ __device__ __forceinline__ void eval_record(const double *__restrict__ rec, int 
         double pr = 0.0, pi = 0.0, cr = dmr, ci = dmi;
         const double mm = (double)m * m;
         for (int n = m; n <= P; n++) {
-            const double *c = rec + 2 * (KTOT * dtri(n, m) + KBEG);
+            const double *c = rec + 2 * KCNT * rec_term(P, n, m);
 #pragma unroll
             for (int a = 0; a < KCNT; a++) acc[a] = __builtin_fma(c[2 * a], cr, __builtin_fma(c[2 * a + 1], ci, acc[a]));
             const double f1 = -(2.0 * n + 1.0) * z * ir2, f2 = -((double)n * n - mm) * ir2;
@@ -728,131 +692,190 @@ __device__ __forceinline__ void cross3(const double a[3], const double b[3], dou
     o[2] = a[0] * b[1] - a[1] * b[0];
 }
 
-// symmetric 3x3 from (xx,xy,xz,yy,yz,zz) times v
+// traceless symmetric 3x3 from (xx,xy,xz,yy,yz) times v (the Hessian of a harmonic function)
 __device__ __forceinline__ void symv(const double *h, const double v[3], double o[3]) {
     o[0] = h[0] * v[0] + h[1] * v[1] + h[2] * v[2];
     o[1] = h[1] * v[0] + h[3] * v[1] + h[4] * v[2];
-    o[2] = h[2] * v[0] + h[4] * v[1] + h[5] * v[2];
+    o[2] = h[2] * v[0] + h[4] * v[1] - (h[0] + h[3]) * v[2];
 }
 
-// traction of the exterior flow from the 26 traction arrays (layout of k_expand)
+// traction of the exterior flow from the 23 traction arrays (layout of k_expand)
 __device__ __forceinline__ void traction_from(const double *A, const double x[3], const double v[3], double t[3]) {
     const double r2 = x[0] * x[0] + x[1] * x[1] + x[2] * x[2];
     const double xv = x[0] * v[0] + x[1] * v[1] + x[2] * v[2];
-    const double *g2 = A + 6, *g3 = A + 16;
-    const double h3 = A[15], pr = A[25];
+    const double *g2 = A + 5, *g3 = A + 14;
+    const double h3 = A[13], pr = A[22];
     const double vg2 = v[0] * g2[0] + v[1] * g2[1] + v[2] * g2[2];
     const double vg3 = v[0] * g3[0] + v[1] * g3[1] + v[2] * g3[2];
     double H1v[3], H2v[3], H4v[3], vx[3], H4vx[3], xH4v[3];
     symv(A + 0, v, H1v);
-    symv(A + 9, v, H2v);
-    symv(A + 19, v, H4v);
+    symv(A + 8, v, H2v);
+    symv(A + 17, v, H4v);
     cross3(v, x, vx);
-    symv(A + 19, vx, H4vx);
+    symv(A + 17, vx, H4vx);
     cross3(x, H4v, xH4v);
     for (int c = 0; c < 3; c++)
         t[c] = -pr * v[c] + 2.0 * H1v[c] + 2.0 * xv * g2[c] + 2.0 * x[c] * vg2 + 2.0 * r2 * H2v[c] +
                2.0 * h3 * v[c] + x[c] * vg3 + xv * g3[c] + xH4v[c] + H4vx[c];
 }
 
-// One work item = one 64-lane wave: targets [tstart, tstart+tcount) of sphere T
-// against the expansion of sphere S (S == T: self).  MODE 0: single layer,
-// 2: synthesis of the projected density (self items only); the traction runs
-// in k_sheval_src.  MODE 0 writes the item's contribution (lab frame,
-// coefficients applied) to scratch[slot + 3*lane]; MODE 2 writes out directly.
+// One work item of the single layer = one wave: targets [tstart, tstart+tcount)
+// of sphere T against the expansion of its near sphere S; the contribution (lab
+// frame, coefficient applied) goes to scratch[slot + 3 target].  The traction
+// runs in k_sheval_src.
 // Workgroups go to the 8 XCDs round-robin, so workgroup b takes item
 // (b % 8) * ceil(nitems / 8) + b / 8: each XCD runs a contiguous range of the
 // items, whose chunks and neighbouring targets read the same source records
-// (63 KB at p = 12) from its own L2.  The grid is 8 ceil(nitems / 8).
-template <int MODE>
+// from its own L2.  The grid is 8 ceil(nitems / 8).
 __global__ __launch_bounds__(64) void k_sheval(DevGeom g, const double *__restrict__ rec,
                                                const EvalItem *__restrict__ items, int nitems,
-                                               double *__restrict__ scratch, double *__restrict__ out, double cSL,
-                                               double cTrac, const int *__restrict__ active) {
+                                               double *__restrict__ scratch, double cSL,
+                                               const int *__restrict__ active) {
     const int chunk = (int)(gridDim.x >> 3);
     const int pos = (int)(blockIdx.x & 7) * chunk + (int)(blockIdx.x >> 3);
     if (pos >= nitems) return;
     const EvalItem it = items[pos];
     const int T = it.trg, S = it.src;
     if (active && !active[g.sph_susp[T]]) return;
-    const int lane = threadIdx.x;
-    if (lane >= it.tcount) return;
-    const int64_t gp = g.pt_off[T] + it.tstart + lane;
-    const double X[3] = {g.coords[3 * gp], g.coords[3 * gp + 1], g.coords[3 * gp + 2]};
     const double *q = g.quat + 4 * S;
     const double R = g.rad[S];
     const double iR = 1.0 / R;
-    const double d[3] = {(X[0] - g.pos[3 * S]) * iR, (X[1] - g.pos[3 * S + 1]) * iR, (X[2] - g.pos[3 * S + 2]) * iR};
-    double xi[3], res[3], lab[3];
-    qrot(q, d, xi, true);
-    const int P = g.order[S] + 2;
-    const double *recS = rec + g.rec_off[S];
-    if (MODE == 0) {
-        double A[kRecSL];
-        eval_record<kRecSL, 0, kRecSL>(recS, P, xi[0], xi[1], xi[2], A);
+    for (int k = threadIdx.x; k < it.tcount; k += 64) {
+        const int64_t gp = g.pt_off[T] + it.tstart + k;
+        const double d[3] = {(g.coords[3 * gp] - g.pos[3 * S]) * iR, (g.coords[3 * gp + 1] - g.pos[3 * S + 1]) * iR,
+                             (g.coords[3 * gp + 2] - g.pos[3 * S + 2]) * iR};
+        double xi[3], res[3], lab[3], A[kRecSL], xg4[3];
+        qrot(q, d, xi, true);
+        eval_record<kRecSL>(rec + g.rec_off[S], g.order[S] + 2, xi[0], xi[1], xi[2], A);
         const double r2 = xi[0] * xi[0] + xi[1] * xi[1] + xi[2] * xi[2];
-        double xg4[3];
         cross3(xi, A + 7, xg4);
         for (int c = 0; c < 3; c++) res[c] = A[c] + r2 * A[3 + c] + xi[c] * A[6] + xg4[c];
         qrot(q, res, lab, false);
-        for (int c = 0; c < 3; c++) scratch[it.slot + 3 * lane + c] = cSL * R * lab[c];
-    } else {
-        double A[7];
-        eval_record<kRecTrac, 26, 7>(recS, P, xi[0], xi[1], xi[2], A);
-        double xq[3];
-        cross3(xi, A + 4, xq);
-        for (int c = 0; c < 3; c++) res[c] = A[0] * xi[c] + A[1 + c] + xq[c];
-        qrot(q, res, lab, false);
-        for (int c = 0; c < 3; c++) out[3 * gp + c] = lab[c];
+        for (int c = 0; c < 3; c++) scratch[it.slot + 3 * k + c] = cSL * R * lab[c];
     }
 }
 
-// Traction evaluation of the self and near items with the source's record in
-// LDS: one workgroup of kSrcWaves waves per source sphere S runs all items
-// whose source is S (its self item and its near targets' chunks), the waves
-// taking the items in turn.  The record (kRecTrac complex arrays per term,
-// (p+3)(p+4)/2 terms: 63 KB at p = 12) is read from global memory once per
-// source instead of once per item through the scalar cache, whose loads each
-// term of the item loop waited on; with up to 256 VGPRs per lane (2 waves per
-// SIMD, which the LDS allows anyway) each term's LDS reads issue together.
-// eval_lds is eval_record with the coefficients read from LDS: the same
-// operations in the same order.
-// One launch per sphere order over that order's spheres (in k-d order), LDS
-// sized to its record; workgroup b takes list entry (b % 8) ceil(n / 8) + b / 8
+// Traction evaluation of the near items with the source's record in LDS: one
+// workgroup of kSrcWaves waves per source sphere S runs all items whose source
+// is S, the waves taking the items in turn.  The record (kRecTrac complex
+// arrays per term, (p+3)(p+4)/2 terms: 44 KB at p = 12) is read from global
+// memory once per source.  A broadcast LDS read of 16 bytes returns 16 bytes to
+// every lane, and one term is 23 of them against 46 FMAs, so the LDS return path
+// bounds a wave with one target per lane; items of more than 64 targets put two
+// on each lane, and the FP64 VALU bounds it.  With up to 256 VGPRs per lane (2
+// waves per SIMD) the reads of one batch overlap the arithmetic of the batch before.
+// One launch per sphere order over that order's spheres with near neighbours,
+// LDS sized to its record; workgroup b takes list entry (b % 8) ceil(n / 8) + b / 8
 // (XCD-contiguous, as k_sheval).
 constexpr int kSrcWaves = 4;
 
-template <int KCNT>
-__device__ __forceinline__ void eval_lds(const double2 *__restrict__ srec, int P, double x, double y, double z,
-                                         double *acc) {
+template <int CNT>
+__device__ __forceinline__ void lds_batch(const double2 *c, double2 *v) {
 #pragma unroll
-    for (int a = 0; a < KCNT; a++) acc[a] = 0.0;
-    const double r2 = x * x + y * y + z * z;
-    const double ir2 = 1.0 / r2;
-    double dmr = rsqrt_f64(r2), dmi = 0.0; // D_m^m
+    for (int a = 0; a < CNT; a++) v[a] = c[a];
+    __builtin_amdgcn_sched_barrier(0); // these reads before the arithmetic that follows
+}
+template <int N, int BEG, int CNT>
+__device__ __forceinline__ void term_batch(const double2 *v, const double *cr, const double *ci,
+                                           double (*acc)[kRecTrac]) {
+#pragma unroll
+    for (int a = 0; a < CNT; a++)
+#pragma unroll
+        for (int t = 0; t < N; t++)
+            acc[t][BEG + a] = __builtin_fma(v[a].x, cr[t], __builtin_fma(v[a].y, ci[t], acc[t][BEG + a]));
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// acc[t][a] = sum over the terms (n, m) of Re(c_a D_n^m(xi_t)).  The terms of a
+// record lie in the order of the loop (m, then n), so that a term's 23
+// coefficients are read in batches of six, each while the batch before is used:
+// left to itself the compiler waits for every read of the two-target form (its
+// registers do not hold a whole term).  srec has kSrcBatch entries of slack.
+constexpr int kSrcBatch = 6;
+template <int N>
+__device__ __forceinline__ void eval_lds(const double2 *__restrict__ srec, int P, const double (*xi)[3],
+                                         double (*acc)[kRecTrac]) {
+    static_assert(kRecTrac == 23, "batches of 6, 6, 6 and 5");
+    double nir2[N], nzi[N], dmr[N], dmi[N];
+#pragma unroll
+    for (int t = 0; t < N; t++) {
+#pragma unroll
+        for (int a = 0; a < kRecTrac; a++) acc[t][a] = 0.0;
+        const double r2 = xi[t][0] * xi[t][0] + xi[t][1] * xi[t][1] + xi[t][2] * xi[t][2];
+        nir2[t] = -1.0 / r2;
+        nzi[t] = xi[t][2] * nir2[t];
+        dmr[t] = rsqrt_f64(r2); // D_m^m
+        dmi[t] = 0.0;
+    }
+    const double2 *c = srec;
+    double2 u[kSrcBatch], v[kSrcBatch];
+    lds_batch<6>(c, u);
     for (int m = 0; m <= P; m++) {
-        if (m > 0) {
-            const double f = -(2.0 * m - 1.0) * ir2;
-            const double nr = f * (dmr * x - dmi * y), ni = f * (dmr * y + dmi * x);
-            dmr = nr;
-            dmi = ni;
-        }
-        double pr = 0.0, pi = 0.0, cr = dmr, ci = dmi;
-        const double mm = (double)m * m;
-        for (int n = m; n <= P; n++) {
-            const double2 *c = srec + kRecTrac * dtri(n, m);
+        double pr[N], pi[N], cr[N], ci[N];
 #pragma unroll
-            for (int a = 0; a < KCNT; a++) {
-                const double2 v = c[a];
-                acc[a] = __builtin_fma(v.x, cr, __builtin_fma(v.y, ci, acc[a]));
+        for (int t = 0; t < N; t++) {
+            if (m > 0) {
+                const double f = (2.0 * m - 1.0) * nir2[t];
+                const double nr = f * (dmr[t] * xi[t][0] - dmi[t] * xi[t][1]),
+                             ni = f * (dmr[t] * xi[t][1] + dmi[t] * xi[t][0]);
+                dmr[t] = nr;
+                dmi[t] = ni;
             }
-            const double f1 = -(2.0 * n + 1.0) * z * ir2, f2 = -((double)n * n - mm) * ir2;
-            const double nr = __builtin_fma(f1, cr, f2 * pr), ni = __builtin_fma(f1, ci, f2 * pi);
-            pr = cr;
-            pi = ci;
-            cr = nr;
-            ci = ni;
+            pr[t] = pi[t] = 0.0;
+            cr[t] = dmr[t];
+            ci[t] = dmi[t];
         }
+        double odd = 2.0 * m + 1.0, nm = 0.0; // 2 n + 1, n^2 - m^2
+        for (int n = m; n <= P; n++, c += kRecTrac) {
+            lds_batch<6>(c + 6, v);
+            term_batch<N, 0, 6>(u, cr, ci, acc);
+            lds_batch<6>(c + 12, u);
+            term_batch<N, 6, 6>(v, cr, ci, acc);
+            lds_batch<5>(c + 18, v);
+            term_batch<N, 12, 6>(u, cr, ci, acc);
+            lds_batch<6>(c + 23, u);
+            term_batch<N, 18, 5>(v, cr, ci, acc);
+#pragma unroll
+            for (int t = 0; t < N; t++) {
+                const double f1 = odd * nzi[t], f2 = nm * nir2[t];
+                const double nr = __builtin_fma(f1, cr[t], f2 * pr[t]), ni = __builtin_fma(f1, ci[t], f2 * pi[t]);
+                pr[t] = cr[t];
+                pi[t] = ci[t];
+                cr[t] = nr;
+                ci[t] = ni;
+            }
+            nm += odd;
+            odd += 2.0;
+        }
+    }
+}
+
+// targets k = lane, lane + 64, ... (N of them; those beyond the item repeat its first) of one item
+template <int N>
+__device__ __forceinline__ void eval_item(const DevGeom &g, const EvalItem &it, const double2 *srec, int P,
+                                          const double *q, const double *cen, double iR, double cTrac, int lane,
+                                          double *__restrict__ scratch) {
+    const int64_t g0 = g.pt_off[it.trg] + it.tstart;
+    double xi[N][3], vb[N][3], A[N][kRecTrac];
+#pragma unroll
+    for (int t = 0; t < N; t++) {
+        const int k = lane + 64 * t;
+        const int64_t gp = g0 + (k < it.tcount ? k : 0);
+        const double d[3] = {(g.coords[3 * gp] - cen[0]) * iR, (g.coords[3 * gp + 1] - cen[1]) * iR,
+                             (g.coords[3 * gp + 2] - cen[2]) * iR};
+        const double Nl[3] = {g.norms[3 * gp], g.norms[3 * gp + 1], g.norms[3 * gp + 2]};
+        qrot(q, d, xi[t], true);
+        qrot(q, Nl, vb[t], true);
+    }
+    eval_lds<N>(srec, P, xi, A);
+#pragma unroll
+    for (int t = 0; t < N; t++) {
+        const int k = lane + 64 * t;
+        double res[3], lab[3];
+        traction_from(A[t], xi[t], vb[t], res);
+        qrot(q, res, lab, false);
+        if (k < it.tcount)
+            for (int c = 0; c < 3; c++) scratch[it.slot + 3 * k + c] = cTrac * lab[c];
     }
 }
 
@@ -870,7 +893,6 @@ __global__ __launch_bounds__(64 * kSrcWaves) __attribute__((amdgpu_waves_per_eu(
     // near pairs lie within one suspension: the test is uniform over the workgroup
     if (active && !active[g.sph_susp[S]]) return;
     const int64_t i0 = src_off[S], i1 = src_off[S + 1];
-    if (i0 == i1) return;
     const int P = g.order[S] + 2;
     const int nrec = kRecTrac * ((P + 1) * (P + 2) / 2);
     const double2 *recS = reinterpret_cast<const double2 *>(rec + g.rec_off[S]);
@@ -878,34 +900,14 @@ __global__ __launch_bounds__(64 * kSrcWaves) __attribute__((amdgpu_waves_per_eu(
     __syncthreads();
     const int lane = threadIdx.x & 63;
     const double *q = g.quat + 4 * S;
-    const double R = g.rad[S];
-    const double iR = 1.0 / R;
-    const double cx = g.pos[3 * S], cy = g.pos[3 * S + 1], cz = g.pos[3 * S + 2];
+    const double iR = 1.0 / g.rad[S];
+    const double cen[3] = {g.pos[3 * S], g.pos[3 * S + 1], g.pos[3 * S + 2]};
     for (int64_t k = i0 + (threadIdx.x >> 6); k < i1; k += kSrcWaves) {
         const EvalItem it = items[k];
-        if (lane >= it.tcount) continue;
-        const int T = it.trg;
-        const int64_t gp = g.pt_off[T] + it.tstart + lane;
-        const double d[3] = {(g.coords[3 * gp] - cx) * iR, (g.coords[3 * gp + 1] - cy) * iR,
-                             (g.coords[3 * gp + 2] - cz) * iR};
-        const double Nl[3] = {g.norms[3 * gp], g.norms[3 * gp + 1], g.norms[3 * gp + 2]};
-        double xi[3], vb[3], res[3], lab[3];
-        qrot(q, d, xi, true);
-        qrot(q, Nl, vb, true);
-        if (T == S) {
-            double A[kRecTrac];
-            eval_lds<kRecTrac>(srec, P, xi[0], xi[1], xi[2], A);
-            traction_from(A, xi, vb, res);
-            double xq[3];
-            cross3(xi, A + 30, xq);
-            for (int c = 0; c < 3; c++) res[c] += 0.5 * (A[26] * xi[c] + A[27 + c] + xq[c]);
-        } else {
-            double A[kRecTracNear];
-            eval_lds<kRecTracNear>(srec, P, xi[0], xi[1], xi[2], A);
-            traction_from(A, xi, vb, res);
-        }
-        qrot(q, res, lab, false);
-        for (int c = 0; c < 3; c++) scratch[it.slot + 3 * lane + c] = cTrac * lab[c];
+        if (it.tcount > 64)
+            eval_item<2>(g, it, srec, P, q, cen, iR, cTrac, lane, scratch);
+        else
+            eval_item<1>(g, it, srec, P, q, cen, iR, cTrac, lane, scratch);
     }
 }
 
@@ -965,7 +967,7 @@ void launch_sheval_items(const DevGeom &g, int mode, const double *rec, const Ev
             const int a = by_src->order_off[p], n = by_src->order_off[p + 1] - a;
             if (n <= 0) continue;
             const int P = p + 2;
-            const size_t lds = sizeof(double2) * kRecTrac * ((P + 1) * (P + 2) / 2);
+            const size_t lds = sizeof(double2) * (kRecTrac * ((P + 1) * (P + 2) / 2) + kSrcBatch);
             static size_t lds_set = 0;
             if (lds > 65536 && lds > lds_set) {
                 if (hipFuncSetAttribute((const void *)k_sheval_src, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -979,8 +981,7 @@ void launch_sheval_items(const DevGeom &g, int mode, const double *rec, const Ev
         }
         return;
     }
-    k_sheval<0><<<dim3(8 * ((nitems + 7) / 8)), dim3(64), 0, s>>>(g, rec, items, nitems, scratch, nullptr, cSL,
-                                                                   cTrac, active);
+    k_sheval<<<dim3(8 * ((nitems + 7) / 8)), dim3(64), 0, s>>>(g, rec, items, nitems, scratch, cSL, active);
 }
 
 void launch_sheval_gather(const DevGeom &g, const int64_t *trg_slot_off, const int *trg_nsrc, const double *scratch,
@@ -989,13 +990,6 @@ void launch_sheval_gather(const DevGeom &g, const int64_t *trg_slot_off, const i
     if (!g.nsph) return;
     k_sheval_gather<<<dim3(g.nsph), dim3(256), 0, s>>>(g, trg_slot_off, trg_nsrc, scratch, far, in, out, cId, cLOP,
                                                       overwrite ? 1 : 0, active);
-}
-
-void launch_synthesis(const DevGeom &g, const double *rec, const EvalItem *self_items, int nitems, double *out,
-                      hipStream_t s, const int *active) {
-    if (!g.nsph || nitems <= 0) return;
-    k_sheval<2><<<dim3(8 * ((nitems + 7) / 8)), dim3(64), 0, s>>>(g, rec, self_items, nitems, nullptr, out, 0.0, 0.0,
-                                                                  active);
 }
 
 __global__ void k_identity(DevGeom g, const double *__restrict__ in, double *__restrict__ out, double cId,

@@ -29,13 +29,14 @@ struct DevGeom {
     const int *sph_susp = nullptr; // N
     const int64_t *pt_off = nullptr;   // N+1
     const int64_t *coef_off = nullptr; // N+1 (6Q doubles per sphere)
-    const int64_t *rec_off = nullptr;  // N+1 (2*kRecTrac*tri(p+2) doubles per sphere)
+    const int64_t *rec_off = nullptr;  // N+1 (2*kRecTrac*tri(p+2) doubles per sphere with near neighbours)
     const double *coords = nullptr;    // 3P lab
     const double *norms = nullptr;     // 3P lab
     const double *w = nullptr;         // P
     const int64_t *near_off = nullptr; // N+1
     const int *near_src = nullptr;
     const int64_t *body_off = nullptr; // per tile: first element of its body-frame grid values (see body_cols)
+    const int64_t *coef_body_off = nullptr; // per tile: first element of its coefficients in the same layout
 };
 
 // Chunks of the DOF vector used by the segmented BLAS-1 kernels.
@@ -98,20 +99,24 @@ void launch_equiv_forces(int ncell, int K, int Kc, const double *P, const double
 // the source records src64 / src32 (NULL: not wanted).
 void launch_pack_body(const DevGeom &g, const double *in, double *bd, float *bf, double *src64, float *src32,
                       int max_points, hipStream_t s);
-void launch_analysis(const DevGeom &g, const ShGemm &M, const double *body, double *coef, const int *active,
-                     hipStream_t s);
+// coef: per sphere; cbody: the same as GEMM columns (per tile)
+void launch_analysis(const DevGeom &g, const ShGemm &M, const double *body, double *coef, double *cbody,
+                     const int *active, hipStream_t s);
+// out[mul dst_off[S] + 3 point + c] = coef R_S^rpow (M coefficients of S), lab frame: M a
+// synthesis with per-degree blocks (a sphere's operator on its own surface)
+void launch_synthesis(const DevGeom &g, const ShGemm &M, const double *cbody, const int64_t *dst_off, int mul,
+                      double coef, int rpow, double *out, const int *active, hipStream_t s);
 void launch_levels_down(const DevGeom &g, const ShGemm &M, bool fp64, const void *body, const LevelViews &L,
                         const int *active, hipStream_t s);
 void launch_pack_levels(const DevGeom &g, bool fp64, const LevelViews &L, void *body, int max_points, hipStream_t s);
 // out += the level fields on the fine grids
 void launch_levels_up(const DevGeom &g, const ShGemm &M, bool fp64, const void *body, const LevelViews &L, double *out,
                       const int *active, hipStream_t s);
-// per sphere and degree n: (F_r, F_s) <- 2x2 block tab[5n..5n+3], F_t <- tab[5n+4] F_t (in place)
-void launch_degree_blocks(const DevGeom &g, double *coef, const double *tab, const int *active, hipStream_t s);
 // mode 0: single-layer record (kRecSL arrays), 1: traction record (kRecTrac arrays)
-void launch_expand(const DevGeom &g, int mode, const double *coef, double *rec, const int *active, hipStream_t s,
-                   int max_order);
-// One self/near evaluation work item: targets [tstart, tstart+tcount) (<= 64) of
+// of the n spheres in list
+void launch_expand(const DevGeom &g, int mode, const int *list, int n, const double *coef, double *rec,
+                   const int *active, hipStream_t s, int max_order);
+// One near evaluation work item: targets [tstart, tstart+tcount) (<= 128) of
 // sphere trg against the expansion of sphere src; its contribution goes to
 // scratch[slot ...] (3 doubles per target).
 struct EvalItem {
@@ -123,8 +128,8 @@ struct EvalItem {
 // The same items grouped by source sphere: source S owns items
 // [src_off[S], src_off[S + 1]).  The traction evaluation (mode 1) runs one
 // workgroup per source with the source's record staged in LDS, one launch per
-// sphere order (LDS sized to that order's record): srcs lists the spheres by
-// order, those of order p at [order_off[p], order_off[p + 1]).
+// sphere order (LDS sized to that order's record): srcs lists the spheres that
+// have items by order, those of order p at [order_off[p], order_off[p + 1]).
 struct SrcItems {
     const EvalItem *items = nullptr;
     const int64_t *src_off = nullptr;
@@ -139,7 +144,7 @@ struct FarSum {
     int64_t stride = 0;
 };
 
-// per-item self/near evaluations (mode 0: cSL single layer, 1: cTrac traction) into scratch
+// per-item near evaluations (mode 0: cSL single layer, 1: cTrac traction) into scratch
 void launch_sheval_items(const DevGeom &g, int mode, const double *rec, const EvalItem *items, int nitems,
                          double *scratch, double cSL, double cTrac, const int *active, hipStream_t s,
                          const SrcItems *by_src = nullptr);
@@ -151,10 +156,6 @@ void launch_sheval_gather(const DevGeom &g, const int64_t *trg_slot_off, const i
 void launch_identity(const DevGeom &g, const double *in, double *out, double cId, const int *active,
                      hipStream_t s);
 void launch_lop(const DevGeom &g, const double *in, double *out, double cLOP, const int *active, hipStream_t s);
-// out = P in (grid values of the band-limited projection) from a traction record (self items only)
-void launch_synthesis(const DevGeom &g, const double *rec, const EvalItem *self_items, int nitems, double *out,
-                      hipStream_t s, const int *active = nullptr);
-
 // segmented BLAS-1 over chunks (one segment per suspension)
 void launch_seg_dot(const double *a, const double *b, const Chunk *chunks, int nchunks, double *partial,
                     const int *active, hipStream_t s);

@@ -125,6 +125,27 @@ std::vector<double> pole_rows(int p) {
     return rows;
 }
 
+std::vector<double> synthesis_of_blocks(int p, const std::vector<double> &blocks) {
+    const ShTables &t = sh_tables(p);
+    const size_t n3 = 3 * (size_t)t.npts;
+    std::vector<double> m(n3 * 6 * t.Q);
+    for (int n = 0; n <= p; n++)
+        for (int k = tri(n, 0); k < tri(n + 1, 0); k++)
+            for (int c = 0; c < 2; c++) {
+                const double *b = &blocks[5 * n];
+                const double *sr = &t.synth[n3 * (2 * k + c)], *ss = &t.synth[n3 * (2 * t.Q + 2 * k + c)],
+                             *st = &t.synth[n3 * (4 * t.Q + 2 * k + c)];
+                double *mr = &m[n3 * (2 * k + c)], *ms = &m[n3 * (2 * t.Q + 2 * k + c)],
+                       *mt = &m[n3 * (4 * t.Q + 2 * k + c)];
+                for (size_t i = 0; i < n3; i++) {
+                    mr[i] = b[0] * sr[i] + b[2] * ss[i];
+                    ms[i] = b[1] * sr[i] + b[3] * ss[i];
+                    mt[i] = b[4] * st[i];
+                }
+            }
+    return m;
+}
+
 static std::unique_ptr<ShTables> build_tables(int p) {
     auto t = std::make_unique<ShTables>();
     t->p = p;

@@ -4,6 +4,8 @@
 //   analysis     coef[S] = A_p q_S^-1 in_S                  (Shexp::calcSpectralCoeff, Sphere/Shexp.cpp:408-447)
 //   level down   level sources of S = w q_S D_p q_S^-1 in_S (D_p: all levels' resampling matrices, stacked by rows)
 //   level up     out_S += q_S U_p q_S^-1 levels_S           (U_p: the same, stacked by columns)
+//   synthesis    out_S = q_S Y_p coef[S]                    (Y_p: with per-degree blocks, the operators of a sphere on
+//                                                            its own surface, Sphere/Shexp.cpp:503-624)
 //
 // A workgroup computes 48 matrix rows (16 points x 3 components, or 48
 // coefficients) for one tile of 16 spheres; its four waves split the columns
@@ -112,7 +114,13 @@ __global__ __launch_bounds__(256) void k_pack_levels(DevGeom g, LevelViews L, T 
         if (3 * k + c < cols) body[base + body_at(3 * k + c, t)] = (T)o[c];
 }
 
-enum { ANALYSIS, LEVEL_DOWN, LEVEL_UP };
+enum { ANALYSIS, LEVEL_DOWN, LEVEL_UP, SYNTHESIS };
+
+struct SynthOut {
+    const int64_t *off;
+    int mul, rpow;
+    double coef;
+};
 
 // blockIdx.x: row block of 48, blockIdx.y: tile.  Operands of the 16x16x4
 // instructions: A[i][k] in lane i + 16k, B[k][j] in lane j + 16k; D[i][j] in lane
@@ -122,7 +130,8 @@ enum { ANALYSIS, LEVEL_DOWN, LEVEL_UP };
 // 48 w + 16 rb + i of the analysis.
 template <typename T, int KIND>
 __global__ __launch_bounds__(256) void k_sh_gemm(DevGeom g, ShGemm M, const int64_t *__restrict__ body_off,
-                                                 const T *__restrict__ body, LevelViews L, double *__restrict__ out,
+                                                 const T *__restrict__ body, LevelViews L, SynthOut Y,
+                                                 double *__restrict__ out, double *__restrict__ cbody,
                                                  const int *__restrict__ active) {
     typedef T T4 __attribute__((ext_vector_type(4)));
     __shared__ T red[4][12][64];
@@ -168,7 +177,10 @@ __global__ __launch_bounds__(256) void k_sh_gemm(DevGeom g, ShGemm M, const int6
         const int rows = 3 * (p + 1) * (p + 2);
         for (int rb = 0; rb < 3; rb++) {
             const int r = 48 * w + 16 * rb + i;
-            if (r < rows) out[g.coef_off[S] + r] = v[rb];
+            if (r < rows) {
+                out[g.coef_off[S] + r] = v[rb];
+                cbody[g.coef_body_off[blockIdx.y] + body_at(r, t)] = v[rb];
+            }
         }
         return;
     }
@@ -179,6 +191,13 @@ __global__ __launch_bounds__(256) void k_sh_gemm(DevGeom g, ShGemm M, const int6
         if (j >= (p + 1) * (2 * p + 2)) return;
         double *dst = out + 3 * (g.pt_off[S] + j);
         for (int c = 0; c < 3; c++) dst[c] += o[c];
+        return;
+    }
+    if (KIND == SYNTHESIS) {
+        if (j >= (p + 1) * (2 * p + 2)) return;
+        const double f = Y.rpow ? Y.coef * g.rad[S] : Y.coef;
+        double *dst = out + Y.mul * Y.off[S] + 3 * j;
+        for (int c = 0; c < 3; c++) dst[c] = f * o[c];
         return;
     }
     const int *first = L.first[p];
@@ -209,11 +228,18 @@ void launch_pack_body(const DevGeom &g, const double *in, double *bd, float *bf,
         k_pack_body<false, true><<<grid, dim3(256), 0, s>>>(g, in, bd, bf, src64, src32);
 }
 
-void launch_analysis(const DevGeom &g, const ShGemm &M, const double *body, double *coef, const int *active,
-                     hipStream_t s) {
+void launch_analysis(const DevGeom &g, const ShGemm &M, const double *body, double *coef, double *cbody,
+                     const int *active, hipStream_t s) {
     if (!g.nsph || !g.ntiles) return;
     k_sh_gemm<double, ANALYSIS><<<dim3(M.max_blk, g.ntiles), dim3(256), 0, s>>>(g, M, g.body_off, body, LevelViews{},
-                                                                               coef, active);
+                                                                               SynthOut{}, coef, cbody, active);
+}
+
+void launch_synthesis(const DevGeom &g, const ShGemm &M, const double *cbody, const int64_t *dst_off, int mul,
+                      double coef, int rpow, double *out, const int *active, hipStream_t s) {
+    if (!g.nsph || !g.ntiles) return;
+    k_sh_gemm<double, SYNTHESIS><<<dim3(M.max_blk, g.ntiles), dim3(256), 0, s>>>(
+        g, M, g.coef_body_off, cbody, LevelViews{}, SynthOut{dst_off, mul, rpow, coef}, out, nullptr, active);
 }
 
 void launch_levels_down(const DevGeom &g, const ShGemm &M, bool fp64, const void *body, const LevelViews &L,
@@ -221,11 +247,11 @@ void launch_levels_down(const DevGeom &g, const ShGemm &M, bool fp64, const void
     if (!g.nsph || !g.ntiles) return;
     const dim3 grid(M.max_blk, g.ntiles);
     if (fp64)
-        k_sh_gemm<double, LEVEL_DOWN><<<grid, dim3(256), 0, s>>>(g, M, g.body_off, (const double *)body, L, nullptr,
-                                                                active);
+        k_sh_gemm<double, LEVEL_DOWN><<<grid, dim3(256), 0, s>>>(g, M, g.body_off, (const double *)body, L, SynthOut{},
+                                                                nullptr, nullptr, active);
     else
-        k_sh_gemm<float, LEVEL_DOWN><<<grid, dim3(256), 0, s>>>(g, M, g.body_off, (const float *)body, L, nullptr,
-                                                               active);
+        k_sh_gemm<float, LEVEL_DOWN><<<grid, dim3(256), 0, s>>>(g, M, g.body_off, (const float *)body, L, SynthOut{},
+                                                               nullptr, nullptr, active);
 }
 
 void launch_pack_levels(const DevGeom &g, bool fp64, const LevelViews &L, void *body, int max_points, hipStream_t s) {
@@ -242,9 +268,11 @@ void launch_levels_up(const DevGeom &g, const ShGemm &M, bool fp64, const void *
     if (!g.nsph || !g.ntiles) return;
     const dim3 grid(M.max_blk, g.ntiles);
     if (fp64)
-        k_sh_gemm<double, LEVEL_UP><<<grid, dim3(256), 0, s>>>(g, M, L.body_off, (const double *)body, L, out, active);
+        k_sh_gemm<double, LEVEL_UP><<<grid, dim3(256), 0, s>>>(g, M, L.body_off, (const double *)body, L, SynthOut{}, out,
+                                                              nullptr, active);
     else
-        k_sh_gemm<float, LEVEL_UP><<<grid, dim3(256), 0, s>>>(g, M, L.body_off, (const float *)body, L, out, active);
+        k_sh_gemm<float, LEVEL_UP><<<grid, dim3(256), 0, s>>>(g, M, L.body_off, (const float *)body, L, SynthOut{}, out,
+                                                             nullptr, active);
 }
 
 } // namespace sphstk
