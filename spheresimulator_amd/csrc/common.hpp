@@ -71,6 +71,10 @@ struct ShTables {
 };
 
 const ShTables &sh_tables(int p);
+// The tables of degree q on the grid of a far-field level: as many points as a
+// rule needs that integrates degree 2q (fewer than the Gauss-Legendre grid of
+// order q, whose rings crowd at the poles), for orders without one that grid.
+const ShTables &level_tables(int q);
 
 // The synthesis rows at the body-frame poles +z and -z: 6 rows (north x, y, z,
 // south x, y, z) of 6Q coefficients each, row-major.
@@ -90,6 +94,8 @@ struct Resample {
     std::vector<double> down, up;
 };
 const Resample &resample_tables(int p, int pc);
+// The same to and from the level grid of degree pc <= p (no identity at pc == p).
+const Resample &level_resample(int p, int pc);
 void gauss_legendre(int n, std::vector<double> &x, std::vector<double> &w);
 
 // Equivalent-source template of the far-field cell aggregation (equiv.cpp):

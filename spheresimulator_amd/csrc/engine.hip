@@ -538,6 +538,7 @@ void Operator::autotune_inner(double &budget_s) {
         LevelSet keep = std::move(ls32_);
         ls32_.tpl = tpl;
         ls32_.nlev = keep.nlev;
+        ls32_.first_level = keep.first_level;
         std::copy(keep.alo, keep.alo + kMaxLevels, ls32_.alo);
         std::copy(keep.order, keep.order + kMaxLevels, ls32_.order);
         ls32_.fp64 = false;
@@ -945,8 +946,22 @@ void kd_order(const double *pos, int *idx, int b, int e, int leaf) {
 void Operator::ensure_levels(LevelSet &S) {
     if (S.ready) return;
     PhaseTimer pt(S.fp64 ? "FP64 outer level set" : "FP32 inner level set");
+    drop_fine_levels(S);
     const double *a = S.alo;
-    auto lorder = [&](int l, int p) { return S.order[l] < 0 ? level_order(l, p) : std::min(p, S.order[l]); };
+    // points of a sphere on each level, and those of the Gauss-Legendre grid of
+    // the same order, by which the use of source cells is decided: the cells'
+    // fit also carries degrees that the two coarsest levels drop (1500 spheres
+    // p=12 in chains: inner operator 4.6e-6 off with them, 5.1e-6 without), so
+    // they stay where they were worth it before the levels had fewer points
+    std::vector<std::array<int, kMaxOrder + 1>> level_points(S.nlev, std::array<int, kMaxOrder + 1>{}), weight = level_points;
+    for (int l = 0; l < S.nlev; l++)
+        for (int p : order_)
+            if (!level_points[l][p]) {
+                const ShTables &t = level_grid(S, l, p);
+                level_points[l][p] = t.npts;
+                weight[l][p] = grid_points(t.p);
+            }
+    auto lpoints = [&](int l, int p) { return level_points[l][p]; };
     // k-d order of the spheres within each suspension
     std::vector<int> perm(nsph_), rank(nsph_);
     for (int i = 0; i < nsph_; i++) perm[i] = i;
@@ -960,7 +975,7 @@ void Operator::ensure_levels(LevelSet &S) {
     // mid runs in sphere index space.
     auto tn = std::make_unique<PhaseTimer>("  level pair classes");
     std::vector<Runs> mid(nsph_);
-    const int nlev = S.nlev;
+    const int nlev = S.nlev, c0 = nlev - 2; // source cells serve the last two levels
     std::vector<std::vector<Runs>> lvl(nlev, std::vector<Runs>(nsph_));
     std::vector<int> sph_s0(nsph_), sph_s1(nsph_);
     for (int b = 0; b < nsusp_; b++)
@@ -1053,16 +1068,15 @@ void Operator::ensure_levels(LevelSet &S) {
                     if (std::sqrt(ex * ex + ey * ey + ez * ez) >= S.cell_theta * crho[c] + rad_[t]) {
                         int lmin = nlev;
                         double member_pairs = 0.0;
-                        for (int r = cell_r0[c]; r < cell_r1[c] && lmin >= 2; r++) {
+                        for (int r = cell_r0[c]; r < cell_r1[c] && lmin >= c0; r++) {
                             const int sm = perm[r], lm = klass(t, sm);
                             lmin = std::min(lmin, lm);
                             if (lm >= 0)
-                                member_pairs += double(grid_points(lorder(lm, order_[sm]))) *
-                                                grid_points(lorder(lm, order_[t]));
+                                member_pairs += double(weight[lm][order_[sm]]) * weight[lm][order_[t]];
                         }
-                        if (lmin >= 2) {
-                            run_append(crun[rt][lmin - 2], (int)c);
-                            saved[t] += member_pairs - double(Keq) * grid_points(lorder(lmin, order_[t]));
+                        if (lmin >= c0) {
+                            run_append(crun[rt][lmin - c0], (int)c);
+                            saved[t] += member_pairs - double(Keq) * weight[lmin][order_[t]];
                             continue;
                         }
                     }
@@ -1115,14 +1129,13 @@ void Operator::ensure_levels(LevelSet &S) {
         std::vector<int64_t> off_by_sph(nsph_);
         for (int r = 0; r < nsph_; r++) {
             const int s = perm[r];
-            const int p = order_[s], pc = lorder(l, p);
-            off[r + 1] = off[r] + grid_points(pc);
+            off[r + 1] = off[r] + lpoints(l, order_[s]);
             off_by_sph[s] = off[r];
         }
         const int64_t nc = off[nsph_];
         std::vector<double> cc(3 * nc), cn(3 * nc), cw(nc);
         for (int s = 0; s < nsph_; s++) {
-            const ShTables &t = sh_tables(lorder(l, order_[s]));
+            const ShTables &t = level_grid(S, l, order_[s]);
             for (int q = 0; q < t.npts; q++) {
                 const int64_t g = off_by_sph[s] + q;
                 double nv[3];
@@ -1239,7 +1252,7 @@ void Operator::ensure_levels(LevelSet &S) {
         for (int i = 0; i < 2; i++) {
             std::vector<Runs> runs(nsph_);
             for (int r = 0; r < nsph_; r++) runs[r] = crun[r][i];
-            build_far_lists(A->lists[i], nsusp_, susp_sph_off_, level_off[2 + i], eq_off, runs, S.tpl, 0, kWantItems,
+            build_far_lists(A->lists[i], nsusp_, susp_sph_off_, level_off[c0 + i], eq_off, runs, S.tpl, 0, kWantItems,
                             nullptr, &susp_cell_off);
             A->lists[i].slots();
             A->pairs += A->lists[i].pairs;
@@ -1255,11 +1268,44 @@ void Operator::ensure_levels(LevelSet &S) {
         V.stride[l] = 3 * L.npts;
         V.part[l][0] = L.lists.part.p;
         V.nslot[l][0] = L.lists.nslot();
-        const FarLists *C = S.agg && l >= 2 ? &S.agg->lists[l - 2] : nullptr;
+        const FarLists *C = S.agg && l >= c0 ? &S.agg->lists[l - c0] : nullptr;
         V.part[l][1] = C ? C->part.p : nullptr;
         V.nslot[l][1] = C ? C->nslot() : 0;
     }
     S.ready = true;
+}
+
+// A level of order q serves spheres of higher order p on the level grid of q;
+// the others keep their own grid there (-1), which truncates nothing.
+static int order_on_level(const LevelSet &S, int l, int p) {
+    const int q = S.order[l] < 0 ? level_order(S.first_level + l, p) : S.order[l];
+    return q < p ? q : -1;
+}
+const ShTables &Operator::level_grid(const LevelSet &S, int l, int p) const {
+    const int q = order_on_level(S, l, p);
+    return q < 0 ? sh_tables(p) : level_tables(q);
+}
+const Resample &Operator::level_matrices(const LevelSet &S, int l, int p) const {
+    const int q = order_on_level(S, l, p);
+    return q < 0 ? resample_tables(p, p) : level_resample(p, q);
+}
+
+// Levels on which every sphere keeps its own grid are the fine grid: their pairs
+// go to the list of the pairs closer than the first level (spheres of order 8:
+// the first FP32 level and the first levels of the FP64 set).
+void Operator::drop_fine_levels(LevelSet &S) const {
+    std::vector<bool> used(kMaxOrder + 1, false);
+    for (int p : order_) used[p] = true;
+    while (S.nlev > 2) {
+        for (int p = 0; p <= kMaxOrder; p++)
+            if (used[p] && order_on_level(S, 0, p) >= 0) return;
+        for (int l = 1; l < S.nlev; l++) {
+            S.alo[l - 1] = S.alo[l];
+            S.order[l - 1] = S.order[l];
+        }
+        S.nlev--;
+        S.first_level++;
+    }
 }
 
 // The resampling matrices between the fine grids and all levels of a set as one
@@ -1278,9 +1324,8 @@ void Operator::level_transforms(LevelSet &S) {
         std::vector<const Resample *> rs;
         std::vector<int> key{p};
         for (int l = 0; l < S.nlev; l++) {
-            const int pc = S.order[l] < 0 ? level_order(l, p) : std::min(p, S.order[l]);
-            rs.push_back(&resample_tables(p, pc));
-            key.push_back(pc);
+            rs.push_back(&level_matrices(S, l, p));
+            key.push_back(order_on_level(S, l, p));
             V.first[p][l + 1] = V.first[p][l] + rs[l]->nc;
         }
         const int n = rs[0]->n, nl = V.first[p][S.nlev];
@@ -1372,7 +1417,7 @@ void Operator::far_levels(LevelSet &S, int kind, double coef, const int *active,
     if (ev_a) SPHSTK_HIP(hipEventRecord(ev_a, stream_));
     if (A)
         for (int i = 0; i < 2; i++)
-            far_slots(A->lists[i], kind, 1, A->eq32.p, nullptr, nullptr, S.levels[2 + i]->trg32.p, coef, active);
+            far_slots(A->lists[i], kind, 1, A->eq32.p, nullptr, nullptr, S.levels[S.nlev - 2 + i]->trg32.p, coef, active);
     for (auto &L : S.levels) {
         if (S.fp64)
             far_slots(L->lists, kind, 0, L->src64.p, L->coords.p, L->norms.p, nullptr, coef, active);

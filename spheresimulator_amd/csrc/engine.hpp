@@ -151,6 +151,7 @@ struct CellAgg {
 constexpr int kNumLevels = 4; // levels of the FP32 sets (source cells on their last two)
 struct LevelSet {
     int nlev = kNumLevels;   // levels in use
+    int first_level = 0;     // levels dropped before them (drop_fine_levels)
     double alo[kMaxLevels];  // separations (in units of R_s + R_t) where levels 0..nlev-1 start
     int order[kMaxLevels];   // grid order of each level (capped by the sphere's order)
     bool fp64 = false;       // FP64 pair sums (else FP32)
@@ -163,7 +164,7 @@ struct LevelSet {
     DevBuf<int64_t> d_body_off;       // per tile: body-frame values of its level points
     DevBuf<double> body64;            // those values (FP64 set, FP32 sets)
     DevBuf<float> body32;
-    bool cells = false;               // aggregate sources over cells on levels 2-3
+    bool cells = false;               // aggregate sources over cells on the last two levels
     double cell_theta = kCellTheta;   // cells serve targets beyond cell_theta cell radii
     int equiv_k = kEquivK;            // equivalent point forces per cell
     std::unique_ptr<CellAgg> agg;
@@ -285,6 +286,11 @@ class Operator {
                  const float *trg32, const Chunk *chunks, int nchunks, double coef, double *out, const int *active);
     void ensure_levels(LevelSet &S);
     void level_transforms(LevelSet &S);
+    // grid of a sphere of order p on level l of a set, and the matrices between
+    // it and the fine grid
+    const ShTables &level_grid(const LevelSet &S, int l, int p) const;
+    const Resample &level_matrices(const LevelSet &S, int l, int p) const;
+    void drop_fine_levels(LevelSet &S) const;
     void far_copies(int kind, double coef, const double *in, const int *active, hipEvent_t ev_a);
     // tile-shape autotuner: times candidate work-list shapes on this problem
     void autotune_fine(double &budget_s);

@@ -146,6 +146,9 @@ std::vector<double> synthesis_of_blocks(int p, const std::vector<double> &blocks
     return m;
 }
 
+// Analysis and synthesis matrices of degree p on the points and weights of t.
+static void fill_matrices(ShTables *t, int p);
+
 static std::unique_ptr<ShTables> build_tables(int p) {
     auto t = std::make_unique<ShTables>();
     t->p = p;
@@ -167,6 +170,111 @@ static std::unique_ptr<ShTables> build_tables(int p) {
             t->w[q] = 2.0 * kPi / nphi * wg[p - j];
         }
     }
+    fill_matrices(t.get(), p);
+    return t;
+}
+
+// Quadrature rules on the sphere with octahedral symmetry (the structure is
+// Lebedev's, Zh. Vychisl. Mat. Mat. Fiz. 16 (1976)): per orbit a point, its
+// coordinates in ascending order, and the weight of each of its images under
+// permutations and signs, the weights of a rule adding up to one.  Solved by
+// Newton's method from random starts on the moments of (x^4 + y^4 + z^4)^a
+// (xyz)^2b, which span the invariant polynomials on the sphere.  A rule for
+// order q integrates degree 2q + 1, as the Gauss-Legendre grid of 2 (q + 1)^2
+// points does, with about two thirds of its points: a far-field level evaluates
+// the product of two spheres' points.
+struct Orbit {
+    double x, y, z, w;
+};
+static const std::vector<Orbit> kRules[] = {
+    // order 1: 6 points (degree 3)
+    {{0.0, 0.0, 1.0, 0.16666666666666666}},
+    // order 2: 14 points (degree 5)
+    {{0.0, 0.0, 1.0, 0.06666666666666611},
+     {0.5773502691896258, 0.5773502691896258, 0.5773502691896258, 0.07500000000000041}},
+    // order 3: 26 points (degree 7)
+    {{0.0, 0.0, 1.0, 0.047619047619047006},
+     {0.0, 0.7071067811865475, 0.7071067811865475, 0.03809523809523829},
+     {0.5773502691896258, 0.5773502691896258, 0.5773502691896258, 0.0321428571428573}},
+    // order 4: 38 points (degree 9)
+    {{0.0, 0.0, 1.0, 0.00952380952380907},
+     {0.5773502691896258, 0.5773502691896258, 0.5773502691896258, 0.0321428571428573},
+     {0.0, 0.45970084338098427, 0.8880738339771146, 0.028571428571428636}},
+    // order 5: 50 points (degree 11)
+    {{0.0, 0.0, 1.0, 0.012698412698412223},
+     {0.0, 0.7071067811865475, 0.7071067811865475, 0.022574955908289444},
+     {0.5773502691896258, 0.5773502691896258, 0.5773502691896258, 0.021093750000000102},
+     {0.30151134457776424, 0.30151134457776424, 0.9045340337332904, 0.02017333553791886}},
+    // order 6: 74 points (degree 13)
+    {{0.0, 0.0, 1.0, 0.000513067179731495},
+     {0.0, 0.7071067811865475, 0.7071067811865475, 0.016604069565742573},
+     {0.5773502691896258, 0.5773502691896258, 0.5773502691896258, -0.02958603896103527},
+     {0.4803844614152578, 0.4803844614152578, 0.7337993857053474, 0.026576207082158427},
+     {0.0, 0.3207726489807671, 0.947156221362591, 0.016522170993715835}},
+    // order 7: 86 points (degree 15)
+    {{0.0, 0.0, 1.0, 0.01154401154401075},
+     {0.5773502691896258, 0.5773502691896258, 0.5773502691896258, 0.011943909085856397},
+     {0.1890635528853951, 0.6943540066026664, 0.6943540066026664, 0.011876501294537375},
+     {0.3696028464541496, 0.3696028464541496, 0.8525183117012681, 0.0111105557106034},
+     {0.0, 0.37424303909033896, 0.9273306571511734, 0.011812303746904403}},
+    // order 8: 110 points (degree 17)
+    {{0.0, 0.0, 1.0, 0.003828270494933668},
+     {0.5773502691896258, 0.5773502691896258, 0.5773502691896258, 0.009793737512487627},
+     {0.1851156353447231, 0.1851156353447231, 0.9651240350865992, 0.00821173728319195},
+     {0.39568947305593716, 0.39568947305593716, 0.8287699812525967, 0.009595471336071065},
+     {0.21595729184585932, 0.6904210483822905, 0.6904210483822905, 0.009942814891177858},
+     {0.0, 0.47836902881216736, 0.8781589106040568, 0.00969499636166317}},
+    // order 9: 146 points (degree 19)
+    {{0.0, 0.0, 1.0, 0.0005996313688613017},
+     {0.0, 0.7071067811865475, 0.7071067811865475, 0.007372999718619262},
+     {0.5773502691896258, 0.5773502691896258, 0.5773502691896258, 0.007210515360146086},
+     {0.15746766720392918, 0.15746766720392918, 0.9748886436771664, 0.007574394159056108},
+     {0.41749612279649856, 0.41749612279649856, 0.8070898183596309, 0.006753829486315507},
+     {0.291298882209546, 0.6764410400114222, 0.6764410400114222, 0.007116355493118483},
+     {0.14035538117128105, 0.4493328323269971, 0.8822700112603075, 0.0069910873533014575}},
+    // order 10: 170 points (degree 21)
+    {{0.0, 0.0, 1.0, 0.005544842902030009},
+     {0.0, 0.7071067811865475, 0.7071067811865475, 0.00607133277067263},
+     {0.5773502691896258, 0.5773502691896258, 0.5773502691896258, 0.0063836747735153895},
+     {0.25512526211144787, 0.25512526211144787, 0.9326425903126717, 0.00518338758774642},
+     {0.30079359513765364, 0.6743601460362872, 0.6743601460362872, 0.006317929009815409},
+     {0.43189106967195323, 0.43189106967195323, 0.7917955593934788, 0.00620167000658926},
+     {0.0, 0.2613931360334841, 0.9652324219764794, 0.005477143385138053},
+     {0.1446630744324903, 0.49904531617954023, 0.8544158046846995, 0.005968383987680958}},
+};
+
+static std::unique_ptr<ShTables> build_level_tables(int q) {
+    auto t = std::make_unique<ShTables>();
+    t->p = q;
+    t->Q = tri_size(q);
+    for (const Orbit &o : kRules[q - 1]) {
+        double c[3] = {o.x, o.y, o.z};
+        do {
+            for (int s = 0; s < 8; s++) {
+                bool twice = false;
+                for (int k = 0; k < 3; k++) twice = twice || ((s >> k & 1) && c[k] == 0.0);
+                if (twice) continue;
+                for (int k = 0; k < 3; k++) t->eta.push_back(s >> k & 1 ? -c[k] : c[k]);
+                t->w.push_back(4.0 * kPi * o.w);
+            }
+        } while (std::next_permutation(c, c + 3));
+    }
+    t->npts = (int)t->w.size();
+    fill_matrices(t.get(), q);
+    return t;
+}
+
+const ShTables &level_tables(int q) {
+    if (q < 1 || q > (int)(sizeof kRules / sizeof kRules[0])) return sh_tables(q);
+    static std::mutex mu;
+    static std::map<int, std::unique_ptr<ShTables>> cache;
+    std::lock_guard<std::mutex> lock(mu);
+    auto &t = cache[q];
+    if (!t) t = build_level_tables(q);
+    return *t;
+}
+
+static void fill_matrices(ShTables *t, int p) {
     const int Q = t->Q, rows = 6 * Q, cols = 3 * t->npts;
     t->anal.assign(size_t(rows) * cols, 0.0);
     std::vector<double> invN(Q);
@@ -231,7 +339,6 @@ static std::unique_ptr<ShTables> build_tables(int p) {
                 }
             }
     }
-    return t;
 }
 
 // rows of a coefficient vector (6Q layout) that belong to degrees <= pc
@@ -247,16 +354,16 @@ static std::vector<int> coef_rows_upto(int p, int pc) {
     return r;
 }
 
-static std::unique_ptr<Resample> build_resample(int p, int pc) {
+static std::unique_ptr<Resample> build_resample(int p, int pc, const ShTables &C, bool same) {
     auto rs = std::make_unique<Resample>();
     rs->p = p;
     rs->pc = pc;
-    const ShTables &F = sh_tables(p), &C = sh_tables(rs->pc);
+    const ShTables &F = sh_tables(p);
     rs->n = F.npts;
     rs->nc = C.npts;
     const int QF = F.Q, QC = C.Q;
     const int rowsF = 6 * QF, rowsC = 6 * QC;
-    if (rs->pc == p) { // same grid: identity in both directions
+    if (same) { // same grid: identity in both directions
         const int nn = 3 * F.npts;
         rs->down.assign(size_t(nn) * nn, 0.0);
         for (int i = 0; i < nn; i++) rs->down[size_t(i) * nn + i] = 1.0;
@@ -294,10 +401,19 @@ const Resample &resample_tables(int p, int pc) {
     std::lock_guard<std::mutex> lock(mu);
     auto it = cache.find({p, pc});
     if (it != cache.end()) return *it->second;
-    auto t = build_resample(p, pc);
+    auto t = build_resample(p, pc, sh_tables(pc), pc == p);
     const Resample &ref = *t;
     cache[{p, pc}] = std::move(t);
     return ref;
+}
+
+const Resample &level_resample(int p, int pc) {
+    static std::mutex mu;
+    static std::map<std::pair<int, int>, std::unique_ptr<Resample>> cache;
+    std::lock_guard<std::mutex> lock(mu);
+    auto &t = cache[{p, pc}];
+    if (!t) t = build_resample(p, pc, level_tables(pc), false);
+    return *t;
 }
 
 const ShTables &sh_tables(int p) {
