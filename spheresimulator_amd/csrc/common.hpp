@@ -52,7 +52,7 @@ struct FarGroup {
     int32_t tcount;
     int32_t susp;
     int32_t slot;
-    int32_t pad;
+    int32_t list; // of a joint list: which of its lists
 };
 
 // Number of complex arrays in the per-sphere expansion records.

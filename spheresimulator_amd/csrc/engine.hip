@@ -425,7 +425,6 @@ Operator::Operator(int nsusp, const int *counts, const double *pos, const double
             srcm_.alloc(std::max<int64_t>(4 * (std::min(ncopy_, kMultiCols) + 1) * pt_off_[s0], 8));
         } else {
             build_far_lists(lists_fine_, nsusp_, susp_sph_off_, pt_off_, pt_off_, runs_fine_, tpl, split, kWantItems);
-            lists_fine_.slots();
         }
     }
     ls32_.tpl = ls64_.tpl = lsc_.tpl = tpl;
@@ -471,7 +470,6 @@ void Operator::autotune_fine(double &budget_s) {
     launch_fill(3 * npts_, 1.0, tmp_.p, stream_);
     launch_pack_src_f64(npts_, d_coords_.p, d_w_.p, tmp_.p, src64_.p, stream_);
     auto timed = [&](FarLists &L) {
-        L.slots();
         const double ms = time_far_pass(L, 0, src64_.p, d_coords_.p, d_norms_.p, nullptr);
         budget_s -= 2e-3 * ms;
         return ms;
@@ -507,9 +505,9 @@ void Operator::autotune_fine(double &budget_s) {
 void Operator::autotune_inner(double &budget_s) {
     if (nsph_ == 0 || !multi_level_) return;
     launch_fill(3 * npts_, 1.0, tmp_.p, stream_);
-    pack(tmp_.p, 1);
     auto timed = [&]() {
         auto t0 = std::chrono::steady_clock::now();
+        pack(tmp_.p, 1, &ls32_);
         far_levels(ls32_, 0, 1.0, nullptr, nullptr, nullptr);
         hipEvent_t a, b;
         SPHSTK_HIP(hipEventCreate(&a));
@@ -633,19 +631,13 @@ static void parallel_for(int n, const std::function<void(int, int)> &body, int c
 // FMM, cpp:332-348, :408-433, :641-690).  A group's source intervals are the
 // point ranges of its spheres' runs, with a per-lane mask where the group
 // spans spheres.  Each group's list is cut into `split` slices of nearly equal
-// length, one work item each, launched in order of decreasing work.  With
-// `sph_pos` (sphere centres) the groups are aligned to spheres instead (at most
-// 64 points of one sphere each, so every interval applies to all lanes) and
-// each group records its sphere's centre.
-void build_far_lists(FarLists &L, int nsusp, const std::vector<int64_t> &susp_sph_off,
-                     const std::vector<int64_t> &toff, const std::vector<int64_t> &soff, const std::vector<Runs> &runs,
-                     int tpl, int split, int64_t want_items, const double *sph_pos,
-                     const std::vector<int64_t> *src_susp_off) {
+// length, one work item each, launched in order of decreasing work.
+int append_far_lists(HostLists &H, int nsusp, const std::vector<int64_t> &susp_sph_off, const std::vector<int64_t> &toff,
+                     const std::vector<int64_t> &soff, const std::vector<Runs> &runs, int tpl, int split,
+                     int64_t want_items, const std::vector<int64_t> *src_susp_off, ListBase at) {
     const std::vector<int64_t> &sso = src_susp_off ? *src_susp_off : susp_sph_off;
     SPHSTK_REQUIRE(tpl == 1 || tpl == 2 || tpl == 4, "targets per lane must be 1, 2 or 4");
     SPHSTK_REQUIRE(split >= 0 && split <= 64, "source split must be in [0, 64] (0 = automatic)");
-    const bool aligned = sph_pos != nullptr;
-    SPHSTK_REQUIRE(!aligned || tpl == 1, "sphere-aligned far-field lists use one target per lane");
     const int nsph = (int)toff.size() - 1;
     SPHSTK_REQUIRE((int)runs.size() == nsph, "internal: one run list per target sphere");
     const int64_t ntrg = toff[nsph];
@@ -655,20 +647,13 @@ void build_far_lists(FarLists &L, int nsusp, const std::vector<int64_t> &susp_sp
     const int G = 64 * tpl;
     int64_t nbase = 0;
     for (int b = 0; b < nsusp; b++) {
-        if (aligned) {
-            for (int64_t T = susp_sph_off[b]; T < susp_sph_off[b + 1]; T++) nbase += (toff[T + 1] - toff[T] + G - 1) / G;
-        } else {
-            const int64_t np = toff[susp_sph_off[b + 1]] - toff[susp_sph_off[b]];
-            nbase += (np + G - 1) / G;
-        }
+        const int64_t np = toff[susp_sph_off[b + 1]] - toff[susp_sph_off[b]];
+        nbase += (np + G - 1) / G;
     }
     if (split == 0) {
         const int64_t nb = std::max<int64_t>(nbase, 1);
         split = (int)std::max<int64_t>(1, std::min<int64_t>(8, (want_items + nb - 1) / nb));
     }
-    L.tpl = tpl;
-    L.split = split;
-    L.ntrg = ntrg;
     // the groups (first target, count, suspension), then their interval lists
     // built in parallel over chunks of consecutive groups and concatenated
     struct GSpec {
@@ -679,8 +664,7 @@ void build_far_lists(FarLists &L, int nsusp, const std::vector<int64_t> &susp_sp
     for (int b = 0; b < nsusp; b++) {
         const int64_t p0 = toff[susp_sph_off[b]], p1 = toff[susp_sph_off[b + 1]];
         for (int64_t t0 = p0; t0 < p1;) {
-            const int64_t tend = aligned ? toff[tsph[t0] + 1] : p1;
-            const int cnt = (int)std::min<int64_t>(G, tend - t0);
+            const int cnt = (int)std::min<int64_t>(G, p1 - t0);
             gs.push_back(GSpec{t0, cnt, b});
             t0 += cnt;
         }
@@ -689,8 +673,8 @@ void build_far_lists(FarLists &L, int nsusp, const std::vector<int64_t> &susp_sp
         std::vector<FarGroup> groups;
         std::vector<FarInterval> ivs;
         std::vector<int64_t> work;
-        std::vector<double> cen;
         double pairs = 0.0;
+        bool bad = false;
     };
     const int nparts = (int)std::min<size_t>(64, std::max<size_t>(1, gs.size() / 512));
     std::vector<Part> parts(nparts);
@@ -711,12 +695,9 @@ void build_far_lists(FarLists &L, int nsusp, const std::vector<int64_t> &susp_sp
             const int cnt = gs[gi].cnt, b = gs[gi].b;
             if (tsph[t0] == tsph[t0 + cnt - 1] && tsph[t0] == last_T) {
                 for (int sl = 0; sl < split; sl++) {
-                    P.groups.push_back(FarGroup{t0, last_slots[sl][0], last_slots[sl][1], cnt, b, sl, 0});
+                    P.groups.push_back(FarGroup{t0 + at.trg, last_slots[sl][0], last_slots[sl][1], cnt, b, at.slot + sl,
+                                                H.nlist});
                     P.work.push_back(last_slots[sl][2]);
-                    if (aligned) {
-                        for (int c = 0; c < 3; c++) P.cen.push_back(sph_pos[3 * last_T + c]);
-                        P.cen.push_back(0.0);
-                    }
                 }
                 P.pairs += double(last_work) * cnt;
                 continue;
@@ -788,13 +769,14 @@ void build_far_lists(FarLists &L, int nsusp, const std::vector<int64_t> &susp_sp
             int64_t iv_pos = giv.empty() ? 0 : giv[0].begin;
             for (int sl = 0; sl < split; sl++) {
                 const int64_t quota = gwork * (sl + 1) / split - gwork * sl / split;
-                FarGroup g{t0, (int64_t)P.ivs.size(), 0, cnt, b, sl, 0};
+                FarGroup g{t0 + at.trg, (int64_t)P.ivs.size(), 0, cnt, b, at.slot + sl, H.nlist};
                 int64_t left = quota;
                 while (left > 0 && iv_i < giv.size()) {
                     const int64_t take = std::min(giv[iv_i].end - iv_pos, left);
                     FarInterval piece = giv[iv_i];
-                    piece.begin = iv_pos;
-                    piece.end = iv_pos + take;
+                    piece.begin = iv_pos + at.src;
+                    piece.end = iv_pos + take + at.src;
+                    P.bad = P.bad || iv_pos < soff[sso[b]] || iv_pos + take > soff[sso[b + 1]] || take <= 0;
                     P.ivs.push_back(piece);
                     left -= take;
                     iv_pos += take;
@@ -807,10 +789,6 @@ void build_far_lists(FarLists &L, int nsusp, const std::vector<int64_t> &susp_sp
                 P.groups.push_back(g);
                 P.work.push_back(quota);
                 last_slots[sl] = {g.iv_begin, g.iv_end, quota};
-                if (aligned) {
-                    for (int c = 0; c < 3; c++) P.cen.push_back(sph_pos[3 * Ta + c]);
-                    P.cen.push_back(0.0);
-                }
             }
         }
     };
@@ -820,63 +798,63 @@ void build_far_lists(FarLists &L, int nsusp, const std::vector<int64_t> &susp_sp
             for (int pi = a; pi < e; pi++) build_part(pi);
         },
         1, 2);
-    std::vector<FarGroup> groups;
-    std::vector<FarInterval> ivs;
-    std::vector<int64_t> work;
-    std::vector<double> cen;
     double pairs = 0.0;
-    {
-        size_t ng = 0, ni = 0;
-        for (const Part &P : parts) {
-            ng += P.groups.size();
-            ni += P.ivs.size();
-        }
-        groups.reserve(ng);
-        ivs.reserve(ni);
-        work.reserve(ng);
-        for (Part &P : parts) {
-            const int64_t base = (int64_t)ivs.size();
-            for (FarGroup g : P.groups) {
-                g.iv_begin += base;
-                g.iv_end += base;
-                groups.push_back(g);
-            }
-            ivs.insert(ivs.end(), P.ivs.begin(), P.ivs.end());
-            work.insert(work.end(), P.work.begin(), P.work.end());
-            cen.insert(cen.end(), P.cen.begin(), P.cen.end());
-            pairs += P.pairs;
-            Part().groups.swap(P.groups);
-            std::vector<FarInterval>().swap(P.ivs);
-        }
+    size_t ng = 0, ni = 0;
+    for (const Part &P : parts) {
+        SPHSTK_REQUIRE(!P.bad, "internal: far-field interval out of range");
+        pairs += P.pairs;
+        ng += P.groups.size();
+        ni += P.ivs.size();
     }
-    for (const FarGroup &g : groups) {
-        const int b = g.susp;
-        const int64_t tlo = toff[susp_sph_off[b]], thi = toff[susp_sph_off[b + 1]];
-        const int64_t slo = soff[sso[b]], shi = soff[sso[b + 1]];
-        SPHSTK_REQUIRE(g.tstart >= tlo && g.tstart + g.tcount <= thi && g.tcount > 0 && g.tcount <= G &&
-                           g.slot >= 0 && g.slot < split,
-                       "internal: far-field group out of range");
-        for (int64_t k = g.iv_begin; k < g.iv_end; k++) {
-            SPHSTK_REQUIRE(ivs[k].begin >= slo && ivs[k].end <= shi && ivs[k].begin < ivs[k].end,
-                           "internal: far-field interval out of range");
-            SPHSTK_REQUIRE(!aligned || ivs[k].mask[0] == ~0ull, "internal: masked interval in an aligned list");
+    if (setup_verbose()) std::fprintf(stderr, "[sphstk]     %zu work items, %zu intervals, %.4g pairs\n", ng, ni, pairs);
+    if (pairs == 0.0) return 0;
+    H.pairs += pairs;
+    for (Part &P : parts) {
+        const int64_t base = (int64_t)H.ivs.size();
+        for (FarGroup &g : P.groups) {
+            g.iv_begin += base;
+            g.iv_end += base;
         }
-        SPHSTK_REQUIRE(!aligned || tsph[g.tstart] == tsph[g.tstart + g.tcount - 1],
-                       "internal: aligned far-field group spans spheres");
+        H.groups.insert(H.groups.end(), P.groups.begin(), P.groups.end());
+        H.ivs.insert(H.ivs.end(), P.ivs.begin(), P.ivs.end());
+        H.work.insert(H.work.end(), P.work.begin(), P.work.end());
+        std::vector<FarInterval>().swap(P.ivs);
     }
-    std::vector<int> ord(groups.size());
+    H.nlist++;
+    return split;
+}
+
+// Launch order: by work, in classes of a factor of two, so that no long item
+// starts last; within a class list by list and slice by slice, in the order of
+// the targets, so that the items in flight read one part of one list's sources
+// (measured against the strict order by work: within 1%).
+void upload_far_lists(FarLists &L, HostLists &H, int tpl, int split, int64_t ntrg) {
+    std::vector<int> ord(H.groups.size());
+    std::vector<uint64_t> key(H.groups.size());
     std::iota(ord.begin(), ord.end(), 0);
-    std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return work[a] > work[b]; });
-    L.ngroups = (int)groups.size();
-    L.pairs = pairs;
-    if (setup_verbose())
-        std::fprintf(stderr, "[sphstk]     %d work items, %zu intervals, %.4g pairs\n", L.ngroups, ivs.size(), pairs);
-    L.groups.upload(groups);
-    L.iv.upload(ivs);
+    for (size_t i = 0; i < ord.size(); i++) {
+        int cls = 0;
+        while (cls < 63 && (H.work[i] >> cls) != 0) cls++;
+        key[i] = uint64_t(63 - cls) << 32 | uint64_t(H.groups[i].list) << 16 | uint64_t(H.groups[i].slot);
+    }
+    std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return key[a] < key[b]; });
+    L.tpl = tpl;
+    L.split = split;
+    L.ntrg = ntrg;
+    L.ngroups = (int)H.groups.size();
+    L.pairs = H.pairs;
+    L.groups.upload(H.groups);
+    L.iv.upload(H.ivs);
     L.order.upload(ord);
-    L.aligned = aligned;
-    if (aligned) L.cen.upload(cen);
-    if (split > 1) L.part.alloc(size_t(split) * 3 * std::max<int64_t>(ntrg, 1));
+    L.slots();
+}
+
+void build_far_lists(FarLists &L, int nsusp, const std::vector<int64_t> &susp_sph_off,
+                     const std::vector<int64_t> &toff, const std::vector<int64_t> &soff, const std::vector<Runs> &runs,
+                     int tpl, int split, int64_t want_items, const std::vector<int64_t> *src_susp_off) {
+    HostLists H;
+    const int n = append_far_lists(H, nsusp, susp_sph_off, toff, soff, runs, tpl, split, want_items, src_susp_off);
+    upload_far_lists(L, H, tpl, std::max(n, 1), toff.back());
 }
 
 static std::vector<Chunk> make_chunks(int nsusp, const std::vector<int64_t> &susp_sph_off,
@@ -942,6 +920,11 @@ void kd_order(const double *pos, int *idx, int b, int e, int leaf) {
     kd_order(pos, idx, b + h, e, leaf);
 }
 } // namespace
+
+template <typename T>
+static void put(DevBuf<T> &d, int64_t at, const std::vector<T> &v) {
+    if (!v.empty()) SPHSTK_HIP(hipMemcpy(d.p + at, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
+}
 
 void Operator::ensure_levels(LevelSet &S) {
     if (S.ready) return;
@@ -1115,13 +1098,12 @@ void Operator::ensure_levels(LevelSet &S) {
         }
     }
     tn.reset();
-    {
-        PhaseTimer pm("  mid-range lists");
-        build_far_lists(S.mid, nsusp_, susp_sph_off_, pt_off_, pt_off_, mid, S.tpl, 0, kWantItems);
-        S.mid.slots();
-    }
+    // point sets, one after the other: fine grid, levels, equivalent points
     S.levels.clear();
     std::vector<std::vector<int64_t>> level_off(nlev);
+    std::vector<int64_t> lbase(nlev + 1);
+    lbase[0] = npts_;
+    std::vector<double> lc, ln, lw; // level points of all levels
     for (int l = 0; l < nlev; l++) {
         auto L = std::make_unique<FarLevel>();
         std::vector<int64_t> &off = level_off[l];
@@ -1132,39 +1114,37 @@ void Operator::ensure_levels(LevelSet &S) {
             off[r + 1] = off[r] + lpoints(l, order_[s]);
             off_by_sph[s] = off[r];
         }
-        const int64_t nc = off[nsph_];
-        std::vector<double> cc(3 * nc), cn(3 * nc), cw(nc);
+        const int64_t nc = off[nsph_], at = lbase[l] - npts_;
+        lbase[l + 1] = lbase[l] + nc;
+        lc.resize(3 * (at + nc));
+        ln.resize(3 * (at + nc));
+        lw.resize(at + nc);
         for (int s = 0; s < nsph_; s++) {
             const ShTables &t = level_grid(S, l, order_[s]);
             for (int q = 0; q < t.npts; q++) {
-                const int64_t g = off_by_sph[s] + q;
+                const int64_t g = at + off_by_sph[s] + q;
                 double nv[3];
                 qrot_host(&quat_[4 * s], &t.eta[3 * q], nv);
                 for (int c = 0; c < 3; c++) {
-                    cn[3 * g + c] = nv[c];
-                    cc[3 * g + c] = pos_[3 * s + c] + rad_[s] * nv[c];
+                    ln[3 * g + c] = nv[c];
+                    lc[3 * g + c] = pos_[3 * s + c] + rad_[s] * nv[c];
                 }
-                cw[g] = rad_[s] * rad_[s] * t.w[q];
+                lw[g] = rad_[s] * rad_[s] * t.w[q];
             }
         }
-        L->npts = nc;
         L->d_off_by_sph.upload(off_by_sph);
-        L->coords.upload(cc);
-        L->norms.upload(cn);
-        L->w.upload(cw);
-        PhaseTimer pl("  level lists");
-        build_far_lists(L->lists, nsusp_, susp_sph_off_, off, off, lvl[l], S.tpl, 0, kWantItems);
-        L->lists.slots();
-        if (S.fp64) {
-            L->src64.alloc(std::max<int64_t>(8 * nc, 8));
-            launch_pack_src_f64(nc, L->coords.p, L->w.p, nullptr, L->src64.p, stream_);
-        } else {
-            L->src32.alloc(std::max<int64_t>(8 * nc, 8));
-            L->trg32.alloc(std::max<int64_t>(8 * nc, 8));
-            launch_pack_src_f32(nc, L->coords.p, L->w.p, nullptr, L->src32.p, stream_);
-            launch_pack_trg_f32(nc, L->coords.p, L->norms.p, L->trg32.p, stream_);
-        }
+        L->w.upload(std::vector<double>(lw.begin() + at, lw.end()));
         S.levels.push_back(std::move(L));
+    }
+    const int64_t ntrg = lbase[nlev];
+    HostLists H;
+    std::vector<int> nslot(nlev);
+    {
+        PhaseTimer pm("  mid-range and level lists");
+        S.mid_slots = append_far_lists(H, nsusp_, susp_sph_off_, pt_off_, pt_off_, mid, S.tpl, 0, kWantItems);
+        for (int l = 0; l < nlev; l++)
+            nslot[l] = append_far_lists(H, nsusp_, susp_sph_off_, level_off[l], level_off[l], lvl[l], S.tpl, 0,
+                                        kWantItems, nullptr, ListBase{lbase[l], lbase[l], 0});
     }
     level_transforms(S);
     S.agg.reset();
@@ -1205,6 +1185,7 @@ void Operator::ensure_levels(LevelSet &S) {
         crho.swap(cr);
         susp_cell_off.swap(sco);
     }
+    std::vector<float> eq; // source records of the equivalent points
     if (S.cells && nused > 0) {
         const int ncell = nused;
         PhaseTimer pc("  cells");
@@ -1214,7 +1195,8 @@ void Operator::ensure_levels(LevelSet &S) {
         A->ncell = ncell;
         A->E = &E;
         A->susp_cell_off = susp_cell_off;
-        std::vector<float> chk(8 * (size_t)ncell * Kc, 0.f), eq(8 * (size_t)ncell * K, 0.f);
+        std::vector<float> chk(8 * (size_t)ncell * Kc, 0.f);
+        eq.assign(8 * (size_t)ncell * K, 0.f);
         std::vector<int> csusp(ncell);
         for (int c = 0; c < ncell; c++) {
             for (int i = 0; i < Kc; i++)
@@ -1229,7 +1211,6 @@ void Operator::ensure_levels(LevelSet &S) {
         for (int i = 0; i < n; i++)
             for (int j = 0; j < m; j++) Pcm[(size_t)j * n + i] = E.P[(size_t)i * m + j];
         A->chk32.upload(chk);
-        A->eq32.upload(eq);
         A->P.upload(Pcm);
         A->rho.upload(crho);
         A->susp.upload(csusp);
@@ -1245,32 +1226,66 @@ void Operator::ensure_levels(LevelSet &S) {
             std::sort(mem.begin(), mem.end());
             for (int sm : mem) run_append(chk_runs[c], sm);
         }
-        build_far_lists(A->chk_lists, nsusp_, susp_cell_off, chk_off, pt_off_, chk_runs, 1, 0, kWantItems, nullptr,
+        build_far_lists(A->chk_lists, nsusp_, susp_cell_off, chk_off, pt_off_, chk_runs, 1, 0, kWantItems,
                         &susp_sph_off_);
-        A->chk_lists.slots();
         A->check_pairs = A->chk_lists.pairs;
         for (int i = 0; i < 2; i++) {
             std::vector<Runs> runs(nsph_);
             for (int r = 0; r < nsph_; r++) runs[r] = crun[r][i];
-            build_far_lists(A->lists[i], nsusp_, susp_sph_off_, level_off[c0 + i], eq_off, runs, S.tpl, 0, kWantItems,
-                            nullptr, &susp_cell_off);
-            A->lists[i].slots();
-            A->pairs += A->lists[i].pairs;
+            const int l = c0 + i;
+            nslot[l] += append_far_lists(H, nsusp_, susp_sph_off_, level_off[l], eq_off, runs, S.tpl, 0, kWantItems,
+                                         &susp_cell_off, ListBase{lbase[l], ntrg, nslot[l]});
         }
         S.agg = std::move(A);
     }
+    upload_far_lists(S.all, H, S.tpl, std::max(S.mid_slots, nslot.empty() ? 0 : *std::max_element(nslot.begin(), nslot.end())),
+                     ntrg);
+    // records: positions now, force words per apply
+    // (set-up of a set may run on a host thread of its own: nothing here goes to
+    // the operator's stream, which may be capturing)
+    const int64_t nlp = ntrg - npts_, neq = (int64_t)eq.size() / 8;
+    const hipStream_t st0 = nullptr;
+    auto fine = [&](DevBuf<double> &d, const DevBuf<double> &from) {
+        if (npts_) SPHSTK_HIP(hipMemcpyAsync(d.p, from.p, sizeof(double) * 3 * npts_, hipMemcpyDeviceToDevice, st0));
+    };
+    if (S.fp64) {
+        std::vector<double> rec(8 * (size_t)nlp, 0.0);
+        for (int64_t i = 0; i < nlp; i++) std::copy(&lc[3 * i], &lc[3 * i] + 3, &rec[8 * i]);
+        S.src64.alloc(std::max<int64_t>(8 * ntrg, 8));
+        S.coords.alloc(std::max<int64_t>(3 * ntrg, 3));
+        S.norms.alloc(std::max<int64_t>(3 * ntrg, 3));
+        launch_pack_src_f64(npts_, d_coords_.p, d_w_.p, nullptr, S.src64.p, st0);
+        put(S.src64, 8 * npts_, rec);
+        fine(S.coords, d_coords_);
+        put(S.coords, 3 * npts_, lc);
+        fine(S.norms, d_norms_);
+        put(S.norms, 3 * npts_, ln);
+    } else {
+        std::vector<float> rec(8 * (size_t)(nlp + neq), 0.f), trg(8 * (size_t)nlp, 0.f);
+        for (int64_t i = 0; i < nlp; i++)
+            for (int c = 0; c < 3; c++) {
+                rec[8 * i + c] = trg[8 * i + c] = (float)lc[3 * i + c];
+                trg[8 * i + 3 + c] = (float)ln[3 * i + c];
+            }
+        std::copy(eq.begin(), eq.end(), rec.begin() + 8 * nlp);
+        S.src32.alloc(std::max<int64_t>(8 * (ntrg + neq), 8));
+        S.trg32.alloc(8 * std::max<int64_t>(ntrg, 1));
+        launch_pack_src_f32(npts_, d_coords_.p, d_w_.p, nullptr, S.src32.p, st0);
+        launch_pack_trg_f32(npts_, d_coords_.p, d_norms_.p, S.trg32.p, st0);
+        put(S.src32, 8 * npts_, rec);
+        put(S.trg32, 8 * npts_, trg);
+        if (S.agg) S.agg->eq32 = S.src32.p + 8 * ntrg;
+    }
+    SPHSTK_HIP(hipGetLastError());
+    SPHSTK_HIP(hipStreamSynchronize(st0));
+    LevelViews &V = S.views;
+    V.stride = 3 * ntrg;
     for (int l = 0; l < nlev; l++) {
-        FarLevel &L = *S.levels[l];
-        LevelViews &V = S.views;
-        V.off[l] = L.d_off_by_sph.p;
-        V.w[l] = L.w.p;
-        V.src[l] = S.fp64 ? (void *)L.src64.p : (void *)L.src32.p;
-        V.stride[l] = 3 * L.npts;
-        V.part[l][0] = L.lists.part.p;
-        V.nslot[l][0] = L.lists.nslot();
-        const FarLists *C = S.agg && l >= c0 ? &S.agg->lists[l - c0] : nullptr;
-        V.part[l][1] = C ? C->part.p : nullptr;
-        V.nslot[l][1] = C ? C->nslot() : 0;
+        V.off[l] = S.levels[l]->d_off_by_sph.p;
+        V.w[l] = S.levels[l]->w.p;
+        V.src[l] = S.fp64 ? (void *)(S.src64.p + 8 * lbase[l]) : (void *)(S.src32.p + 8 * lbase[l]);
+        V.part[l] = S.all.part.p ? S.all.part.p + 3 * lbase[l] : nullptr;
+        V.nslot[l] = nslot[l];
     }
     S.ready = true;
 }
@@ -1398,9 +1413,9 @@ void Operator::far_slots(FarLists &L, int kind, int prec, const void *src, const
 }
 
 // Multi-level far field of the densities that pack() left in body64_ or body32_
-// and src64_ or src32_: the sources are resampled to all levels, each list sums
-// its shell of sphere pairs into its slots; the pairs closer than the first
-// level are summed on the fine grid.  levels_up interpolates the level fields
+// and the set's fine-grid sources: the sources are resampled to all levels, then
+// one launch sums each shell of sphere pairs into its slots, the pairs closer
+// than the first level on the fine grid.  levels_up interpolates the level fields
 // back.  ev_a and ev_b bracket the pair sums only.
 void Operator::far_levels(LevelSet &S, int kind, double coef, const int *active, hipEvent_t ev_a, hipEvent_t ev_b) {
     ensure_levels(S);
@@ -1410,24 +1425,13 @@ void Operator::far_levels(LevelSet &S, int kind, double coef, const int *active,
     if (A) {
         // check velocities of each cell's raw fine-grid sources (single layer,
         // FP32 pairs, FP64 sums), then the equivalent point forces
-        far_slots(A->chk_lists, 1, 1, src32_.p, nullptr, nullptr, A->chk32.p, 1.0 / (8.0 * kPi), active);
+        far_slots(A->chk_lists, 1, 1, S.src32.p, nullptr, nullptr, A->chk32.p, 1.0 / (8.0 * kPi), active);
         launch_equiv_forces(A->ncell, A->E->K, A->E->Kc, A->P.p, A->chk_lists.part.p, A->chk_lists.nslot(),
-                            3 * A->chk_lists.ntrg, A->rho.p, A->susp.p, active, A->eq32.p, stream_);
+                            3 * A->chk_lists.ntrg, A->rho.p, A->susp.p, active, A->eq32, stream_);
     }
     if (ev_a) SPHSTK_HIP(hipEventRecord(ev_a, stream_));
-    if (A)
-        for (int i = 0; i < 2; i++)
-            far_slots(A->lists[i], kind, 1, A->eq32.p, nullptr, nullptr, S.levels[S.nlev - 2 + i]->trg32.p, coef, active);
-    for (auto &L : S.levels) {
-        if (S.fp64)
-            far_slots(L->lists, kind, 0, L->src64.p, L->coords.p, L->norms.p, nullptr, coef, active);
-        else
-            far_slots(L->lists, kind, 1, L->src32.p, nullptr, nullptr, L->trg32.p, coef, active);
-    }
-    if (S.fp64)
-        far_slots(S.mid, kind, 0, src64_.p, d_coords_.p, d_norms_.p, nullptr, coef, active);
-    else
-        far_slots(S.mid, kind, 1, src32_.p, nullptr, nullptr, trg32_.p, coef, active);
+    far_slots(S.all, kind, S.fp64 ? 0 : 1, S.fp64 ? (const void *)S.src64.p : (const void *)S.src32.p, S.coords.p,
+              S.norms.p, S.trg32.p, coef, active);
     if (ev_b) SPHSTK_HIP(hipEventRecord(ev_b, stream_));
     launch_pack_levels(geom_, S.fp64, S.views, S.fp64 ? (void *)S.body64.p : (void *)S.body32.p, S.max_lev_pts, stream_);
 }
@@ -1480,9 +1484,7 @@ bool Operator::outer_levels_pay() {
     wait_outer_levels();
     if (outer_pay_ < 0) {
         ensure_levels(ls64_);
-        double ml = ls64_.mid.pairs;
-        for (auto &L : ls64_.levels) ml += L->lists.pairs;
-        outer_pay_ = ml <= 0.75 * lists_fine_.pairs ? 1 : 0;
+        outer_pay_ = ls64_.all.pairs <= 0.75 * lists_fine_.pairs ? 1 : 0;
     }
     return outer_pay_ == 1;
 }
@@ -1491,23 +1493,46 @@ void Operator::ensure_fp32_grid() {
     if (trg32_.p) return;
     trg32_.alloc(8 * std::max<int64_t>(npts_, 1));
     src32_.alloc(8 * std::max<int64_t>(npts_, 1));
-    body32_.alloc(body64_.n);
     launch_pack_trg_f32(npts_, d_coords_.p, d_norms_.p, trg32_.p, stream_);
     launch_pack_src_f32(npts_, d_coords_.p, d_w_.p, nullptr, src32_.p, stream_);
 }
 
-void Operator::pack(const double *in, int prec) {
+LevelSet *Operator::set_of(int prec) {
+    if (nsph_ == 0 || ncopy_ > 1) return nullptr;
+    LevelSet *S = nullptr;
+    if (prec == 2) {
+        S = outer_levels_pay() ? &ls64_ : nullptr; // else too few pair evaluations saved: direct FP64 sum
+    } else if (prec != 0 && multi_level_) {
+        if (prec == 1) wait_inner_levels();
+        S = prec == 3 ? &lsc_ : &ls32_;
+        ensure_levels(*S);
+    }
+    return S;
+}
+
+void Operator::pack(const double *in, int prec, const LevelSet *S) {
     const bool f32 = prec == 1 || prec == 3;
-    if (f32) ensure_fp32_grid();
-    launch_pack_body(geom_, in, body64_.p, f32 && multi_level_ ? body32_.p : nullptr,
-                     (prec == 0 || prec == 2) && ncopy_ == 1 ? src64_.p : nullptr, f32 ? src32_.p : nullptr, max_pts_,
-                     stream_);
+    double *s64 = nullptr;
+    float *s32 = nullptr, *b32 = nullptr;
+    if (S && f32) {
+        body32_.alloc(body64_.n);
+        b32 = body32_.p;
+        s32 = S->src32.p;
+    } else if (S) {
+        s64 = S->src64.p;
+    } else if (f32) {
+        ensure_fp32_grid();
+        s32 = src32_.p;
+    } else if (prec >= 0 && ncopy_ == 1) {
+        s64 = src64_.p;
+    }
+    launch_pack_body(geom_, in, body64_.p, b32, s64, s32, max_pts_, stream_);
 }
 
 // FP64: fine grid, direct sum over all far pairs.  FP32: multi-level (fine for
 // mid-range pairs, coarser grids with distance) unless disabled, in which case
 // the FP32 direct sum.
-FarSum Operator::far(int kind, int prec, double coef, const double *in, const int *active, LevelSet **levels) {
+FarSum Operator::far(LevelSet *S, int kind, int prec, double coef, const double *in, const int *active) {
     const bool timing = (flags_ & 1) != 0 && !capturing_;
     EvPair ev{};
     if (timing) {
@@ -1521,17 +1546,8 @@ FarSum Operator::far(int kind, int prec, double coef, const double *in, const in
         ev.kind = kind;
         ev.prec = prec;
     }
-    LevelSet *S = nullptr;
-    if (ncopy_ > 1)
-        SPHSTK_REQUIRE(prec == 0, "several right-hand sides on one geometry are solved in FP64 only");
-    else if (prec == 2)
-        S = outer_levels_pay() ? &ls64_ : nullptr; // else too few pair evaluations saved: direct FP64 sum
-    else if (prec != 0 && multi_level_) {
-        if (prec == 1) wait_inner_levels();
-        S = prec == 3 ? &lsc_ : &ls32_;
-    }
-    *levels = S;
-    FarLists &L = S ? S->mid : lists_fine_;
+    SPHSTK_REQUIRE(ncopy_ == 1 || prec == 0, "several right-hand sides on one geometry are solved in FP64 only");
+    FarLists &L = lists_fine_;
     if (S) {
         far_levels(*S, kind, coef, active, timing ? ev.a : nullptr, timing ? ev.b : nullptr);
     } else if (ncopy_ > 1) {
@@ -1549,7 +1565,7 @@ FarSum Operator::far(int kind, int prec, double coef, const double *in, const in
         pending_.push_back(ev);
         if (pending_.size() > 64) harvest_events();
     }
-    return FarSum{L.part.p, L.nslot(), 3 * npts_};
+    return S ? FarSum{S->all.part.p, S->mid_slots, 3 * S->all.ntrg} : FarSum{L.part.p, L.nslot(), 3 * npts_};
 }
 
 // applyP2POP (cpp:262-485), accumulating into out (or, overwrite, the whole
@@ -1569,7 +1585,8 @@ void Operator::p2p(const double *in, double *out, double cId, double cSL, double
         return;
     }
     const hipStream_t side = capturing_ ? stream_ : aux_;
-    pack(in, prec);
+    LevelSet *S = set_of(prec);
+    pack(in, prec, S);
     bool first = true;
     for (int kind = 0; kind < 2; kind++) {
         if (!on[kind]) continue;
@@ -1580,8 +1597,7 @@ void Operator::p2p(const double *in, double *out, double cId, double cSL, double
         if (first) analyse(active, side);
         near_terms(kind, cSL, cTrac, active, side);
         if (side != stream_) SPHSTK_HIP(hipEventRecord(ev_join_, side));
-        LevelSet *S = nullptr;
-        const FarSum f = far(kind, prec, kind == 0 ? -3.0 / (4.0 * kPi) * cTrac : cSL / (8.0 * kPi), in, active, &S);
+        const FarSum f = far(S, kind, prec, kind == 0 ? -3.0 / (4.0 * kPi) * cTrac : cSL / (8.0 * kPi), in, active);
         if (side != stream_) SPHSTK_HIP(hipStreamWaitEvent(stream_, ev_join_, 0));
         launch_sheval_gather(geom_, d_trg_slot_off_.p, d_trg_nsrc_.p, evscratch_.p, f, in, out, cid, clop,
                              overwrite && first, active, stream_);
@@ -1744,7 +1760,7 @@ void Operator::rigid_velocity(const double *rho, double inv_mu, double *vel) {
     launch_rigid_avg(geom_, u_ns_.p, inv_mu, vel_ns_.p, stream_);
     launch_far_centre(src64_.p, d_pos_.p, lists_centre_.ngroups, lists_centre_.order.p, lists_centre_.groups.p,
                       lists_centre_.iv.p, centre_part_.p, nsph_, stream_);
-    launch_centre_finish(nsph_, lists_centre_.split, centre_part_.p, d_rad_.p, vel_ns_.p, inv_mu, vel, stream_);
+    launch_centre_finish(nsph_, lists_centre_.nslot(), centre_part_.p, d_rad_.p, vel_ns_.p, inv_mu, vel, stream_);
     SPHSTK_HIP(hipGetLastError());
 }
 
@@ -1994,8 +2010,7 @@ void Operator::kernel_stats(int kind, int prec, double *ms, int64_t *launches, d
                             : (prec == 3 && multi_level_) ? &lsc_
                                                           : nullptr;
         if (S && S->ready) {
-            *pairs = S->mid.pairs + (S->agg ? S->agg->pairs : 0.0);
-            for (auto &L : S->levels) *pairs += L->lists.pairs;
+            *pairs = S->all.pairs;
         } else {
             *pairs = lists_fine_.pairs * (prec == 0 ? ncopy_ : 1); // copies: per-copy lists, all copies summed
         }

@@ -74,8 +74,6 @@ struct FarLists {
     DevBuf<FarInterval> iv;
     DevBuf<int> order;
     DevBuf<double> part; // split partial-sum slots of 3*ntrg doubles
-    DevBuf<double> cen;  // sphere-aligned lists: centre of each group's target sphere (4 per group)
-    bool aligned = false;
     int ngroups = 0, tpl = 1, split = 1;
     double pairs = 0.0; // algorithmic pairs per launch
     int64_t ntrg = 0;
@@ -96,22 +94,36 @@ inline void run_append(Runs &r, int s) {
 }
 Runs runs_of(const std::vector<int> &lst, int s0, int s1, bool include);
 
+// Work items on the host: groups in any order, their intervals, and their work.
+struct HostLists {
+    std::vector<FarGroup> groups;
+    std::vector<FarInterval> ivs;
+    std::vector<int64_t> work;
+    double pairs = 0.0;
+    int nlist = 0;
+};
+// Where a list's points and slots lie in the point sets and slots of a joint
+// list: its targets from target trg on, its sources from source src on, its
+// first slot.
+struct ListBase {
+    int64_t trg = 0, src = 0;
+    int slot = 0;
+};
+// Appends a list's work items; returns its slots (0: it has no pairs).
 // src_susp_off: first source "sphere" (entry of soff) of each suspension when
 // the source point set is not the target's sphere set (NULL: susp_sph_off).
+int append_far_lists(HostLists &H, int nsusp, const std::vector<int64_t> &susp_sph_off, const std::vector<int64_t> &toff,
+                     const std::vector<int64_t> &soff, const std::vector<Runs> &runs, int tpl, int split,
+                     int64_t want_items, const std::vector<int64_t> *src_susp_off = nullptr, ListBase at = ListBase{});
+void upload_far_lists(FarLists &L, HostLists &H, int tpl, int split, int64_t ntrg);
 void build_far_lists(FarLists &L, int nsusp, const std::vector<int64_t> &susp_sph_off,
                      const std::vector<int64_t> &toff, const std::vector<int64_t> &soff, const std::vector<Runs> &runs,
-                     int tpl, int split, int64_t want_items, const double *sph_pos = nullptr,
-                     const std::vector<int64_t> *src_susp_off = nullptr);
+                     int tpl, int split, int64_t want_items, const std::vector<int64_t> *src_susp_off = nullptr);
 
-// One level of the multi-level FP32 far field: per-sphere grids of a lower
-// order, their geometry, resampling tables and work lists.
+// One level of a multi-level far field: per-sphere grids of a lower order.
 struct FarLevel {
-    int64_t npts = 0;
     DevBuf<int64_t> d_off_by_sph; // first level point of each sphere
-    DevBuf<double> coords, norms, w;
-    DevBuf<float> src32, trg32;
-    DevBuf<double> src64;
-    FarLists lists;
+    DevBuf<double> w;
 };
 
 // Device copies of one matrix per order in the layout of the transform GEMMs.
@@ -133,21 +145,23 @@ constexpr double kCellTheta = 4.0;
 struct CellAgg {
     int ncell = 0;
     const EquivTables *E = nullptr;   // the set's equivalent-source template
-    double pairs = 0.0;               // pair evaluations of the two cell lists (per apply)
     double check_pairs = 0.0;         // pair evaluations of the check velocities (per apply)
     std::vector<int64_t> susp_cell_off; // first cell of each suspension
     DevBuf<float> chk32;              // check points as FP32 target records (zero normals)
-    DevBuf<float> eq32;               // equivalent points as FP32 source records (forces per apply)
+    float *eq32 = nullptr;            // equivalent points among the set's source records (forces per apply)
     DevBuf<double> P;                 // template fit, column-major (3K x 3Kc)
     DevBuf<double> rho;               // cell radius
     DevBuf<int> susp;                 // cell suspension
     FarLists chk_lists;               // check points of a cell x the fine grids of its members
                                       // (its slots: the check velocities, 3 Kc per cell)
-    FarLists lists[2];                // level-2 / level-3 target grids x equivalent points
 };
 
 // A multi-level far field: fine-grid sums for the pairs closer than the first
-// level's separation (mid), then one coarser grid per separation shell.
+// level's separation (mid), then one coarser grid per separation shell.  The
+// point sets of the fine grid, the levels and the source cells follow each other
+// in one array of sources and one of targets, so that all lists of the set are
+// one launch (64 points of a level are a few spheres: on their own, the lists of
+// 100 to 1000 spheres each left most of the GPU idle).
 constexpr int kNumLevels = 4; // levels of the FP32 sets (source cells on their last two)
 struct LevelSet {
     int nlev = kNumLevels;   // levels in use
@@ -157,7 +171,10 @@ struct LevelSet {
     bool fp64 = false;       // FP64 pair sums (else FP32)
     int tpl = 1;             // targets per lane of its work lists
     std::vector<std::unique_ptr<FarLevel>> levels;
-    FarLists mid;
+    FarLists all;                     // mid range, levels, source cells
+    int mid_slots = 0;                // slots of the mid range (the fine grid's targets come first)
+    DevBuf<float> src32, trg32;       // source and target records (FP32 set)
+    DevBuf<double> src64, coords, norms; // source records and targets (FP64 set)
     GemmTables down, up;              // resampling to all levels at once, and back
     LevelViews views;
     int max_lev_pts = 0;              // most stacked level points of a sphere
@@ -263,12 +280,14 @@ class Operator {
 
   private:
     // far field of the densities packed by pack() (FP64 direct sum of copies: of
-    // `in`): the fine-grid part as slots; *levels: the level set whose level
-    // fields are still to be added by levels_up (NULL: none)
-    FarSum far(int kind, int prec, double coef, const double *in, const int *active, LevelSet **levels);
+    // `in`): the fine-grid part as slots; the level fields of S are still to be
+    // added by levels_up
+    FarSum far(LevelSet *S, int kind, int prec, double coef, const double *in, const int *active);
+    // the level set of precision prec, built (NULL: direct sums)
+    LevelSet *set_of(int prec);
     // body-frame values and far-field sources of `in` for an apply of precision
-    // prec (-1: the values alone)
-    void pack(const double *in, int prec);
+    // prec on set S (prec -1: the values alone)
+    void pack(const double *in, int prec, const LevelSet *S = nullptr);
     void analyse(const int *active, hipStream_t s) {
         launch_analysis(geom_, anal_.view, body64_.p, coef_.p, cbody_.p, active, s);
     }

@@ -66,9 +66,9 @@ struct LevelViews {
     const int64_t *off[kMaxLevels] = {};
     const double *w[kMaxLevels] = {};
     void *src[kMaxLevels] = {};              // source records (force words written per apply)
-    const double *part[kMaxLevels][2] = {};  // partial-sum slots of the level's lists (level, source cells)
-    int nslot[kMaxLevels][2] = {};
-    int64_t stride[kMaxLevels] = {};         // between slots
+    const double *part[kMaxLevels] = {};     // partial-sum slots of the level's lists (level, then source cells)
+    int nslot[kMaxLevels] = {};
+    int64_t stride = 0;                      // between slots
     const int64_t *body_off = nullptr;       // per tile: body-frame values of the stacked level points
 };
 

@@ -102,11 +102,9 @@ __global__ __launch_bounds__(256) void k_pack_levels(DevGeom g, LevelViews L, T 
         while (k >= first[l + 1]) l++;
         const int64_t i = 3 * (L.off[l][S] + k - first[l]);
         double v[3] = {0.0, 0.0, 0.0};
-        for (int q = 0; q < 2; q++) {
-            const double *part = L.part[l][q] + i;
-            for (int s = 0; s < L.nslot[l][q]; s++, part += L.stride[l])
-                for (int c = 0; c < 3; c++) v[c] += part[c];
-        }
+        const double *part = L.part[l] + i;
+        for (int s = 0; s < L.nslot[l]; s++, part += L.stride)
+            for (int c = 0; c < 3; c++) v[c] += part[c];
         rotate(g.quat + 4 * S, -1.0, v, o);
     }
     const int64_t base = L.body_off[blockIdx.y];
