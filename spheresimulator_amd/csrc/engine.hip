@@ -28,6 +28,7 @@ namespace {
 constexpr int kMaxSupportedOrder = 20; // LDS of the expansion kernel bounds the order
 constexpr int64_t kChunk = 4096;  // DOF per block of the segmented vector kernels
 constexpr int64_t kWantItems = 40000; // far-field work items wanted when a problem is small
+constexpr int64_t kMultiItems = 8192; // the same for several right-hand sides on one geometry
 constexpr int64_t kLookaheadDof = 300000; // GMRES below this many unknowns launches one iteration ahead
 constexpr double kTuneBudget = 3.0;    // seconds per autotuning pass (SPHSTK_FLAG_AUTOTUNE)
 
@@ -420,7 +421,11 @@ Operator::Operator(int nsusp, const int *counts, const double *pos, const double
             const std::vector<int64_t> so0(susp_sph_off_.begin(), susp_sph_off_.begin() + b0 + 1),
                 po0(pt_off_.begin(), pt_off_.begin() + s0 + 1);
             const std::vector<Runs> r0(runs_fine_.begin(), runs_fine_.begin() + s0);
-            build_far_lists(lists_fine_, b0, so0, po0, po0, r0, 1, split, kWantItems);
+            // items for eight waves per SIMD: each slice adds a partial-sum pass
+            // over all copies
+            const int64_t nb = std::max<int64_t>(1, pt_off_[s0] / (64 * kMultiTPL));
+            const int slices = (int)std::max<int64_t>(1, std::min<int64_t>(32, (kMultiItems + nb - 1) / nb));
+            build_far_lists(lists_fine_, b0, so0, po0, po0, r0, kMultiTPL, slices, kWantItems);
             if (lists_fine_.pairs > 0.0) lists_fine_.part.alloc(size_t(lists_fine_.split) * 3 * npts_);
             srcm_.alloc(std::max<int64_t>(4 * (std::min(ncopy_, kMultiCols) + 1) * pt_off_[s0], 8));
         } else {
@@ -1458,7 +1463,7 @@ void Operator::far_copies(int kind, double coef, const double *in, const int *ac
             const int nc = std::min(kMultiCols, ncopy_ - c0);
             launch_far_trac_multi(nc, n0, d_coords_.p, d_norms_.p, d_w_.p, in + c0 * col, col, srcm_.p, L.ngroups,
                                   L.order.p, L.groups.p, L.iv.p, active ? active + c0 * b0 : nullptr, b0,
-                                  L.part.p + c0 * col, coef, 0, 3 * npts_, stream_);
+                                  L.part.p + c0 * col, coef, 3 * npts_, stream_);
         }
         return;
     }

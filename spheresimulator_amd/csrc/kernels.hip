@@ -1454,6 +1454,10 @@ __global__ void k_pack_src_multi(int64_t n0, const double *__restrict__ coords, 
     }
 }
 
+// kMultiTPL targets per lane: a record of 8 densities is 36 doubles, nearly all
+// scalar registers, so the next one cannot be loaded ahead, and one target per
+// lane (74 VALU slots) does not cover its latency (150 spheres p=10, 8 columns:
+// 5.56 ms per apply against 2.6 ms of VALU issue).
 template <int NC>
 __global__ __launch_bounds__(64) void k_far_trac_multi_f64(const double *__restrict__ src,
                                                            const double *__restrict__ coords,
@@ -1462,74 +1466,69 @@ __global__ __launch_bounds__(64) void k_far_trac_multi_f64(const double *__restr
                                                            const FarGroup *__restrict__ groups,
                                                            const FarInterval *__restrict__ iv,
                                                            const int *__restrict__ active, int nsusp0,
-                                                           double *__restrict__ out, double coef, int accumulate,
+                                                           double *__restrict__ out, double coef,
                                                            int64_t slot_stride, int64_t col_stride) {
+    constexpr int N = kMultiTPL;
     const FarGroup G = groups[gorder[blockIdx.x]];
     bool any = !active;
 #pragma unroll
     for (int c = 0; c < NC; c++) any = any || active[c * nsusp0 + G.susp];
     if (!any) return;
     const int lane = threadIdx.x;
-    const int64_t t = G.tstart + (lane < G.tcount ? lane : 0);
-    const double x = coords[3 * t], y = coords[3 * t + 1], z = coords[3 * t + 2];
-    const double nx = norms[3 * t], ny = norms[3 * t + 1], nz = norms[3 * t + 2];
-    double ax[NC], ay[NC], az[NC];
+    double x[N], y[N], z[N], nx[N], ny[N], nz[N], ax[N][NC], ay[N][NC], az[N][NC];
 #pragma unroll
-    for (int c = 0; c < NC; c++) ax[c] = ay[c] = az[c] = 0.0;
+    for (int t = 0; t < N; t++) {
+        const int idx = 64 * t + lane;
+        const int64_t i = G.tstart + (idx < G.tcount ? idx : 0);
+        x[t] = coords[3 * i];
+        y[t] = coords[3 * i + 1];
+        z[t] = coords[3 * i + 2];
+        nx[t] = norms[3 * i];
+        ny[t] = norms[3 * i + 1];
+        nz[t] = norms[3 * i + 2];
+#pragma unroll
+        for (int c = 0; c < NC; c++) ax[t][c] = ay[t][c] = az[t][c] = 0.0;
+    }
     constexpr int RS = 4 * (NC + 1);
-    auto pair = [&](const double *v, bool incl) {
-        const double dx = x - v[0], dy = y - v[1], dz = z - v[2];
-        const double r2 = fmad(dx, dx, fmad(dy, dy, dz * dz));
-        double wq = trac_w_f64(r2);
-        wq = incl ? wq : 0.0;
-        const double dnw = fmad(dx, nx, fmad(dy, ny, dz * nz)) * wq;
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-            const double *f = v + 4 * (c + 1);
-            const double q = fmad(dx, f[0], fmad(dy, f[1], dz * f[2])) * dnw;
-            ax[c] = fmad(q, dx, ax[c]);
-            ay[c] = fmad(q, dy, ay[c]);
-            az[c] = fmad(q, dz, az[c]);
-        }
-    };
-    // up to 4 columns: two sources per step, their wave-uniform (scalar) loads
-    // issued before the arithmetic of either; more columns: one (a record of
-    // 4 (NC + 1) doubles fills the scalar registers)
-    constexpr int U = NC <= 4 ? 2 : 1;
     for (int64_t k = G.iv_begin; k < G.iv_end; k++) {
         const int64_t b = iv[k].begin, e = iv[k].end;
-        const bool incl = ((iv[k].mask[0] >> lane) & 1ull) != 0;
-        int64_t s = b;
-        for (; s + U <= e; s += U) {
-            double v[U][RS];
+        bool incl[N];
 #pragma unroll
-            for (int u = 0; u < U; u++)
-#pragma unroll
-                for (int j = 0; j < RS; j++) v[u][j] = src[RS * (s + u) + j];
-#pragma unroll
-            for (int u = 0; u < U; u++) pair(v[u], incl);
-        }
-        if (s < e) {
+        for (int t = 0; t < N; t++) incl[t] = ((iv[k].mask[t] >> lane) & 1ull) != 0;
+        for (int64_t s = b; s < e; s++) {
             double v[RS];
 #pragma unroll
             for (int j = 0; j < RS; j++) v[j] = src[RS * s + j];
-            pair(v, incl);
+#pragma unroll
+            for (int t = 0; t < N; t++) {
+                const double dx = x[t] - v[0], dy = y[t] - v[1], dz = z[t] - v[2];
+                const double r2 = fmad(dx, dx, fmad(dy, dy, dz * dz));
+                double wq = trac_w_f64(r2);
+                wq = incl[t] ? wq : 0.0;
+                const double dnw = fmad(dx, nx[t], fmad(dy, ny[t], dz * nz[t])) * wq;
+#pragma unroll
+                for (int c = 0; c < NC; c++) {
+                    const double *f = v + 4 * (c + 1);
+                    const double q = fmad(dx, f[0], fmad(dy, f[1], dz * f[2])) * dnw;
+                    ax[t][c] = fmad(q, dx, ax[t][c]);
+                    ay[t][c] = fmad(q, dy, ay[t][c]);
+                    az[t][c] = fmad(q, dz, az[t][c]);
+                }
+            }
         }
     }
-    if (lane >= G.tcount) return;
     const double cf = kTracW * coef;
 #pragma unroll
     for (int c = 0; c < NC; c++) {
         if (active && !active[c * nsusp0 + G.susp]) continue;
-        double *o = out + (accumulate ? 0 : G.slot * slot_stride) + c * col_stride + 3 * (G.tstart + lane);
-        if (accumulate) {
-            o[0] += cf * ax[c];
-            o[1] += cf * ay[c];
-            o[2] += cf * az[c];
-        } else {
-            o[0] = cf * ax[c];
-            o[1] = cf * ay[c];
-            o[2] = cf * az[c];
+#pragma unroll
+        for (int t = 0; t < N; t++) {
+            const int idx = 64 * t + lane;
+            if (idx >= G.tcount) continue;
+            double *o = out + G.slot * slot_stride + c * col_stride + 3 * (G.tstart + idx);
+            o[0] = cf * ax[t][c];
+            o[1] = cf * ay[t][c];
+            o[2] = cf * az[t][c];
         }
     }
 }
@@ -1537,25 +1536,25 @@ __global__ __launch_bounds__(64) void k_far_trac_multi_f64(const double *__restr
 template <int NC>
 static void far_trac_multi(int64_t n0, const double *coords, const double *norms, const double *w, const double *in,
                            int64_t col_stride, double *src, int ngroups, const int *go, const FarGroup *gr,
-                           const FarInterval *iv, const int *active, int nsusp0, double *out, double coef, int acc,
+                           const FarInterval *iv, const int *active, int nsusp0, double *out, double coef,
                            int64_t slot_stride, hipStream_t s) {
     if (n0 > 0)
         k_pack_src_multi<NC><<<dim3((unsigned)((n0 + 255) / 256)), dim3(256), 0, s>>>(n0, coords, w, in, col_stride,
                                                                                      src);
     if (ngroups > 0)
         k_far_trac_multi_f64<NC><<<dim3(ngroups), dim3(64), 0, s>>>(src, coords, norms, go, gr, iv, active, nsusp0, out,
-                                                                   coef, acc, slot_stride, col_stride);
+                                                                   coef, slot_stride, col_stride);
 }
 
 void launch_far_trac_multi(int ncol, int64_t n0, const double *coords, const double *norms, const double *w,
                            const double *in, int64_t col_stride, double *src, int ngroups, const int *go,
                            const FarGroup *gr, const FarInterval *iv, const int *active, int nsusp0, double *out,
-                           double coef, int acc, int64_t slot_stride, hipStream_t s) {
+                           double coef, int64_t slot_stride, hipStream_t s) {
     switch (ncol) {
 #define SPHSTK_MULTI_CASE(NC)                                                                                      \
     case NC:                                                                                                       \
         far_trac_multi<NC>(n0, coords, norms, w, in, col_stride, src, ngroups, go, gr, iv, active, nsusp0, out, coef, \
-                           acc, slot_stride, s);                                                                   \
+                           slot_stride, s);                                                                        \
         break;
         SPHSTK_MULTI_CASE(1)
         SPHSTK_MULTI_CASE(2)

@@ -206,11 +206,13 @@ void launch_fill(int64_t n, double v, double *y, hipStream_t s);
 // FP64 traction far field of ncol (1..8) densities on one geometry: `in` holds
 // ncol DOF vectors col_stride apart, of which the first n0 points carry the
 // geometry and work lists; src is scratch of 4 (ncol + 1) doubles per point;
-// out (or its split slots, slot_stride apart) has the same column layout.
+// the slots (slot_stride apart) have the same column layout.  The work lists are
+// those of kMultiTPL targets per lane.
+constexpr int kMultiTPL = 2;
 void launch_far_trac_multi(int ncol, int64_t n0, const double *coords, const double *norms, const double *w,
                            const double *in, int64_t col_stride, double *src, int ngroups, const int *go,
                            const FarGroup *gr, const FarInterval *iv, const int *active, int nsusp0, double *out,
-                           double coef, int acc, int64_t slot_stride, hipStream_t s);
+                           double coef, int64_t slot_stride, hipStream_t s);
 // sphere-centre far field (Faxen) of packed FP64 sources, 9 sums per centre and slot
 // out (+)= coef K'[rho0] at grid points from distant spheres' rigid-body densities, in closed form (Stokeslet,
 // degenerate quadrupole and rotlet at the centres); force holds (F, T) per sphere
