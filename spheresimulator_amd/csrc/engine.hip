@@ -26,8 +26,11 @@ namespace sphstk {
 namespace {
 
 constexpr int kMaxSupportedOrder = 20; // LDS of the expansion kernel bounds the order
-constexpr int64_t kChunk = 4096;  // DOF per block of the segmented vector kernels
+constexpr int64_t kChunk = 4096;  // most DOF per block of the segmented vector kernels
+constexpr int64_t kMinChunk = 512; // fewest, on problems that would not fill the GPU with kChunk
+constexpr int64_t kWantChunks = 1024;
 constexpr int64_t kWantItems = 40000; // far-field work items wanted when a problem is small
+constexpr int kSumsInBlock = 1024; // GMRES: most chunk partials of a segment that every block adds up itself
 constexpr int64_t kMultiItems = 8192; // the same for several right-hand sides on one geometry
 constexpr int64_t kLookaheadDof = 300000; // GMRES below this many unknowns launches one iteration ahead
 constexpr double kTuneBudget = 3.0;    // seconds per autotuning pass (SPHSTK_FLAG_AUTOTUNE)
@@ -343,7 +346,8 @@ Operator::Operator(int nsusp, const int *counts, const double *pos, const double
     chunks_.upload(ch);
     seg_chunk_off_.upload(sco);
     seg_chunk_off_host_ = sco;
-    partial_.alloc(std::max<size_t>(ch.size(), 1));
+    partial_.alloc(2 * std::max<size_t>(ch.size(), 1));
+    for (int b = 0; b < nsusp_; b++) max_seg_chunks_ = std::max(max_seg_chunks_, sco[b + 1] - sco[b]);
 
     int tpl = 1, split = 0;
     // FP32 inner operator: orders from level_order().  FP64 outer applies: fine
@@ -865,10 +869,12 @@ void build_far_lists(FarLists &L, int nsusp, const std::vector<int64_t> &susp_sp
 static std::vector<Chunk> make_chunks(int nsusp, const std::vector<int64_t> &susp_sph_off,
                                       const std::vector<int64_t> &off, std::vector<int> *seg_off) {
     std::vector<Chunk> ch;
+    const int64_t total = 3 * off[susp_sph_off[nsusp]];
+    const int64_t size = std::min(kChunk, std::max(kMinChunk, (total / kWantChunks + 255) / 256 * 256));
     if (seg_off) seg_off->assign(nsusp + 1, 0);
     for (int b = 0; b < nsusp; b++) {
         const int64_t d0 = 3 * off[susp_sph_off[b]], d1 = 3 * off[susp_sph_off[b + 1]];
-        for (int64_t a = d0; a < d1; a += kChunk) ch.push_back(Chunk{a, std::min(a + kChunk, d1), b, 0});
+        for (int64_t a = d0; a < d1; a += size) ch.push_back(Chunk{a, std::min(a + size, d1), b, 0});
         if (seg_off) (*seg_off)[b + 1] = (int)ch.size();
     }
     return ch;
@@ -2070,7 +2076,6 @@ Mobility::Mobility(int nsusp, const int *counts, const double *pos, const double
     vel_.alloc(std::max(6 * A_->nsph(), 1));
     act_.alloc(A_->nsusp());
     scal_.alloc(4 * (size_t)A_->nsusp());
-    d_nact_.alloc(1);
     coarse_inner_ = prec_ == 1 && (flags & 128) == 0 && A_->has_coarse();
     if (prec_ == 1) A_->prepare_mixed(outer_prec_ == 2, coarse_inner_);
     SPHSTK_HIP(hipStreamSynchronize(A_->stream()));
@@ -2118,6 +2123,9 @@ void Mobility::gmres(const double *b, double *x, bool x_zero, double tol, int pr
     const int nch = A.nchunks();
     const int *sco = A.seg_chunk_off();
     double *part = A.scratch_partial();
+    // a block of the vector kernels adds up the partials of its segment itself
+    // while they are few (every block reads them all)
+    const int sums = A.max_seg_chunks() <= kSumsInBlock ? 1 : 0;
     // inner solve: right preconditioning by the isolated-sphere inverse,
     // A M^-1 u = r, d = M^-1 u (the residual stays the unpreconditioned one)
     const bool rprec = (prec == 1 || prec == 3) && inner_precond_;
@@ -2208,29 +2216,33 @@ void Mobility::gmres(const double *b, double *x, bool x_zero, double tol, int pr
             // Gram-Schmidt twice: all j+1 products of a pass in one kernel),
             // which stores -h.
             const bool cgs2 = prec != 0 && m + 1 <= 64;
-            for (int pass = 0; pass < 2; pass++) {
-                if (cgs2) {
+            double *nv = h_.p + size_t(2 * (m + 1)) * B;
+            double *pp[2] = {part, part + std::max(nch, 1)}; // partials of this step and of the one before
+            int cur = 0;
+            if (cgs2) {
+                for (int pass = 0; pass < 2; pass++) {
                     double *hv = h_.p + size_t(pass * (m + 1)) * B;
                     launch_seg_multi_dot(W, V_.p, n, j + 1, ch, nch, mdot_.p, act_.p, st);
                     launch_seg_multi_reduce(mdot_.p, nch, sco, B, j + 1, hv, 2, act_.p, st);
-                    launch_seg_multi_axpy(W, V_.p, n, hv, j + 1, B, ch, nch, act_.p, st);
-                    continue;
+                    launch_seg_multi_axpy(W, V_.p, n, hv, j + 1, B, ch, nch, act_.p, st, pass ? pp[cur] : nullptr);
                 }
-                for (int i = 0; i <= j; i++) {
-                    double *hv = h_.p + size_t(pass * (m + 1) + i) * B;
-                    launch_seg_dot(W, V_.p + size_t(i) * n, ch, nch, part, act_.p, st);
-                    launch_seg_reduce(part, sco, B, hv, 0, act_.p, st);
-                    launch_seg_axpy(W, V_.p + size_t(i) * n, hv, -1.0, ch, nch, act_.p, st);
+            } else {
+                const double *vp = nullptr;
+                double *hp = nullptr;
+                for (int k = 0; k <= 2 * (j + 1); k++) { // the last step: |w|
+                    const int pass = k / (j + 1), i = k % (j + 1);
+                    const double *Vi = k < 2 * (j + 1) ? V_.p + size_t(i) * n : nullptr;
+                    cur ^= 1;
+                    launch_seg_mgs(W, vp, pp[cur ^ 1], sums, hp, Vi, pp[cur], sco, ch, nch, act_.p, st);
+                    vp = Vi;
+                    hp = Vi ? h_.p + size_t(pass * (m + 1) + i) * B : nv;
+                    if (!sums) launch_seg_reduce(pp[cur], sco, B, hp, 0, act_.p, st);
                 }
             }
-            double *nv = h_.p + size_t(2 * (m + 1)) * B;
-            launch_seg_dot(W, W, ch, nch, part, act_.p, st);
-            launch_seg_reduce(part, sco, B, nv, 0, act_.p, st);
-            launch_seg_reduce(part, sco, B, scal_.p, 1, act_.p, st);
-            launch_seg_scale(W, W, scal_.p, ch, nch, act_.p, st);
+            if (cgs2 && !sums) launch_seg_reduce(pp[cur], sco, B, nv, 0, act_.p, st);
+            launch_seg_normalise(W, pp[cur], sums, nv, sco, ch, nch, act_.p, st);
             launch_gmres_givens(B, j, m, h_.p, cgs2 ? -1.0 : 1.0, d_H_.p, d_cs_.p, d_sn_.p, d_g_.p, d_bn_.p, tol,
-                                act_.p, d_kdim_.p, d_impok_.p, d_relres_.p, d_nact_.p, st);
-            SPHSTK_HIP(hipMemcpyAsync(nact_host_ + (j & 1), d_nact_.p, sizeof(int), hipMemcpyDeviceToHost, st));
+                                act_.p, d_kdim_.p, d_impok_.p, d_relres_.p, nact_host_ + (j & 1), st);
             SPHSTK_HIP(hipEventRecord(nact_ev_[j & 1], st));
             total++;
             kmax = j + 1;

@@ -276,7 +276,8 @@ class Operator {
     const int *seg_chunk_off() const { return seg_chunk_off_.p; }
     const std::vector<int64_t> &susp_sph_off() const { return susp_sph_off_; }
     const std::vector<int64_t> &pt_off() const { return pt_off_; }
-    double *scratch_partial() { return partial_.p; }
+    double *scratch_partial() { return partial_.p; } // two partials per chunk
+    int max_seg_chunks() const { return max_seg_chunks_; }
 
   private:
     // far field of the densities packed by pack() (FP64 direct sum of copies: of
@@ -402,6 +403,7 @@ class Operator {
     DevBuf<Chunk> chunks_;
     DevBuf<int> seg_chunk_off_;
     std::vector<int> seg_chunk_off_host_;
+    int max_seg_chunks_ = 0;
     DevBuf<double> partial_;
 
     // timing
@@ -467,7 +469,7 @@ class Mobility {
     // device-side GMRES least-squares state (per suspension) and the pinned
     // count of active suspensions read one iteration late behind an event
     DevBuf<double> d_H_, d_cs_, d_sn_, d_g_, d_bn_, d_beta_, d_relres_;
-    DevBuf<int> d_cyc_, d_kdim_, d_impok_, d_nact_;
+    DevBuf<int> d_cyc_, d_kdim_, d_impok_;
     int *nact_host_ = nullptr;
     hipEvent_t nact_ev_[2] = {nullptr, nullptr};
 };

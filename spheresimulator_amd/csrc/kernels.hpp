@@ -168,15 +168,23 @@ void launch_seg_axpy(double *y, const double *x, const double *alpha, double sig
 // y = alpha[seg] * x
 void launch_seg_scale(double *y, const double *x, const double *alpha, const Chunk *chunks, int nchunks,
                       const int *active, hipStream_t s);
-// x += sum_i coef[i*nseg + seg] * V[i]   (i < k)
+// modified Gram-Schmidt: h = (sums: added up from pprev, else) hprev, w -= h vprev (vprev NULL: not), then the
+// chunk partials of w.v (v NULL: w.w); and w /= |w| from those of w.w, nv = |w|^2
+void launch_seg_mgs(double *w, const double *vprev, const double *pprev, int sums, double *hprev, const double *v,
+                    double *partial, const int *off, const Chunk *chunks, int nchunks, const int *active,
+                    hipStream_t s);
+void launch_seg_normalise(double *w, const double *partial, int sums, double *nv, const int *off, const Chunk *chunks,
+                          int nchunks, const int *active, hipStream_t s);
 // partial[j * nchunks + chunk] = w . V_j over the chunk, j < k <= 64 (one pass over w)
 void launch_seg_multi_dot(const double *w, const double *V, int64_t ldv, int k, const Chunk *chunks, int nchunks,
                           double *partial, const int *active, hipStream_t s);
 // out[j * nseg + seg] = sum of seg's chunk partials (op 2: negated), j < k
 void launch_seg_multi_reduce(const double *partial, int nchunks, const int *off, int nseg, int k, double *out, int op,
                              const int *active, hipStream_t s);
+// x += sum_i coef[i*nseg + seg] * V[i]   (i < k); norm (optional): chunk partials of x.x afterwards
 void launch_seg_multi_axpy(double *x, const double *V, int64_t ldv, const double *coef, int k, int nseg,
-                           const Chunk *chunks, int nchunks, const int *active, hipStream_t s);
+                           const Chunk *chunks, int nchunks, const int *active, hipStream_t s,
+                           double *norm = nullptr);
 // x = sum_j coef[j nseg + seg] V_j over the active segments (x overwritten there)
 void launch_seg_multi_comb(double *x, const double *V, int64_t ldv, const double *coef, int k, int nseg,
                            const Chunk *chunks, int nchunks, const int *active, hipStream_t s);
