@@ -58,6 +58,7 @@ struct FarGroup {
 // Number of complex arrays in the per-sphere expansion records.
 constexpr int kRecSL = 10;   // grad H1, grad H2, H3, grad H4
 constexpr int kRecTrac = 23; // Hess H1, grad H2, Hess H2, H3, grad H3, Hess H4, P (Hessians without zz)
+constexpr int kRecTracPad = 24; // arrays per term in memory (48 doubles: three rows of 16 lanes)
 
 // Host-side spherical-harmonic tables for one order p.
 struct ShTables {

@@ -215,7 +215,7 @@ Operator::Operator(int nsusp, const int *counts, const double *pos, const double
     }
 
     for (int i = 0; i < nsph_; i++)
-        rec_off_[i + 1] = rec_off_[i] + (near_off_[i + 1] > near_off_[i] ? 2 * kRecTrac * tri_size(order_[i] + 2) : 0);
+        rec_off_[i + 1] = rec_off_[i] + (near_off_[i + 1] > near_off_[i] ? 2 * kRecTracPad * tri_size(order_[i] + 2) : 0);
 
     // slots of the self and near terms: per target sphere its own first, then its
     // near sources in list order; near evaluation work items in chunks of 128

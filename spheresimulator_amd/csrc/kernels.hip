@@ -597,7 +597,7 @@ __global__ __launch_bounds__(256) void k_expand(DevGeom g, int mode, const int *
     }
     __syncthreads();
     // record
-    const int K = (mode == 0) ? kRecSL : kRecTrac;
+    const int K = (mode == 0) ? kRecSL : kRecTracPad;
     double2 *R = reinterpret_cast<double2 *>(rec + g.rec_off[S]);
     const int hd0[5] = {0, 0, 0, 1, 1}, hd1[5] = {0, 1, 2, 1, 2};
     for (int idx = threadIdx.x; idx < K * Q2; idx += blockDim.x) {
@@ -628,7 +628,7 @@ __global__ __launch_bounds__(256) void k_expand(DevGeom g, int mode, const int *
                 c = hget(grad + (2 * 3 + (a - 14)) * Q1, P1, n2, m);
             else if (a < 22)
                 c = dcoef(grad + (3 * 3 + hd0[a - 17]) * Q1, P1, n2, m, hd1[a - 17]);
-            else
+            else if (a == 22)
                 c = hget(base + 4 * Q, p, n2, m);
         }
         const double eps = m ? 2.0 : 1.0;
@@ -757,45 +757,56 @@ __global__ __launch_bounds__(64) void k_sheval(DevGeom g, const double *__restri
 
 // Traction evaluation of the near items with the source's record in LDS: one
 // workgroup of kSrcWaves waves per source sphere S runs all items whose source
-// is S, the waves taking the items in turn.  The record (kRecTrac complex
-// arrays per term, (p+3)(p+4)/2 terms: 44 KB at p = 12) is read from global
-// memory once per source.  A broadcast LDS read of 16 bytes returns 16 bytes to
-// every lane, and one term is 23 of them against 46 FMAs, so the LDS return path
-// bounds a wave with one target per lane; items of more than 64 targets put two
-// on each lane, and the FP64 VALU bounds it.  With up to 256 VGPRs per lane (2
-// waves per SIMD) the reads of one batch overlap the arithmetic of the batch before.
+// is S, the waves taking the items in turn; the record (kRecTracPad complex
+// numbers per term, (p+3)(p+4)/2 terms: 46 KB at p = 12) is read from global
+// memory once per source.
+// A term is 46 coefficients against 46 FMAs per target.  A broadcast LDS read
+// returns its value to every lane, 23 of 16 bytes for each term, which bound the
+// kernel even with two targets per lane (3000 spheres p=12 in chains: 2.0 ms
+// against 1.0 ms of FMA issue).  So lane i of every 16 reads coefficients i, i + 16
+// and i + 32 of a term, three reads of 8 bytes, and v_fmac_f64 takes the
+// coefficient it needs from that lane of its row (DPP row_newbcast, the only DPP
+// form of 64-bit operations; it runs at the rate of the plain FMA).
 // One launch per sphere order over that order's spheres with near neighbours,
 // LDS sized to its record; workgroup b takes list entry (b % 8) ceil(n / 8) + b / 8
 // (XCD-contiguous, as k_sheval).
 constexpr int kSrcWaves = 4;
 
-template <int CNT>
-__device__ __forceinline__ void lds_batch(const double2 *c, double2 *v) {
-#pragma unroll
-    for (int a = 0; a < CNT; a++) v[a] = c[a];
-    __builtin_amdgcn_sched_barrier(0); // these reads before the arithmetic that follows
+// acc[i] += c[lane 2 i of the row] cr + c[lane 2 i + 1] ci for the 8 (7) arrays of
+// one row of coefficients.  All lanes are active.  s_nop: a value that a VALU
+// instruction has just written (were the compiler to copy c) may be read through
+// DPP two wait states later.
+#define SPHSTK_BCAST(n, a, c, x) "v_fmac_f64_dpp %" #a ", %" #c ", " #x " row_newbcast:" #n " row_mask:0xf bank_mask:0xf\n"
+__device__ __forceinline__ void term_row8(double c, double cr, double ci, double *acc) {
+    asm("s_nop 1\n" SPHSTK_BCAST(1, 0, 8, %10) SPHSTK_BCAST(3, 1, 8, %10) SPHSTK_BCAST(5, 2, 8, %10)
+            SPHSTK_BCAST(7, 3, 8, %10) SPHSTK_BCAST(9, 4, 8, %10) SPHSTK_BCAST(11, 5, 8, %10)
+                SPHSTK_BCAST(13, 6, 8, %10) SPHSTK_BCAST(15, 7, 8, %10) SPHSTK_BCAST(0, 0, 8, %9)
+                    SPHSTK_BCAST(2, 1, 8, %9) SPHSTK_BCAST(4, 2, 8, %9) SPHSTK_BCAST(6, 3, 8, %9)
+                        SPHSTK_BCAST(8, 4, 8, %9) SPHSTK_BCAST(10, 5, 8, %9) SPHSTK_BCAST(12, 6, 8, %9)
+                            SPHSTK_BCAST(14, 7, 8, %9)
+        : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]), "+v"(acc[4]), "+v"(acc[5]), "+v"(acc[6]),
+          "+v"(acc[7])
+        : "v"(c), "v"(cr), "v"(ci));
 }
-template <int N, int BEG, int CNT>
-__device__ __forceinline__ void term_batch(const double2 *v, const double *cr, const double *ci,
-                                           double (*acc)[kRecTrac]) {
-#pragma unroll
-    for (int a = 0; a < CNT; a++)
-#pragma unroll
-        for (int t = 0; t < N; t++)
-            acc[t][BEG + a] = __builtin_fma(v[a].x, cr[t], __builtin_fma(v[a].y, ci[t], acc[t][BEG + a]));
-    __builtin_amdgcn_sched_barrier(0);
+__device__ __forceinline__ void term_row7(double c, double cr, double ci, double *acc) {
+    asm("s_nop 1\n" SPHSTK_BCAST(1, 0, 7, %9) SPHSTK_BCAST(3, 1, 7, %9) SPHSTK_BCAST(5, 2, 7, %9)
+            SPHSTK_BCAST(7, 3, 7, %9) SPHSTK_BCAST(9, 4, 7, %9) SPHSTK_BCAST(11, 5, 7, %9)
+                SPHSTK_BCAST(13, 6, 7, %9) SPHSTK_BCAST(0, 0, 7, %8) SPHSTK_BCAST(2, 1, 7, %8)
+                    SPHSTK_BCAST(4, 2, 7, %8) SPHSTK_BCAST(6, 3, 7, %8) SPHSTK_BCAST(8, 4, 7, %8)
+                        SPHSTK_BCAST(10, 5, 7, %8) SPHSTK_BCAST(12, 6, 7, %8)
+        : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]), "+v"(acc[4]), "+v"(acc[5]), "+v"(acc[6])
+        : "v"(c), "v"(cr), "v"(ci));
 }
+#undef SPHSTK_BCAST
 
 // acc[t][a] = sum over the terms (n, m) of Re(c_a D_n^m(xi_t)).  The terms of a
-// record lie in the order of the loop (m, then n), so that a term's 23
-// coefficients are read in batches of six, each while the batch before is used:
-// left to itself the compiler waits for every read of the two-target form (its
-// registers do not hold a whole term).  srec has kSrcBatch entries of slack.
-constexpr int kSrcBatch = 6;
+// record lie in the order of the loop (m, then n); the coefficients of the next
+// term are read while one is used (the last reads one term beyond the record:
+// slack).
 template <int N>
-__device__ __forceinline__ void eval_lds(const double2 *__restrict__ srec, int P, const double (*xi)[3],
+__device__ __forceinline__ void eval_lds(const double *__restrict__ srec, int P, const double (*xi)[3],
                                          double (*acc)[kRecTrac]) {
-    static_assert(kRecTrac == 23, "batches of 6, 6, 6 and 5");
+    static_assert(kRecTrac == 23 && kRecTracPad == 24, "rows of 8, 8 and 7 arrays");
     double nir2[N], nzi[N], dmr[N], dmi[N];
 #pragma unroll
     for (int t = 0; t < N; t++) {
@@ -807,9 +818,8 @@ __device__ __forceinline__ void eval_lds(const double2 *__restrict__ srec, int P
         dmr[t] = rsqrt_f64(r2); // D_m^m
         dmi[t] = 0.0;
     }
-    const double2 *c = srec;
-    double2 u[kSrcBatch], v[kSrcBatch];
-    lds_batch<6>(c, u);
+    const double *c = srec + (threadIdx.x & 15);
+    double v0 = c[0], v1 = c[16], v2 = c[32];
     for (int m = 0; m <= P; m++) {
         double pr[N], pi[N], cr[N], ci[N];
 #pragma unroll
@@ -826,15 +836,18 @@ __device__ __forceinline__ void eval_lds(const double2 *__restrict__ srec, int P
             ci[t] = dmi[t];
         }
         double odd = 2.0 * m + 1.0, nm = 0.0; // 2 n + 1, n^2 - m^2
-        for (int n = m; n <= P; n++, c += kRecTrac) {
-            lds_batch<6>(c + 6, v);
-            term_batch<N, 0, 6>(u, cr, ci, acc);
-            lds_batch<6>(c + 12, u);
-            term_batch<N, 6, 6>(v, cr, ci, acc);
-            lds_batch<5>(c + 18, v);
-            term_batch<N, 12, 6>(u, cr, ci, acc);
-            lds_batch<6>(c + 23, u);
-            term_batch<N, 18, 5>(v, cr, ci, acc);
+        for (int n = m; n <= P; n++) {
+            c += 2 * kRecTracPad;
+            const double w0 = c[0], w1 = c[16], w2 = c[32];
+#pragma unroll
+            for (int t = 0; t < N; t++) {
+                term_row8(v0, cr[t], ci[t], acc[t]);
+                term_row8(v1, cr[t], ci[t], acc[t] + 8);
+                term_row7(v2, cr[t], ci[t], acc[t] + 16);
+            }
+            v0 = w0;
+            v1 = w1;
+            v2 = w2;
 #pragma unroll
             for (int t = 0; t < N; t++) {
                 const double f1 = odd * nzi[t], f2 = nm * nir2[t];
@@ -852,7 +865,7 @@ __device__ __forceinline__ void eval_lds(const double2 *__restrict__ srec, int P
 
 // targets k = lane, lane + 64, ... (N of them; those beyond the item repeat its first) of one item
 template <int N>
-__device__ __forceinline__ void eval_item(const DevGeom &g, const EvalItem &it, const double2 *srec, int P,
+__device__ __forceinline__ void eval_item(const DevGeom &g, const EvalItem &it, const double *srec, int P,
                                           const double *q, const double *cen, double iR, double cTrac, int lane,
                                           double *__restrict__ scratch) {
     const int64_t g0 = g.pt_off[it.trg] + it.tstart;
@@ -885,7 +898,8 @@ __global__ __launch_bounds__(64 * kSrcWaves) __attribute__((amdgpu_waves_per_eu(
                                                               const int *__restrict__ srcs, int nsrc,
                                                               double *__restrict__ scratch, double cTrac,
                                                               const int *__restrict__ active) {
-    extern __shared__ double2 srec[];
+    extern __shared__ double2 srec2[];
+    double *srec = reinterpret_cast<double *>(srec2);
     const int chunk = (int)(gridDim.x >> 3);
     const int pos = (int)(blockIdx.x & 7) * chunk + (int)(blockIdx.x >> 3);
     if (pos >= nsrc) return;
@@ -894,9 +908,9 @@ __global__ __launch_bounds__(64 * kSrcWaves) __attribute__((amdgpu_waves_per_eu(
     if (active && !active[g.sph_susp[S]]) return;
     const int64_t i0 = src_off[S], i1 = src_off[S + 1];
     const int P = g.order[S] + 2;
-    const int nrec = kRecTrac * ((P + 1) * (P + 2) / 2);
+    const int nrec = kRecTracPad * ((P + 1) * (P + 2) / 2);
     const double2 *recS = reinterpret_cast<const double2 *>(rec + g.rec_off[S]);
-    for (int i = threadIdx.x; i < nrec; i += blockDim.x) srec[i] = recS[i];
+    for (int i = threadIdx.x; i < nrec; i += blockDim.x) srec2[i] = recS[i];
     __syncthreads();
     const int lane = threadIdx.x & 63;
     const double *q = g.quat + 4 * S;
@@ -967,7 +981,7 @@ void launch_sheval_items(const DevGeom &g, int mode, const double *rec, const Ev
             const int a = by_src->order_off[p], n = by_src->order_off[p + 1] - a;
             if (n <= 0) continue;
             const int P = p + 2;
-            const size_t lds = sizeof(double2) * (kRecTrac * ((P + 1) * (P + 2) / 2) + kSrcBatch);
+            const size_t lds = sizeof(double2) * kRecTracPad * ((P + 1) * (P + 2) / 2 + 1);
             static size_t lds_set = 0;
             if (lds > 65536 && lds > lds_set) {
                 if (hipFuncSetAttribute((const void *)k_sheval_src, hipFuncAttributeMaxDynamicSharedMemorySize,

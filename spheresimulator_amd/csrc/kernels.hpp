@@ -29,7 +29,7 @@ struct DevGeom {
     const int *sph_susp = nullptr; // N
     const int64_t *pt_off = nullptr;   // N+1
     const int64_t *coef_off = nullptr; // N+1 (6Q doubles per sphere)
-    const int64_t *rec_off = nullptr;  // N+1 (2*kRecTrac*tri(p+2) doubles per sphere with near neighbours)
+    const int64_t *rec_off = nullptr;  // N+1 (2*kRecTracPad*tri(p+2) doubles per sphere with near neighbours)
     const double *coords = nullptr;    // 3P lab
     const double *norms = nullptr;     // 3P lab
     const double *w = nullptr;         // P
