@@ -297,6 +297,7 @@ class Operator {
     // that of M^-1 - 2 I (precondition); laid out on first use
     enum SurfaceOp { kSurfTrac, kSurfSL, kSurfValue, kSurfInverse, kNumSurf };
     const ShGemm &surface(SurfaceOp k);
+    void self_terms(int kind, double cSL, double cTrac, const int *active, hipStream_t s);
     void near_terms(int kind, double cSL, double cTrac, const int *active, hipStream_t s);
     void far_slots(FarLists &L, int kind, int prec, const void *src, const double *tcoords, const double *tnorms,
                    const float *trg32, double coef, const int *active);
@@ -335,7 +336,7 @@ class Operator {
     int flags_;
     int max_order_ = 0;
     hipStream_t stream_ = nullptr, aux_ = nullptr;
-    hipEvent_t ev_fork_ = nullptr, ev_join_ = nullptr;
+    hipEvent_t ev_fork_ = nullptr, ev_join_ = nullptr, ev_coef_ = nullptr;
     int device_ = 0;
 
     std::vector<double> pos_, rad_, quat_;
