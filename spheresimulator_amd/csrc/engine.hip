@@ -374,14 +374,31 @@ Operator::Operator(int nsusp, const int *counts, const double *pos, const double
     ls64_.fp64 = true;
     // coarse FP32 operator of the mixed form's preconditioning solves: orders
     // 5, 4, 3, 2 from 2, 3, 5, 8 (R_s + R_t) (capped at p), source cells of 32
-    // equivalent point forces from 2.5 cell radii (on the check sphere)
-    lsc_.alo[0] = 2.0, lsc_.alo[1] = 3.0, lsc_.alo[2] = 5.0, lsc_.alo[3] = 8.0;
-    lsc_.order[0] = 5, lsc_.order[1] = 4, lsc_.order[2] = 3, lsc_.order[3] = 2;
+    // equivalent point forces from 2.5 cell radii (on the check sphere).  Spheres
+    // of order above 10 also meet their nearest far neighbours, from 1.5, on a
+    // grid of order 10 (170 points; order 12 has 338) instead of their own: that
+    // shell is half of the set's pair evaluations (1500 spheres p=12 in chains:
+    // 1.79e9 -> 0.95e9).  Its truncation (2^-11 at 1.5) is below order 5's at 2,
+    // and order 5 then starts a little later, so that the set's error does not grow.
+    if (nsph_ > 0 && *std::max_element(order_.begin(), order_.end()) > 10) {
+        lsc_.nlev = 5;
+        const double a[5] = {1.5, 2.05, 3.0, 5.0, 8.0};
+        const int q[5] = {10, 5, 4, 3, 2};
+        std::copy(a, a + 5, lsc_.alo);
+        std::copy(q, q + 5, lsc_.order);
+    } else {
+        const double a[4] = {2.0, 3.0, 5.0, 8.0};
+        const int q[4] = {5, 4, 3, 2};
+        std::copy(a, a + 4, lsc_.alo);
+        std::copy(q, q + 4, lsc_.order);
+    }
     lsc_.fp64 = false;
     lsc_.cells = ls32_.cells;
     lsc_.cell_theta = 2.5;
     lsc_.equiv_k = 32;
     if (const char *v = std::getenv("SPHSTK_COARSE_ALPHA")) {
+        lsc_.nlev = 4;
+        for (int l = 0; l < 4; l++) lsc_.order[l] = 5 - l;
         const int got = std::sscanf(v, "%lf,%lf,%lf,%lf:%d,%d,%d,%d", &lsc_.alo[0], &lsc_.alo[1], &lsc_.alo[2],
                                     &lsc_.alo[3], &lsc_.order[0], &lsc_.order[1], &lsc_.order[2], &lsc_.order[3]);
         if (got != 4 && got != 8) throw Error(-1, "SPHSTK_COARSE_ALPHA: a0,a1,a2,a3[:p0,p1,p2,p3]");
@@ -395,7 +412,7 @@ Operator::Operator(int nsusp, const int *counts, const double *pos, const double
     }
     for (const LevelSet *S : {&ls32_, &ls64_, &lsc_}) {
         SPHSTK_REQUIRE(S->alo[0] >= 1.5, "level separations must start at >= 1.5");
-        SPHSTK_REQUIRE(S->nlev >= 1 && S->nlev <= kMaxLevels && (!S->cells || S->nlev == kNumLevels),
+        SPHSTK_REQUIRE(S->nlev >= 1 && S->nlev <= kMaxLevels && (!S->cells || S->nlev >= 2),
                        "internal: level count");
         for (int l = 1; l < S->nlev; l++)
             SPHSTK_REQUIRE(S->alo[l] > S->alo[l - 1], "level separations must increase");

@@ -162,7 +162,7 @@ struct CellAgg {
 // in one array of sources and one of targets, so that all lists of the set are
 // one launch (64 points of a level are a few spheres: on their own, the lists of
 // 100 to 1000 spheres each left most of the GPU idle).
-constexpr int kNumLevels = 4; // levels of the FP32 sets (source cells on their last two)
+constexpr int kNumLevels = 4; // levels of the FP32 inner set (source cells on a set's last two)
 struct LevelSet {
     int nlev = kNumLevels;   // levels in use
     int first_level = 0;     // levels dropped before them (drop_fine_levels)
