@@ -137,16 +137,17 @@ int sphstk_operator_apply_inner(sphstk_operator *op, const double *X, double *Y,
 /* The FP64 outer operator of the mixed-precision solve (its right-hand side and
  * refinement residuals), Y := beta Y + alpha A64ml X (one column).  No
  * counterpart in the reference (whose far field is an FMM to a set tolerance):
- * FP64 pair sums with sphere pairs farther apart than 7 (R_s + R_t)
- * interacting through coarser grids of order min(p, 8), min(p, 6), min(p, 5)
- * and min(p, 4) from 7, 14, 28 and 56 (R_s + R_t) on; self and near terms as
- * A64; relative error about 1e-9 against A64. */
+ * FP64 pair sums with sphere pairs farther apart than 4.8 (R_s + R_t)
+ * interacting through coarser grids of order 10, 9, 8, 7, 6 and 5 (capped at p)
+ * from 4.8, 5.8, 7.35, 10.05, 15.1 and 26 (R_s + R_t) on (farther for unequal
+ * radii); self and near terms as A64; relative error about 1e-9 against A64. */
 int sphstk_operator_apply_outer(sphstk_operator *op, const double *X, double *Y, double alpha, double beta);
 
 /* The coarse FP32 operator of the mixed-precision solve's inner solves (their
  * refinement steps run GMRES on it), Y := beta Y + alpha Ac X (one column).  No
  * counterpart in the reference: as the FP32 inner operator, with coarse grids of
- * order 5, 4, 3 and 2 (capped at p) from 2, 3, 5 and 8 (R_s + R_t) on
+ * order 5, 4, 3 and 2 (capped at p) from about 2, 3, 5 and 8 (R_s + R_t) on, and
+ * of order 10 from 1.5 when some sphere's order is above that
  * (SPHSTK_COARSE_ALPHA); relative error about 1e-2 against A64; unless
  * SPHSTK_FLAG_FP32_DIRECT was given at creation, in which case it is A32. */
 int sphstk_operator_apply_coarse(sphstk_operator *op, const double *X, double *Y, double alpha, double beta);

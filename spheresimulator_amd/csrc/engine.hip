@@ -373,21 +373,25 @@ Operator::Operator(int nsusp, const int *counts, const double *pos, const double
     }
     ls64_.fp64 = true;
     // coarse FP32 operator of the mixed form's preconditioning solves: orders
-    // 5, 4, 3, 2 from 2, 3, 5, 8 (R_s + R_t) (capped at p), source cells of 32
+    // 5, 4, 3, 2 from about 2, 3, 5, 8 (R_s + R_t) (capped at p), source cells of 32
     // equivalent point forces from 2.5 cell radii (on the check sphere).  Spheres
     // of order above 10 also meet their nearest far neighbours, from 1.5, on a
     // grid of order 10 (170 points; order 12 has 338) instead of their own: that
     // shell is half of the set's pair evaluations (1500 spheres p=12 in chains:
     // 1.79e9 -> 0.95e9).  Its truncation (2^-11 at 1.5) is below order 5's at 2,
     // and order 5 then starts a little later, so that the set's error does not grow.
+    // Without that level the separations lie a little beyond 2, 3, 5, 8: the
+    // octahedral grids' interpolation adds 0.5 % to the error that Gauss-Legendre
+    // grids had from there, and this takes it off again (256 spheres p=8: 9.23e-4 ->
+    // 8.98e-4 for 1 % more pair evaluations).
     if (nsph_ > 0 && *std::max_element(order_.begin(), order_.end()) > 10) {
         lsc_.nlev = 5;
-        const double a[5] = {1.5, 2.05, 3.0, 5.0, 8.0};
+        const double a[5] = {1.5, 2.05, 3.01, 5.01, 8.02};
         const int q[5] = {10, 5, 4, 3, 2};
         std::copy(a, a + 5, lsc_.alo);
         std::copy(q, q + 5, lsc_.order);
     } else {
-        const double a[4] = {2.0, 3.0, 5.0, 8.0};
+        const double a[4] = {2.01, 3.01, 5.01, 8.02};
         const int q[4] = {5, 4, 3, 2};
         std::copy(a, a + 4, lsc_.alo);
         std::copy(q, q + 4, lsc_.order);
