@@ -262,13 +262,13 @@ def main():
     both = {"ms": stc["ms"] + st32["ms"], "launches": stc["launches"] + st32["launches"],
             "pairs": (stc["pairs"] * stc["launches"] + st32["pairs"] * st32["launches"]) /
                      max(1, stc["launches"] + st32["launches"])}
-    f32 = far_roofline(both, FP32_VALU_PEAK, "k_far_f32<traction>: all FP32 pair-sum launches of a solve (coarse "
-                       "operator: mid range, 4 levels, 2 cell lists per apply; FP32 operator: likewise)", 7)
+    f32 = far_roofline(both, FP32_VALU_PEAK, "k_far_f32<traction>: all FP32 pair-sum launches of a solve (one per "
+                       "apply of either operator: mid range, levels and cell lists together)", 1)
     if f32 is not None:
-        f32["coarse"] = far_roofline(stc, FP32_VALU_PEAK, "k_far_f32<traction>, coarse operator", 7)
-        f32["inner"] = far_roofline(st32, FP32_VALU_PEAK, "k_far_f32<traction>, FP32 operator", 7)
+        f32["coarse"] = far_roofline(stc, FP32_VALU_PEAK, "k_far_f32<traction>, coarse operator", 1)
+        f32["inner"] = far_roofline(st32, FP32_VALU_PEAK, "k_far_f32<traction>, FP32 operator", 1)
     f64 = far_roofline(st64ml, FP64_VALU_PEAK, "k_far_f64_lvl<traction>: the mid-range list and 6 level lists of "
-                       "one FP64 residual apply", 7)
+                       "one FP64 residual apply in one launch", 1)
     out["roofline"], other = dominant(f32, f64, both, st64ml, cnt["steps"])
     if other is not None:
         out["mixed"]["fp32_far" if other is f32 else "fp64_outer_far"] = other
