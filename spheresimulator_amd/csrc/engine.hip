@@ -36,6 +36,7 @@ constexpr int64_t kWantItems = 40000; // far-field work items wanted when a prob
 // 32; a solve 7.31, 6.79 and 6.84 ms; 100 spheres mixed 9.37, 9.19 and 9.50 ms.
 constexpr int64_t kMaxSlices = 16;
 constexpr int64_t kMultiItems = 8192; // the same for several right-hand sides on one geometry
+constexpr size_t kJoinIntervals = 65536; // host work lists: intervals up to which parts are joined for one upload
 constexpr int kSumsInBlock = 1024; // GMRES: most chunk partials of a segment that every block adds up itself
 constexpr int64_t kLookaheadDof = 300000; // GMRES below this many unknowns launches one iteration ahead
 constexpr double kTuneBudget = 3.0;    // seconds per autotuning pass (SPHSTK_FLAG_AUTOTUNE)
@@ -637,6 +638,11 @@ Runs runs_of(const std::vector<int> &lst, int s0, int s1, bool include) {
     return r;
 }
 
+template <typename T>
+static void put(DevBuf<T> &d, int64_t at, const std::vector<T> &v) {
+    if (!v.empty()) SPHSTK_HIP(hipMemcpy(d.p + at, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
+}
+
 // Runs a parallel loop over [0, n) on the host's cores (at most 16 threads),
 // handing out `chunk` indices at a time (0: automatic); serial below `serial_below`.
 static void parallel_for(int n, const std::function<void(int, int)> &body, int chunk = 0, int serial_below = 256) {
@@ -847,13 +853,17 @@ int append_far_lists(HostLists &H, int nsusp, const std::vector<int64_t> &susp_s
     if (pairs == 0.0) return 0;
     H.pairs += pairs;
     for (Part &P : parts) {
-        const int64_t base = (int64_t)H.ivs.size();
+        const int64_t base = H.niv;
         for (FarGroup &g : P.groups) {
             g.iv_begin += base;
             g.iv_end += base;
         }
         H.groups.insert(H.groups.end(), P.groups.begin(), P.groups.end());
-        H.ivs.insert(H.ivs.end(), P.ivs.begin(), P.ivs.end());
+        H.niv += (int64_t)P.ivs.size();
+        if (!H.iv_parts.empty() && H.iv_parts.back().size() + P.ivs.size() <= kJoinIntervals)
+            H.iv_parts.back().insert(H.iv_parts.back().end(), P.ivs.begin(), P.ivs.end());
+        else
+            H.iv_parts.push_back(std::move(P.ivs));
         H.work.insert(H.work.end(), P.work.begin(), P.work.end());
         std::vector<FarInterval>().swap(P.ivs);
     }
@@ -881,7 +891,13 @@ void upload_far_lists(FarLists &L, HostLists &H, int tpl, int split, int64_t ntr
     L.ngroups = (int)H.groups.size();
     L.pairs = H.pairs;
     L.groups.upload(H.groups);
-    L.iv.upload(H.ivs);
+    L.iv.alloc(H.niv);
+    int64_t at = 0;
+    for (std::vector<FarInterval> &v : H.iv_parts) {
+        put(L.iv, at, v);
+        at += (int64_t)v.size();
+        std::vector<FarInterval>().swap(v);
+    }
     L.order.upload(ord);
     L.slots();
 }
@@ -959,11 +975,6 @@ void kd_order(const double *pos, int *idx, int b, int e, int leaf) {
     kd_order(pos, idx, b + h, e, leaf);
 }
 } // namespace
-
-template <typename T>
-static void put(DevBuf<T> &d, int64_t at, const std::vector<T> &v) {
-    if (!v.empty()) SPHSTK_HIP(hipMemcpy(d.p + at, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
-}
 
 void Operator::ensure_levels(LevelSet &S) {
     if (S.ready) return;
