@@ -65,3 +65,16 @@ def test_multi_level_operators_at_tile_edges(n, orders):
     assert rel(op.apply_outer(x), y) < 2e-9
     assert rel(op.apply_inner(x), y) < 5e-5
     assert rel(op.apply_coarse(x), y) < 5e-2
+
+
+@pytest.mark.parametrize("n,orders", [(17, (11,)), (18, (10, 11)), (20, (16, 12, 8)), (5, (20,))])
+def test_coarse_operator_with_next_neighbours_on_a_level(n, orders):
+    """Neighbours between 1.5 and 2 (R_s + R_t), which orders above 10 sum on a
+    level of order 10: its truncation there is at most 2^-11, order 5's behind it
+    1.1e-3; ten times the larger for the handful of degrees at the cut."""
+    pos, rad, quat = line(n, 1.5, n + 200)
+    order = np.resize(np.array(orders, dtype=np.int32), n)
+    op = S.SphereSTKSHOperator(pos, rad, quat, order, 0.5, 0.0, 1.0, 1.0)
+    x = np.random.default_rng(n).standard_normal(op.n_dof)
+    op.projectNullSpace(x)
+    assert rel(op.apply_coarse(x), op.apply(x)) < 1.1e-2
