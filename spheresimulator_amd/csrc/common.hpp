@@ -95,7 +95,8 @@ struct Resample {
     std::vector<double> down, up;
 };
 const Resample &resample_tables(int p, int pc);
-// The same to and from the level grid of degree pc <= p (no identity at pc == p).
+// The same to and from the level grid of degree pc <= p (no identity at pc == p); up, for
+// p > pc, also carries what the level grid shows of degree pc + 1.
 const Resample &level_resample(int p, int pc);
 void gauss_legendre(int n, std::vector<double> &x, std::vector<double> &w);
 
