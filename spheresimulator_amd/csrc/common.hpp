@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstdint>
 #include <stdexcept>
 #include <string>
@@ -98,6 +99,28 @@ const Resample &resample_tables(int p, int pc);
 // The same to and from the level grid of degree pc <= p (no identity at pc == p); up, for
 // p > pc, also carries what the level grid shows of degree pc + 1.
 const Resample &level_resample(int p, int pc);
+// Pairs that the final velocities and the right-hand side treat at sphere
+// centres instead of grid points:
+// * the rigid-body averages of u = S[rho] (V = mean u / mu, Omega = 3/(8 pi R^4
+//   mu) sum w R n x u) through Faxen's laws, the exact surface averages, which
+//   the target grid's quadrature of order p reproduces to C q^(2p+2),
+//   q = R_t / (d - R_s);
+// * the traction of a rigid-body density in closed form, which the source
+//   grid's quadrature reproduces to C q^(2p+2), q = R_s / (d - R_t).
+// C is 10 to 500 for the traction (most at small q), up to 50 for the averages.
+// Beyond kFaxenSep (R_s + R_t) all pairs (traction, equal radii: 7e-10 at p = 6,
+// 4e-13 at p = 8; radii 1:3, p = 6: 4e-8), closer ones where the powers of both
+// spheres are below kFaxenTol, so that closed form and grid sum differ by less
+// than the 5e-15 to which the sum over a grid is rounded: equal radii from 3.46
+// (R_s + R_t) at p = 10, 2.75 at p = 12, 2.08 at p = 16.
+constexpr double kFaxenSep = 4.0;
+constexpr double kFaxenTol = 1e-17;
+inline bool centre_pair(double d, double rs, int ps, double rt, int pt) {
+    if (d >= kFaxenSep * (rs + rt)) return true;
+    const double qs = rs / (d - rt), qt = rt / (d - rs);
+    return std::pow(qs, 2 * ps + 2) <= kFaxenTol && std::pow(qt, 2 * pt + 2) <= kFaxenTol;
+}
+
 void gauss_legendre(int n, std::vector<double> &x, std::vector<double> &w);
 
 // Equivalent-source template of the far-field cell aggregation (equiv.cpp):

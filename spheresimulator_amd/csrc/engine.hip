@@ -1705,26 +1705,6 @@ std::vector<std::vector<int>> Operator::neighbours_within(double amax) const {
     return nb;
 }
 
-// Pairs that the final velocities and the right-hand side treat at sphere
-// centres instead of grid points:
-// * the rigid-body averages of u = S[rho] (V = mean u / mu, Omega = 3/(8 pi R^4
-//   mu) sum w R n x u) through Faxen's laws, the exact surface averages, which
-//   the target grid's quadrature of order p reproduces to ~q^(2p+2),
-//   q = R_t / (d - R_s);
-// * the traction of a rigid-body density in closed form, which the source
-//   grid's quadrature reproduces to ~q^(2p+2), q = R_s / (d - R_t).
-// Both hold beyond kFaxenSep (R_s + R_t) (below 1.5e-12 for p >= 6 and equal
-// radii), and closer where the spheres' orders keep both powers below the same
-// 1.5e-12: from 1.9 (R_s + R_t) at p = 12, 1.6 at p = 16 (with the fixed distance
-// the pairs in between, 97 spheres around each at volume fraction 0.2, went
-// point by point: 24 ms each way at 3000 spheres p=12, of 677 ms).
-constexpr double kFaxenSep = 4.0;
-constexpr double kFaxenTol = 1.5e-12;
-static bool centre_pair(double d, double rs, int ps, double rt, int pt) {
-    if (d >= kFaxenSep * (rs + rt)) return true;
-    const double qs = rs / (d - rt), qt = rt / (d - rs);
-    return std::pow(qs, 2 * ps + 2) <= kFaxenTol && std::pow(qt, 2 * pt + 2) <= kFaxenTol;
-}
 void Operator::ensure_centre() {
     if (!centre_ready_) {
         PhaseTimer pt("final-velocity lists");
