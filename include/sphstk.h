@@ -138,8 +138,8 @@ int sphstk_operator_apply_inner(sphstk_operator *op, const double *X, double *Y,
  * refinement residuals), Y := beta Y + alpha A64ml X (one column).  No
  * counterpart in the reference (whose far field is an FMM to a set tolerance):
  * FP64 pair sums with sphere pairs farther apart than 4.8 (R_s + R_t)
- * interacting through coarser grids of order 10, 9, 8, 7, 6 and 5 (capped at p)
- * from 4.8, 5.8, 7.35, 10.05, 15.1 and 26 (R_s + R_t) on (farther for unequal
+ * interacting through coarser grids of order 10, 9, 8, 7 and 5 (capped at p)
+ * from 4.8, 5.8, 7.35, 10.05 and 23 (R_s + R_t) on (farther for unequal
  * radii); self and near terms as A64; relative error about 1e-9 against A64. */
 int sphstk_operator_apply_outer(sphstk_operator *op, const double *X, double *Y, double alpha, double beta);
 

@@ -358,19 +358,22 @@ Operator::Operator(int nsusp, const int *counts, const double *pos, const double
 
     int tpl = 1, split = 0;
     // FP32 inner operator: orders from level_order().  FP64 outer applies: fine
-    // below s' = 4.8, then orders 10, 9, 8, 7, 6, 5 from s' = 4.8, 5.8, 7.35,
-    // 10.05, 15.1, 26 (the radius-aware separation of ensure_levels()), where a
-    // level's worst truncation ratio (2 s' - 1)^-(q + 1) is 5.6e-11 to 5.9e-11.
+    // below s' = 4.8, then orders 10, 9, 8, 7, 5 from s' = 4.8, 5.8, 7.35, 10.05, 23
+    // (the radius-aware separation of ensure_levels()), where the error of a pair of
+    // order 12 is 3.7e-10, 7.2e-10, 9.8e-10, 9.4e-10 and 1.9e-9 of a density of size
+    // one (Gauss-Legendre grids of orders 10 to 5 from 4.8, 5.8, 7.35, 10.05, 15.1
+    // and 26: 2.2e-9 to 2.9e-9).  Order 6 has order 7's points, and none of them are
+    // saved between 10.05 and 23 by it.
     ls32_.alo[0] = 3.0, ls32_.alo[1] = 6.0, ls32_.alo[2] = 9.0, ls32_.alo[3] = 16.0;
     ls32_.order[0] = ls32_.order[1] = ls32_.order[2] = ls32_.order[3] = -1;
     ls32_.fp64 = false;
     ls32_.cells = (flags & 32) == 0;
-    ls64_.nlev = 6;
+    ls64_.nlev = 5;
     {
-        const double a[6] = {4.8, 5.8, 7.35, 10.05, 15.1, 26.0};
-        const int q[6] = {10, 9, 8, 7, 6, 5};
-        std::copy(a, a + 6, ls64_.alo);
-        std::copy(q, q + 6, ls64_.order);
+        const double a[5] = {4.8, 5.8, 7.35, 10.05, 23.0};
+        const int q[5] = {10, 9, 8, 7, 5};
+        std::copy(a, a + 5, ls64_.alo);
+        std::copy(q, q + 5, ls64_.order);
     }
     ls64_.fp64 = true;
     // coarse FP32 operator of the mixed form's preconditioning solves: orders

@@ -58,7 +58,7 @@ int main() {
         {10, 6, 3.0, 1.0}, {12, 7, 3.0, 1.0}, {14, 8, 3.0, 1.0},   {16, 9, 3.0, 1.0},   {18, 10, 3.0, 0.4},
         {20, 11, 3.0, 1.0}, {12, 5, 6.0, 1.0}, {16, 6, 6.0, 1.0},  {12, 4, 9.0, 1.0},   {12, 3, 16.0, 1.0},
         {12, 10, 4.8, 1.0}, {12, 9, 5.8, 1.0}, {12, 8, 7.35, 1.0}, {12, 7, 10.05, 1.0}, {12, 6, 15.1, 1.0},
-        {12, 5, 26.0, 1.0}, {12, 10, 1.5, 1.0}, {12, 10, 1.5, 3.0}, {11, 10, 1.5, 1.0}};
+        {12, 5, 23.0, 1.0}, {12, 10, 1.5, 1.0}, {12, 10, 1.5, 3.0}, {11, 10, 1.5, 1.0}};
     int fails = 0;
     for (int q = 1; q <= 12; q++)
         for (double w : level_tables(q).w)
