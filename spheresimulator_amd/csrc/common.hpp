@@ -53,7 +53,7 @@ struct FarGroup {
     int32_t tcount;
     int32_t susp;
     int32_t slot;
-    int32_t list; // of a joint list: which of its lists
+    int32_t set; // of a joint list: which of its target sets
 };
 
 // Number of complex arrays in the per-sphere expansion records.

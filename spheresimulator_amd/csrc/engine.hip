@@ -461,7 +461,8 @@ Operator::Operator(int nsusp, const int *counts, const double *pos, const double
             const int64_t nb = std::max<int64_t>(1, pt_off_[s0] / (64 * kMultiTPL));
             const int slices = (int)std::max<int64_t>(1, std::min<int64_t>(32, (kMultiItems + nb - 1) / nb));
             build_far_lists(lists_fine_, b0, so0, po0, po0, r0, kMultiTPL, slices, kWantItems);
-            if (lists_fine_.pairs > 0.0) lists_fine_.part.alloc(size_t(lists_fine_.split) * 3 * npts_);
+            lists_fine_.map.stride[0] = 3 * npts_; // a slot holds all copies
+            lists_fine_.npart = size_t(lists_fine_.split) * 3 * npts_;
             srcm_.alloc(std::max<int64_t>(4 * (std::min(ncopy_, kMultiCols) + 1) * pt_off_[s0], 8));
         } else {
             build_far_lists(lists_fine_, nsusp_, susp_sph_off_, pt_off_, pt_off_, runs_fine_, tpl, split, kWantItems);
@@ -678,7 +679,7 @@ static void parallel_for(int n, const std::function<void(int, int)> &body, int c
 // point ranges of its spheres' runs, with a per-lane mask where the group
 // spans spheres.  Each group's list is cut into `split` slices of nearly equal
 // length, one work item each, launched in order of decreasing work.
-int append_far_lists(HostLists &H, int nsusp, const std::vector<int64_t> &susp_sph_off, const std::vector<int64_t> &toff,
+void append_far_lists(HostLists &H, int nsusp, const std::vector<int64_t> &susp_sph_off, const std::vector<int64_t> &toff,
                      const std::vector<int64_t> &soff, const std::vector<Runs> &runs, int tpl, int split,
                      int64_t want_items, const std::vector<int64_t> *src_susp_off, ListBase at) {
     const std::vector<int64_t> &sso = src_susp_off ? *src_susp_off : susp_sph_off;
@@ -686,7 +687,9 @@ int append_far_lists(HostLists &H, int nsusp, const std::vector<int64_t> &susp_s
     SPHSTK_REQUIRE(split >= 0 && split <= 64, "source split must be in [0, 64] (0 = automatic)");
     const int nsph = (int)toff.size() - 1;
     SPHSTK_REQUIRE((int)runs.size() == nsph, "internal: one run list per target sphere");
-    const int64_t ntrg = toff[nsph];
+    const int64_t ntrg = toff[nsph], trg0 = H.sets[at.set].first;
+    const int slot0 = H.sets[at.set].nslot;
+    SPHSTK_REQUIRE(H.sets[at.set].n == ntrg, "internal: targets of a joint list");
     std::vector<int32_t> tsph(ntrg);
     for (int i = 0; i < nsph; i++)
         for (int64_t k = toff[i]; k < toff[i + 1]; k++) tsph[k] = i;
@@ -741,8 +744,8 @@ int append_far_lists(HostLists &H, int nsusp, const std::vector<int64_t> &susp_s
             const int cnt = gs[gi].cnt, b = gs[gi].b;
             if (tsph[t0] == tsph[t0 + cnt - 1] && tsph[t0] == last_T) {
                 for (int sl = 0; sl < split; sl++) {
-                    P.groups.push_back(FarGroup{t0 + at.trg, last_slots[sl][0], last_slots[sl][1], cnt, b, at.slot + sl,
-                                                H.nlist});
+                    P.groups.push_back(FarGroup{t0 + trg0, last_slots[sl][0], last_slots[sl][1], cnt, b, slot0 + sl,
+                                                at.set});
                     P.work.push_back(last_slots[sl][2]);
                 }
                 P.pairs += double(last_work) * cnt;
@@ -815,7 +818,7 @@ int append_far_lists(HostLists &H, int nsusp, const std::vector<int64_t> &susp_s
             int64_t iv_pos = giv.empty() ? 0 : giv[0].begin;
             for (int sl = 0; sl < split; sl++) {
                 const int64_t quota = gwork * (sl + 1) / split - gwork * sl / split;
-                FarGroup g{t0 + at.trg, (int64_t)P.ivs.size(), 0, cnt, b, at.slot + sl, H.nlist};
+                FarGroup g{t0 + trg0, (int64_t)P.ivs.size(), 0, cnt, b, slot0 + sl, at.set};
                 int64_t left = quota;
                 while (left > 0 && iv_i < giv.size()) {
                     const int64_t take = std::min(giv[iv_i].end - iv_pos, left);
@@ -853,7 +856,7 @@ int append_far_lists(HostLists &H, int nsusp, const std::vector<int64_t> &susp_s
         ni += P.ivs.size();
     }
     if (setup_verbose()) std::fprintf(stderr, "[sphstk]     %zu work items, %zu intervals, %.4g pairs\n", ng, ni, pairs);
-    if (pairs == 0.0) return 0;
+    if (pairs == 0.0) return;
     H.pairs += pairs;
     for (Part &P : parts) {
         const int64_t base = H.niv;
@@ -870,27 +873,34 @@ int append_far_lists(HostLists &H, int nsusp, const std::vector<int64_t> &susp_s
         H.work.insert(H.work.end(), P.work.begin(), P.work.end());
         std::vector<FarInterval>().swap(P.ivs);
     }
-    H.nlist++;
-    return split;
+    H.sets[at.set].nslot += split;
 }
 
 // Launch order: by work, in classes of a factor of two, so that no long item
-// starts last; within a class list by list and slice by slice, in the order of
+// starts last; within a class by target sets and slice by slice, in the order of
 // the targets, so that the items in flight read one part of one list's sources
 // (measured against the strict order by work: within 1%).
-void upload_far_lists(FarLists &L, HostLists &H, int tpl, int split, int64_t ntrg) {
+void upload_far_lists(FarLists &L, HostLists &H, int tpl) {
     std::vector<int> ord(H.groups.size());
     std::vector<uint64_t> key(H.groups.size());
     std::iota(ord.begin(), ord.end(), 0);
     for (size_t i = 0; i < ord.size(); i++) {
         int cls = 0;
         while (cls < 63 && (H.work[i] >> cls) != 0) cls++;
-        key[i] = uint64_t(63 - cls) << 32 | uint64_t(H.groups[i].list) << 16 | uint64_t(H.groups[i].slot);
+        key[i] = uint64_t(63 - cls) << 32 | uint64_t(H.groups[i].set) << 16 | uint64_t(H.groups[i].slot);
     }
     std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return key[a] < key[b]; });
     L.tpl = tpl;
-    L.split = split;
-    L.ntrg = ntrg;
+    L.split = std::max(H.sets[0].nslot, 1);
+    L.ntrg = H.sets[0].n;
+    L.npart = 0;
+    for (size_t k = 0; k < H.sets.size(); k++) {
+        // each set has the slots that its own lists need: the coarse levels, with few
+        // targets, are cut into many slices, the fine grid, with most, into few
+        L.map.stride[k] = 3 * H.sets[k].n;
+        L.map.base[k] = (int64_t)L.npart - 3 * H.sets[k].first;
+        L.npart += size_t(H.sets[k].nslot) * 3 * H.sets[k].n;
+    }
     L.ngroups = (int)H.groups.size();
     L.pairs = H.pairs;
     L.groups.upload(H.groups);
@@ -902,15 +912,15 @@ void upload_far_lists(FarLists &L, HostLists &H, int tpl, int split, int64_t ntr
         std::vector<FarInterval>().swap(v);
     }
     L.order.upload(ord);
-    L.slots();
 }
 
 void build_far_lists(FarLists &L, int nsusp, const std::vector<int64_t> &susp_sph_off,
                      const std::vector<int64_t> &toff, const std::vector<int64_t> &soff, const std::vector<Runs> &runs,
                      int tpl, int split, int64_t want_items, const std::vector<int64_t> *src_susp_off) {
     HostLists H;
-    const int n = append_far_lists(H, nsusp, susp_sph_off, toff, soff, runs, tpl, split, want_items, src_susp_off);
-    upload_far_lists(L, H, tpl, std::max(n, 1), toff.back());
+    H.sets.push_back({0, toff.back(), 0});
+    append_far_lists(H, nsusp, susp_sph_off, toff, soff, runs, tpl, split, want_items, src_susp_off);
+    upload_far_lists(L, H, tpl);
 }
 
 static std::vector<Chunk> make_chunks(int nsusp, const std::vector<int64_t> &susp_sph_off,
@@ -1191,13 +1201,14 @@ void Operator::ensure_levels(LevelSet &S) {
     }
     const int64_t ntrg = lbase[nlev];
     HostLists H;
-    std::vector<int> nslot(nlev);
+    H.sets.push_back({0, npts_, 0});
+    for (int l = 0; l < nlev; l++) H.sets.push_back({lbase[l], lbase[l + 1] - lbase[l], 0});
     {
         PhaseTimer pm("  mid-range and level lists");
-        S.mid_slots = append_far_lists(H, nsusp_, susp_sph_off_, pt_off_, pt_off_, mid, S.tpl, 0, kWantItems);
+        append_far_lists(H, nsusp_, susp_sph_off_, pt_off_, pt_off_, mid, S.tpl, 0, kWantItems);
         for (int l = 0; l < nlev; l++)
-            nslot[l] = append_far_lists(H, nsusp_, susp_sph_off_, level_off[l], level_off[l], lvl[l], S.tpl, 0,
-                                        kWantItems, nullptr, ListBase{lbase[l], lbase[l], 0});
+            append_far_lists(H, nsusp_, susp_sph_off_, level_off[l], level_off[l], lvl[l], S.tpl, 0, kWantItems,
+                             nullptr, ListBase{1 + l, lbase[l]});
     }
     level_transforms(S);
     S.agg.reset();
@@ -1281,18 +1292,19 @@ void Operator::ensure_levels(LevelSet &S) {
         }
         build_far_lists(A->chk_lists, nsusp_, susp_cell_off, chk_off, pt_off_, chk_runs, 1, 0, kWantItems,
                         &susp_sph_off_);
-        A->check_pairs = A->chk_lists.pairs;
+        A->chk_lists.slots();
         for (int i = 0; i < 2; i++) {
             std::vector<Runs> runs(nsph_);
             for (int r = 0; r < nsph_; r++) runs[r] = crun[r][i];
             const int l = c0 + i;
-            nslot[l] += append_far_lists(H, nsusp_, susp_sph_off_, level_off[l], eq_off, runs, S.tpl, 0, kWantItems,
-                                         &susp_cell_off, ListBase{lbase[l], ntrg, nslot[l]});
+            append_far_lists(H, nsusp_, susp_sph_off_, level_off[l], eq_off, runs, S.tpl, 0, kWantItems, &susp_cell_off,
+                             ListBase{1 + l, ntrg});
         }
         S.agg = std::move(A);
     }
-    upload_far_lists(S.all, H, S.tpl, std::max(S.mid_slots, nslot.empty() ? 0 : *std::max_element(nslot.begin(), nslot.end())),
-                     ntrg);
+    upload_far_lists(S.all, H, S.tpl);
+    S.all.slots();
+    S.mid_slots = H.sets[0].nslot;
     // records: positions now, force words per apply
     // (set-up of a set may run on a host thread of its own: nothing here goes to
     // the operator's stream, which may be capturing)
@@ -1332,13 +1344,13 @@ void Operator::ensure_levels(LevelSet &S) {
     SPHSTK_HIP(hipGetLastError());
     SPHSTK_HIP(hipStreamSynchronize(st0));
     LevelViews &V = S.views;
-    V.stride = 3 * ntrg;
     for (int l = 0; l < nlev; l++) {
         V.off[l] = S.levels[l]->d_off_by_sph.p;
         V.w[l] = S.levels[l]->w.p;
         V.src[l] = S.fp64 ? (void *)(S.src64.p + 8 * lbase[l]) : (void *)(S.src32.p + 8 * lbase[l]);
-        V.part[l] = S.all.part.p ? S.all.part.p + 3 * lbase[l] : nullptr;
-        V.nslot[l] = nslot[l];
+        V.part[l] = S.all.part.p ? S.all.part.p + S.all.map.base[1 + l] + 3 * lbase[l] : nullptr;
+        V.nslot[l] = H.sets[1 + l].nslot;
+        V.stride[l] = S.all.map.stride[1 + l];
     }
     S.ready = true;
 }
@@ -1450,9 +1462,10 @@ void Operator::far_run(FarLists &L, int kind, int prec, const void *src, const d
                        const double *tnorms, const float *trg32, const Chunk *chunks, int nchunks, double coef,
                        double *out, const int *active) {
     if (L.pairs == 0.0) return; // e.g. a level that no sphere pair reaches
+    if (L.split > 1) L.slots();
     double *dst = L.split > 1 ? L.part.p : out;
     const int acc = L.split > 1 ? 0 : 1;
-    launch_far(kind, prec, L.tpl, src, tcoords, tnorms, trg32, L.ntrg, L.ngroups, L.order.p, L.groups.p, L.iv.p,
+    launch_far(kind, prec, L.tpl, src, tcoords, tnorms, trg32, L.map, L.ngroups, L.order.p, L.groups.p, L.iv.p,
                active, dst, coef, acc, stream_, &L != &lists_fine_);
     if (L.split > 1) launch_slot_reduce(out, L.part.p, L.split, 3 * L.ntrg, chunks, nchunks, active, stream_);
 }
@@ -1461,7 +1474,8 @@ void Operator::far_run(FarLists &L, int kind, int prec, const void *src, const d
 void Operator::far_slots(FarLists &L, int kind, int prec, const void *src, const double *tcoords, const double *tnorms,
                          const float *trg32, double coef, const int *active) {
     if (L.pairs == 0.0) return; // e.g. a level that no sphere pair reaches
-    launch_far(kind, prec, L.tpl, src, tcoords, tnorms, trg32, L.ntrg, L.ngroups, L.order.p, L.groups.p, L.iv.p,
+    L.slots();
+    launch_far(kind, prec, L.tpl, src, tcoords, tnorms, trg32, L.map, L.ngroups, L.order.p, L.groups.p, L.iv.p,
                active, L.part.p, coef, 0, stream_, &L != &lists_fine_);
 }
 
@@ -1506,6 +1520,7 @@ void Operator::far_copies(int kind, double coef, const double *in, const int *ac
     const int64_t n0 = npts_ / ncopy_, col = 3 * n0;
     if (ev_a) SPHSTK_HIP(hipEventRecord(ev_a, stream_));
     if (L.pairs == 0.0) return;
+    L.slots();
     if (kind == 0) {
         for (int c0 = 0; c0 < ncopy_; c0 += kMultiCols) {
             const int nc = std::min(kMultiCols, ncopy_ - c0);
@@ -1518,7 +1533,7 @@ void Operator::far_copies(int kind, double coef, const double *in, const int *ac
     for (int c = 0; c < ncopy_; c++) {
         const int *act = active ? active + c * b0 : nullptr;
         launch_pack_src_f64(n0, d_coords_.p, d_w_.p, in + c * col, src64_.p, stream_);
-        launch_far(kind, 0, L.tpl, src64_.p, d_coords_.p, d_norms_.p, nullptr, npts_, L.ngroups, L.order.p,
+        launch_far(kind, 0, L.tpl, src64_.p, d_coords_.p, d_norms_.p, nullptr, L.map, L.ngroups, L.order.p,
                    L.groups.p, L.iv.p, act, L.part.p + c * col, coef, 0, stream_);
     }
 }
@@ -1618,7 +1633,7 @@ FarSum Operator::far(LevelSet *S, int kind, int prec, double coef, const double 
         pending_.push_back(ev);
         if (pending_.size() > 64) harvest_events();
     }
-    return S ? FarSum{S->all.part.p, S->mid_slots, 3 * S->all.ntrg} : FarSum{L.part.p, L.nslot(), 3 * npts_};
+    return S ? FarSum{S->all.part.p, S->mid_slots, 3 * npts_} : FarSum{L.part.p, L.nslot(), 3 * npts_};
 }
 
 // applyP2POP (cpp:262-485), accumulating into out (or, overwrite, the whole

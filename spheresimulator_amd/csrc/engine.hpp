@@ -73,13 +73,15 @@ struct FarLists {
     DevBuf<FarGroup> groups;
     DevBuf<FarInterval> iv;
     DevBuf<int> order;
-    DevBuf<double> part; // split partial-sum slots of 3*ntrg doubles
+    DevBuf<double> part; // partial-sum slots
+    SlotMap map;         // where they lie in it
+    size_t npart = 0;    // their size
     int ngroups = 0, tpl = 1, split = 1;
     double pairs = 0.0; // algorithmic pairs per launch
     int64_t ntrg = 0;
-    // the slots as the consumers of the sum read them (a list without pairs has none)
+    // allocates the slots, of the lists whose sums go there (without pairs there are none)
     void slots() {
-        if (pairs > 0.0) part.alloc(size_t(split) * 3 * ntrg);
+        if (pairs > 0.0) part.alloc(npart);
     }
     int nslot() const { return pairs > 0.0 ? split : 0; }
 };
@@ -104,22 +106,27 @@ struct HostLists {
     int64_t niv = 0;
     std::vector<int64_t> work;
     double pairs = 0.0;
-    int nlist = 0;
+    // the target sets: first target, number of targets, slots of the lists so far
+    struct Targets {
+        int64_t first = 0, n = 0;
+        int nslot = 0;
+    };
+    std::vector<Targets> sets;
 };
-// Where a list's points and slots lie in the point sets and slots of a joint
-// list: its targets from target trg on, its sources from source src on, its
-// first slot.
+// Where a list's points lie in those of a joint list: its target set, and its
+// sources from source src on.
 struct ListBase {
-    int64_t trg = 0, src = 0;
-    int slot = 0;
+    int set = 0;
+    int64_t src = 0;
 };
-// Appends a list's work items; returns its slots (0: it has no pairs).
+// Appends a list's work items, with slots of its own behind those of its target
+// set's lists before it (none if it has no pairs).
 // src_susp_off: first source "sphere" (entry of soff) of each suspension when
 // the source point set is not the target's sphere set (NULL: susp_sph_off).
-int append_far_lists(HostLists &H, int nsusp, const std::vector<int64_t> &susp_sph_off, const std::vector<int64_t> &toff,
+void append_far_lists(HostLists &H, int nsusp, const std::vector<int64_t> &susp_sph_off, const std::vector<int64_t> &toff,
                      const std::vector<int64_t> &soff, const std::vector<Runs> &runs, int tpl, int split,
                      int64_t want_items, const std::vector<int64_t> *src_susp_off = nullptr, ListBase at = ListBase{});
-void upload_far_lists(FarLists &L, HostLists &H, int tpl, int split, int64_t ntrg);
+void upload_far_lists(FarLists &L, HostLists &H, int tpl);
 void build_far_lists(FarLists &L, int nsusp, const std::vector<int64_t> &susp_sph_off,
                      const std::vector<int64_t> &toff, const std::vector<int64_t> &soff, const std::vector<Runs> &runs,
                      int tpl, int split, int64_t want_items, const std::vector<int64_t> *src_susp_off = nullptr);
@@ -149,7 +156,6 @@ constexpr double kCellTheta = 4.0;
 struct CellAgg {
     int ncell = 0;
     const EquivTables *E = nullptr;   // the set's equivalent-source template
-    double check_pairs = 0.0;         // pair evaluations of the check velocities (per apply)
     std::vector<int64_t> susp_cell_off; // first cell of each suspension
     DevBuf<float> chk32;              // check points as FP32 target records (zero normals)
     float *eq32 = nullptr;            // equivalent points among the set's source records (forces per apply)

@@ -249,13 +249,13 @@ __device__ __forceinline__ void far_range(const R *__restrict__ src, int64_t b, 
     }
 }
 
-// accumulate != 0: out += coef*acc.  accumulate == 0: out[slot*slot_stride + ...] = coef*acc
+// accumulate != 0: out += coef*acc.  accumulate == 0: the sums go to the group's slot
 // (one partial-sum slot per source slice, reduced afterwards in slot order).
 template <int TPL>
 __device__ __forceinline__ void store_far(const FarGroup &G, int lane, const double *ax, const double *ay,
                                           const double *az, double *__restrict__ out, double coef, int accumulate,
-                                          int64_t slot_stride) {
-    if (!accumulate) out += G.slot * slot_stride;
+                                          const SlotMap &slots) {
+    if (!accumulate) out += slots.base[G.set] + G.slot * slots.stride[G.set];
 #pragma unroll
     for (int t = 0; t < TPL; t++) {
         const int idx = t * 64 + lane;
@@ -279,7 +279,7 @@ __device__ __forceinline__ void far_f64_body(const double *__restrict__ src, con
                                              const double *__restrict__ norms, const int *__restrict__ gorder,
                                              const FarGroup *__restrict__ groups, const FarInterval *__restrict__ iv,
                                              const int *__restrict__ active, double *__restrict__ out, double coef,
-                                             int accumulate, int64_t slot_stride) {
+                                             int accumulate, const SlotMap slots) {
     const int gi = gorder[blockIdx.x];
     const FarGroup G = groups[gi];
     if (active && !active[G.susp]) return;
@@ -311,7 +311,7 @@ __device__ __forceinline__ void far_f64_body(const double *__restrict__ src, con
         else
             far_range<KIND, TPL, true>(src, b, e, x, y, z, nx, ny, nz, incl, ax, ay, az);
     }
-    store_far<TPL>(G, lane, ax, ay, az, out, KIND == 0 ? kTracW * coef : coef, accumulate, slot_stride);
+    store_far<TPL>(G, lane, ax, ay, az, out, KIND == 0 ? kTracW * coef : coef, accumulate, slots);
 }
 
 // The direct FP64 far field (the whole fine grid) and the same sum over the
@@ -323,8 +323,8 @@ __global__ __launch_bounds__(64) void k_far_f64(const double *__restrict__ src, 
                                                 const FarGroup *__restrict__ groups,
                                                 const FarInterval *__restrict__ iv, const int *__restrict__ active,
                                                 double *__restrict__ out, double coef, int accumulate,
-                                                int64_t slot_stride) {
-    far_f64_body<KIND, TPL>(src, coords, norms, gorder, groups, iv, active, out, coef, accumulate, slot_stride);
+                                                const SlotMap slots) {
+    far_f64_body<KIND, TPL>(src, coords, norms, gorder, groups, iv, active, out, coef, accumulate, slots);
 }
 template <int KIND, int TPL>
 __global__ __launch_bounds__(64) void k_far_f64_lvl(const double *__restrict__ src, const double *__restrict__ coords,
@@ -332,8 +332,8 @@ __global__ __launch_bounds__(64) void k_far_f64_lvl(const double *__restrict__ s
                                                     const FarGroup *__restrict__ groups,
                                                     const FarInterval *__restrict__ iv, const int *__restrict__ active,
                                                     double *__restrict__ out, double coef, int accumulate,
-                                                    int64_t slot_stride) {
-    far_f64_body<KIND, TPL>(src, coords, norms, gorder, groups, iv, active, out, coef, accumulate, slot_stride);
+                                                    const SlotMap slots) {
+    far_f64_body<KIND, TPL>(src, coords, norms, gorder, groups, iv, active, out, coef, accumulate, slots);
 }
 
 // far field, FP32 pair arithmetic with two-level accumulation: FP32 partial sums
@@ -345,7 +345,7 @@ __global__ __launch_bounds__(64) void k_far_f32(const float *__restrict__ src, c
                                                 const int *__restrict__ gorder, const FarGroup *__restrict__ groups,
                                                 const FarInterval *__restrict__ iv, const int *__restrict__ active,
                                                 double *__restrict__ out, double coef, int accumulate,
-                                                int64_t slot_stride) {
+                                                const SlotMap slots) {
     const int gi = gorder[blockIdx.x];
     const FarGroup G = groups[gi];
     if (active && !active[G.susp]) return;
@@ -391,14 +391,14 @@ __global__ __launch_bounds__(64) void k_far_f32(const float *__restrict__ src, c
             }
         }
     }
-    store_far<TPL>(G, lane, ax, ay, az, out, coef, accumulate, slot_stride);
+    store_far<TPL>(G, lane, ax, ay, az, out, coef, accumulate, slots);
 }
 
 struct FarLaunch {
     const void *src;
     const double *tcoords, *tnorms;
     const float *trg32;
-    int64_t ntrg;
+    const SlotMap &slots;
     bool levels;
 };
 
@@ -406,16 +406,15 @@ template <int KIND, int TPL>
 static void far_dispatch_prec(int prec, const FarLaunch &a, int ngroups, const int *go, const FarGroup *gr,
                               const FarInterval *iv, const int *active, double *out, double coef, int acc,
                               hipStream_t s) {
-    const int64_t stride = 3 * a.ntrg;
     if (prec == 0 && a.levels)
         k_far_f64_lvl<KIND, TPL><<<dim3(ngroups), dim3(64), 0, s>>>((const double *)a.src, a.tcoords, a.tnorms, go,
-                                                                   gr, iv, active, out, coef, acc, stride);
+                                                                   gr, iv, active, out, coef, acc, a.slots);
     else if (prec == 0)
         k_far_f64<KIND, TPL><<<dim3(ngroups), dim3(64), 0, s>>>((const double *)a.src, a.tcoords, a.tnorms, go, gr,
-                                                               iv, active, out, coef, acc, stride);
+                                                               iv, active, out, coef, acc, a.slots);
     else
         k_far_f32<KIND, TPL><<<dim3(ngroups), dim3(64), 0, s>>>((const float *)a.src, a.trg32, go, gr, iv, active,
-                                                               out, coef, acc, stride);
+                                                               out, coef, acc, a.slots);
 }
 
 template <int KIND>
@@ -431,11 +430,11 @@ static void far_dispatch_tpl(int tpl, int prec, const FarLaunch &a, int ngroups,
 }
 
 void launch_far(int kind, int prec, int tpl, const void *src, const double *tcoords, const double *tnorms,
-                const float *trg32, int64_t ntrg, int ngroups, const int *go, const FarGroup *gr,
+                const float *trg32, const SlotMap &slots, int ngroups, const int *go, const FarGroup *gr,
                 const FarInterval *iv, const int *active, double *out, double coef, int acc, hipStream_t s,
                 bool levels) {
     if (ngroups <= 0) return;
-    const FarLaunch a{src, tcoords, tnorms, trg32, ntrg, levels};
+    const FarLaunch a{src, tcoords, tnorms, trg32, slots, levels};
     if (kind == 0)
         far_dispatch_tpl<0>(tpl, prec, a, ngroups, go, gr, iv, active, out, coef, acc, s);
     else

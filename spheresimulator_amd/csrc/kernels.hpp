@@ -68,8 +68,14 @@ struct LevelViews {
     void *src[kMaxLevels] = {};              // source records (force words written per apply)
     const double *part[kMaxLevels] = {};     // partial-sum slots of the level's lists (level, then source cells)
     int nslot[kMaxLevels] = {};
-    int64_t stride = 0;                      // between slots
+    int64_t stride[kMaxLevels] = {};         // between slots
     const int64_t *body_off = nullptr;       // per tile: body-frame values of the stacked level points
+};
+
+// Partial sums of work lists: slot s of target t of target set k (of a joint list:
+// the fine grid, then the levels) lies at base[k] + s stride[k] + 3 t.
+struct SlotMap {
+    int64_t base[1 + kMaxLevels] = {}, stride[1 + kMaxLevels] = {};
 };
 
 // source records (x, y, z, w*in, 0, 0) (in NULL: zero forces) and FP32 target records (x, n, 0, 0) of n points
@@ -79,11 +85,11 @@ void launch_pack_src_f32(int64_t n, const double *coords, const double *w, const
                          hipStream_t s);
 void launch_pack_trg_f32(int64_t n, const double *coords, const double *norms, float *trg, hipStream_t s);
 
-// far field over ntrg targets (FP64: tcoords/tnorms, FP32: trg32 records):
+// far field (FP64: targets tcoords/tnorms, FP32: trg32 records):
 // accumulate=1: out += coef * sum over the listed pairs;
-// accumulate=0: slot k of out (stride 3*ntrg) = coef * the sum over source slice k
+// accumulate=0: slot k of out (slots) = coef * the sum over source slice k
 void launch_far(int kind, int prec, int tpl, const void *src, const double *tcoords, const double *tnorms,
-                const float *trg32, int64_t ntrg, int ngroups, const int *group_order, const FarGroup *groups,
+                const float *trg32, const SlotMap &slots, int ngroups, const int *group_order, const FarGroup *groups,
                 const FarInterval *iv, const int *active, double *out, double coef, int accumulate, hipStream_t s,
                 bool levels = false);
 

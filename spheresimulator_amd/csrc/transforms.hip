@@ -103,7 +103,7 @@ __global__ __launch_bounds__(256) void k_pack_levels(DevGeom g, LevelViews L, T 
         const int64_t i = 3 * (L.off[l][S] + k - first[l]);
         double v[3] = {0.0, 0.0, 0.0};
         const double *part = L.part[l] + i;
-        for (int s = 0; s < L.nslot[l]; s++, part += L.stride)
+        for (int s = 0; s < L.nslot[l]; s++, part += L.stride[l])
             for (int c = 0; c < 3; c++) v[c] += part[c];
         rotate(g.quat + 4 * S, -1.0, v, o);
     }
