@@ -377,35 +377,29 @@ Operator::Operator(int nsusp, const int *counts, const double *pos, const double
     }
     ls64_.fp64 = true;
     // coarse FP32 operator of the mixed form's preconditioning solves: orders
-    // 5, 4, 3, 2 from about 2, 3, 5, 8 (R_s + R_t) (capped at p), source cells of 32
-    // equivalent point forces from 2.5 cell radii (on the check sphere).  Spheres
-    // of order above 10 also meet their nearest far neighbours, from 1.5, on a
-    // grid of order 10 (170 points; order 12 has 338) instead of their own: that
-    // shell is half of the set's pair evaluations (1500 spheres p=12 in chains:
-    // 1.79e9 -> 0.95e9).  Its truncation (2^-11 at 1.5) is below order 5's at 2,
-    // and order 5 then starts a little later, so that the set's error does not grow.
-    // Without that level the separations lie a little beyond 2, 3, 5, 8: the
-    // octahedral grids' interpolation adds 0.5 % to the error that Gauss-Legendre
-    // grids had from there, and this takes it off again (256 spheres p=8: 9.23e-4 ->
-    // 8.98e-4 for 1 % more pair evaluations).
-    if (nsph_ > 0 && *std::max_element(order_.begin(), order_.end()) > 10) {
-        lsc_.nlev = 5;
-        const double a[5] = {1.5, 2.05, 3.01, 5.01, 8.02};
+    // 5, 4, 3, 2 from 2, 3, 5, 8 (R_s + R_t) (capped at p), source cells of 32
+    // equivalent point forces from 2.5 cell radii (on the check sphere).  A sphere of
+    // order above 10 also meets its nearest far neighbours, from 1.5, on a grid of
+    // order 10 (170 points; order 12 has 338) instead of its own: that shell is half
+    // of the set's pair evaluations (1500 spheres p=12 in chains: 1.79e9 -> 0.95e9).
+    // Whether a pair does is a matter of the two spheres alone (klass in
+    // ensure_levels), so that a suspension's operator does not depend on the orders
+    // of the others of a batch.
+    lsc_.nlev = 5;
+    {
+        const double a[5] = {1.5, 2.0, 3.0, 5.0, 8.0};
         const int q[5] = {10, 5, 4, 3, 2};
         std::copy(a, a + 5, lsc_.alo);
         std::copy(q, q + 5, lsc_.order);
-    } else {
-        const double a[4] = {2.01, 3.01, 5.01, 8.02};
-        const int q[4] = {5, 4, 3, 2};
-        std::copy(a, a + 4, lsc_.alo);
-        std::copy(q, q + 4, lsc_.order);
     }
+    lsc_.high_order = 10;
     lsc_.fp64 = false;
     lsc_.cells = ls32_.cells;
     lsc_.cell_theta = 2.5;
     lsc_.equiv_k = 32;
     if (const char *v = std::getenv("SPHSTK_COARSE_ALPHA")) {
         lsc_.nlev = 4;
+        lsc_.high_order = 0;
         for (int l = 0; l < 4; l++) lsc_.order[l] = 5 - l;
         const int got = std::sscanf(v, "%lf,%lf,%lf,%lf:%d,%d,%d,%d", &lsc_.alo[0], &lsc_.alo[1], &lsc_.alo[2],
                                     &lsc_.alo[3], &lsc_.order[0], &lsc_.order[1], &lsc_.order[2], &lsc_.order[3]);
@@ -578,6 +572,7 @@ void Operator::autotune_inner(double &budget_s) {
         ls32_.tpl = tpl;
         ls32_.nlev = keep.nlev;
         ls32_.first_level = keep.first_level;
+        ls32_.high_order = keep.high_order;
         std::copy(keep.alo, keep.alo + kMaxLevels, ls32_.alo);
         std::copy(keep.order, keep.order + kMaxLevels, ls32_.order);
         ls32_.fp64 = false;
@@ -1074,7 +1069,10 @@ void Operator::ensure_levels(LevelSet &S) {
         // q = max(R_s / (d - R_t), R_t / (d - R_s)) (the source density's
         // truncated degrees decay like R_s / (d - R_t) at the target, the
         // target grid's interpolation error like R_t / (d - R_s)): s' = s for
-        // equal radii, smaller (a finer level) for unequal ones.
+        // equal radii, smaller (a finer level) for unequal ones.  So does the coarse
+        // set's level for high orders, which else would replace exact sums with a
+        // truncation of (R_big / (d - R_small))^11, 3.6e-3 for radii 1:3 at 1.5 where
+        // equal radii have 2^-11.
         auto klass = [&](int t, int s) {
             if (s == t) return -3;
             const double ddx = pos_[3 * s] - pos_[3 * t], ddy = pos_[3 * s + 1] - pos_[3 * t + 1],
@@ -1082,17 +1080,16 @@ void Operator::ensure_levels(LevelSet &S) {
             const double d2 = ddx * ddx + ddy * ddy + ddz * ddz;
             const double rr = 1.5 * rad_[s] + 1.5 * rad_[t], rs = rad_[s] + rad_[t];
             if (d2 < rr * rr) return -2;
-            double sep;
-            if (S.fp64) {
-                const double d = std::sqrt(d2);
+            const double d = std::sqrt(d2);
+            auto aware = [&] {
                 const double q = std::max(rad_[s] / (d - rad_[t]), rad_[t] / (d - rad_[s]));
-                sep = 0.5 * (1.0 / q + 1.0);
-            } else {
-                sep = std::sqrt(d2) / rs;
-            }
+                return 0.5 * (1.0 / q + 1.0);
+            };
+            const double sep = S.fp64 ? aware() : d / rs;
             if (sep < a[0]) return -1;
             int l = 0;
             while (l + 1 < nlev && sep >= a[l + 1]) l++;
+            if (l == 0 && S.high_order && (std::max(order_[s], order_[t]) <= S.high_order || aware() < a[0])) return -1;
             return l;
         };
         auto member = [&](int t, int r, int rt) {
@@ -1385,6 +1382,7 @@ void Operator::drop_fine_levels(LevelSet &S) const {
         }
         S.nlev--;
         S.first_level++;
+        S.high_order = 0;
     }
 }
 

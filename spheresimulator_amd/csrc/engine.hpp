@@ -176,6 +176,7 @@ constexpr int kNumLevels = 4; // levels of the FP32 inner set (source cells on a
 struct LevelSet {
     int nlev = kNumLevels;   // levels in use
     int first_level = 0;     // levels dropped before them (drop_fine_levels)
+    int high_order = 0;      // level 0 is for pairs with a sphere of order above this (0: for all)
     double alo[kMaxLevels];  // separations (in units of R_s + R_t) where levels 0..nlev-1 start
     int order[kMaxLevels];   // grid order of each level (capped by the sphere's order)
     bool fp64 = false;       // FP64 pair sums (else FP32)
