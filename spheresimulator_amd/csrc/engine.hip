@@ -578,7 +578,6 @@ void Operator::autotune_inner(double &budget_s) {
         ls32_.fp64 = false;
         ls32_.cells = keep.cells;
         ls32_.ready = false;
-        ls32_.levels.clear();
         auto tb = std::chrono::steady_clock::now();
         ensure_levels(ls32_);
         budget_s -= std::chrono::duration<double>(std::chrono::steady_clock::now() - tb).count();
@@ -1159,42 +1158,18 @@ void Operator::ensure_levels(LevelSet &S) {
     }
     tn.reset();
     // point sets, one after the other: fine grid, levels, equivalent points
-    S.levels.clear();
     std::vector<std::vector<int64_t>> level_off(nlev);
-    std::vector<int64_t> lbase(nlev + 1);
+    std::vector<int64_t> lbase(nlev + 1), off_by_sph(size_t(nlev) * nsph_);
     lbase[0] = npts_;
-    std::vector<double> lc, ln, lw; // level points of all levels
     for (int l = 0; l < nlev; l++) {
-        auto L = std::make_unique<FarLevel>();
         std::vector<int64_t> &off = level_off[l];
         off.assign(nsph_ + 1, 0);
-        std::vector<int64_t> off_by_sph(nsph_);
         for (int r = 0; r < nsph_; r++) {
             const int s = perm[r];
             off[r + 1] = off[r] + lpoints(l, order_[s]);
-            off_by_sph[s] = off[r];
+            off_by_sph[size_t(l) * nsph_ + s] = off[r];
         }
-        const int64_t nc = off[nsph_], at = lbase[l] - npts_;
-        lbase[l + 1] = lbase[l] + nc;
-        lc.resize(3 * (at + nc));
-        ln.resize(3 * (at + nc));
-        lw.resize(at + nc);
-        for (int s = 0; s < nsph_; s++) {
-            const ShTables &t = level_grid(S, l, order_[s]);
-            for (int q = 0; q < t.npts; q++) {
-                const int64_t g = at + off_by_sph[s] + q;
-                double nv[3];
-                qrot_host(&quat_[4 * s], &t.eta[3 * q], nv);
-                for (int c = 0; c < 3; c++) {
-                    ln[3 * g + c] = nv[c];
-                    lc[3 * g + c] = pos_[3 * s + c] + rad_[s] * nv[c];
-                }
-                lw[g] = rad_[s] * rad_[s] * t.w[q];
-            }
-        }
-        L->d_off_by_sph.upload(off_by_sph);
-        L->w.upload(std::vector<double>(lw.begin() + at, lw.end()));
-        S.levels.push_back(std::move(L));
+        lbase[l + 1] = lbase[l] + off[nsph_];
     }
     const int64_t ntrg = lbase[nlev];
     HostLists H;
@@ -1305,50 +1280,60 @@ void Operator::ensure_levels(LevelSet &S) {
     // records: positions now, force words per apply
     // (set-up of a set may run on a host thread of its own: nothing here goes to
     // the operator's stream, which may be capturing)
+    PhaseTimer pr("  records");
     const int64_t nlp = ntrg - npts_, neq = (int64_t)eq.size() / 8;
     const hipStream_t st0 = nullptr;
-    auto fine = [&](DevBuf<double> &d, const DevBuf<double> &from) {
-        if (npts_) SPHSTK_HIP(hipMemcpyAsync(d.p, from.p, sizeof(double) * 3 * npts_, hipMemcpyDeviceToDevice, st0));
-    };
+    S.off.upload(off_by_sph);
+    S.w.alloc(std::max<int64_t>(nlp, 1));
+    LevelPoints P;
+    LevelViews &V = S.views;
     if (S.fp64) {
-        std::vector<double> rec(8 * (size_t)nlp, 0.0);
-        for (int64_t i = 0; i < nlp; i++) std::copy(&lc[3 * i], &lc[3 * i] + 3, &rec[8 * i]);
         S.src64.alloc(std::max<int64_t>(8 * ntrg, 8));
         S.coords.alloc(std::max<int64_t>(3 * ntrg, 3));
         S.norms.alloc(std::max<int64_t>(3 * ntrg, 3));
         launch_pack_src_f64(npts_, d_coords_.p, d_w_.p, nullptr, S.src64.p, st0);
-        put(S.src64, 8 * npts_, rec);
-        fine(S.coords, d_coords_);
-        put(S.coords, 3 * npts_, lc);
-        fine(S.norms, d_norms_);
-        put(S.norms, 3 * npts_, ln);
+        SPHSTK_HIP(hipMemcpyAsync(S.coords.p, d_coords_.p, sizeof(double) * 3 * npts_, hipMemcpyDeviceToDevice, st0));
+        SPHSTK_HIP(hipMemcpyAsync(S.norms.p, d_norms_.p, sizeof(double) * 3 * npts_, hipMemcpyDeviceToDevice, st0));
+        P.src64 = S.src64.p, P.coords = S.coords.p, P.norms = S.norms.p;
     } else {
-        std::vector<float> rec(8 * (size_t)(nlp + neq), 0.f), trg(8 * (size_t)nlp, 0.f);
-        for (int64_t i = 0; i < nlp; i++)
-            for (int c = 0; c < 3; c++) {
-                rec[8 * i + c] = trg[8 * i + c] = (float)lc[3 * i + c];
-                trg[8 * i + 3 + c] = (float)ln[3 * i + c];
-            }
-        std::copy(eq.begin(), eq.end(), rec.begin() + 8 * nlp);
         S.src32.alloc(std::max<int64_t>(8 * (ntrg + neq), 8));
         S.trg32.alloc(8 * std::max<int64_t>(ntrg, 1));
         launch_pack_src_f32(npts_, d_coords_.p, d_w_.p, nullptr, S.src32.p, st0);
         launch_pack_trg_f32(npts_, d_coords_.p, d_norms_.p, S.trg32.p, st0);
-        put(S.src32, 8 * npts_, rec);
-        put(S.trg32, 8 * npts_, trg);
+        put(S.src32, 8 * ntrg, eq);
         if (S.agg) S.agg->eq32 = S.src32.p + 8 * ntrg;
+        P.src32 = S.src32.p, P.trg32 = S.trg32.p;
     }
-    SPHSTK_HIP(hipGetLastError());
-    SPHSTK_HIP(hipStreamSynchronize(st0));
-    LevelViews &V = S.views;
     for (int l = 0; l < nlev; l++) {
-        V.off[l] = S.levels[l]->d_off_by_sph.p;
-        V.w[l] = S.levels[l]->w.p;
+        V.off[l] = S.off.p + size_t(l) * nsph_;
+        V.w[l] = S.w.p + (lbase[l] - npts_);
         V.src[l] = S.fp64 ? (void *)(S.src64.p + 8 * lbase[l]) : (void *)(S.src32.p + 8 * lbase[l]);
         V.part[l] = S.all.part.p ? S.all.part.p + S.all.map.base[1 + l] + 3 * lbase[l] : nullptr;
         V.nslot[l] = H.sets[1 + l].nslot;
         V.stride[l] = S.all.map.stride[1 + l];
+        P.base[l] = lbase[l];
     }
+    // the body-frame grids in use
+    std::vector<double> tab;
+    std::vector<int2> grids(size_t(nlev) * (kMaxOrder + 1), int2{0, 0});
+    for (int l = 0; l < nlev; l++)
+        for (int p = 0; p <= kMaxOrder; p++)
+            if (level_points[l][p]) {
+                const ShTables &t = level_grid(S, l, p);
+                grids[size_t(l) * (kMaxOrder + 1) + p] = int2{(int)(tab.size() / 4), t.npts};
+                for (int q = 0; q < t.npts; q++) {
+                    tab.insert(tab.end(), &t.eta[3 * q], &t.eta[3 * q] + 3);
+                    tab.push_back(t.w[q]);
+                }
+            }
+    DevBuf<double> d_tab;
+    DevBuf<int2> d_grids;
+    d_tab.upload(tab);
+    d_grids.upload(grids);
+    P.tab = d_tab.p, P.grids = d_grids.p, P.w = S.w.p;
+    launch_level_points(geom_, P, V, st0);
+    SPHSTK_HIP(hipGetLastError());
+    SPHSTK_HIP(hipStreamSynchronize(st0));
     S.ready = true;
 }
 
@@ -1363,8 +1348,7 @@ const ShTables &Operator::level_grid(const LevelSet &S, int l, int p) const {
     return q < 0 ? sh_tables(p) : level_tables(q);
 }
 const Resample &Operator::level_matrices(const LevelSet &S, int l, int p) const {
-    const int q = order_on_level(S, l, p);
-    return q < 0 ? resample_tables(p, p) : level_resample(p, q);
+    return level_resample(p, order_on_level(S, l, p));
 }
 
 // Levels on which every sphere keeps its own grid are the fine grid: their pairs
@@ -1390,7 +1374,8 @@ void Operator::drop_fine_levels(LevelSet &S) const {
 // matrix per order: levels stacked by rows (down) and by columns (up), so that
 // each direction is one launch (four or six levels had one launch each way per
 // level, each too small to fill the GPU: 1024 spheres p=12, FP32 set, 8
-// launches of 138 us per apply).
+// launches of 138 us per apply).  Levels that are a sphere's own grid have no part
+// in it (as identity matrices they were 490 of 540 rows for order 6 beside order 16).
 void Operator::level_transforms(LevelSet &S) {
     std::vector<bool> used(kMaxOrder + 1, false);
     for (int p : order_) used[p] = true;
@@ -1399,14 +1384,21 @@ void Operator::level_transforms(LevelSet &S) {
     S.max_lev_pts = 0;
     for (int p = 0; p <= kMaxOrder; p++) {
         if (!used[p]) continue;
-        std::vector<const Resample *> rs;
+        std::vector<const Resample *> rs(S.nlev, nullptr);
         std::vector<int> key{p};
         for (int l = 0; l < S.nlev; l++) {
-            rs.push_back(&level_matrices(S, l, p));
-            key.push_back(order_on_level(S, l, p));
-            V.first[p][l + 1] = V.first[p][l] + rs[l]->nc;
+            const int q = order_on_level(S, l, p);
+            key.push_back(q);
+            V.first[p][l + 1] = V.first[p][l];
+            if (q < 0) {
+                V.own[p] |= 1u << l;
+            } else {
+                rs[l] = &level_matrices(S, l, p);
+                V.first[p][l + 1] += rs[l]->nc;
+            }
         }
-        const int n = rs[0]->n, nl = V.first[p][S.nlev];
+        const int n = grid_points(p), nl = V.first[p][S.nlev];
+        if (!nl) continue;
         S.max_lev_pts = std::max(S.max_lev_pts, nl);
         std::vector<int> lev_of(nl);
         for (int l = 0; l < S.nlev; l++) std::fill(lev_of.begin() + V.first[p][l], lev_of.begin() + V.first[p][l + 1], l);
@@ -1580,6 +1572,7 @@ void Operator::pack(const double *in, int prec, const LevelSet *S) {
     const bool f32 = prec == 1 || prec == 3;
     double *s64 = nullptr;
     float *s32 = nullptr, *b32 = nullptr;
+    const LevelViews L = S ? S->views : LevelViews{};
     if (S && f32) {
         body32_.alloc(body64_.n);
         b32 = body32_.p;
@@ -1592,7 +1585,7 @@ void Operator::pack(const double *in, int prec, const LevelSet *S) {
     } else if (prec >= 0 && ncopy_ == 1) {
         s64 = src64_.p;
     }
-    launch_pack_body(geom_, in, body64_.p, b32, s64, s32, max_pts_, stream_);
+    launch_pack_body(geom_, in, body64_.p, b32, s64, s32, L, max_pts_, stream_);
 }
 
 // FP64: fine grid, direct sum over all far pairs.  FP32: multi-level (fine for
@@ -1672,8 +1665,8 @@ void Operator::p2p(const double *in, double *out, double cId, double cSL, double
         if (side != stream_) SPHSTK_HIP(hipStreamWaitEvent(stream_, ev_coef_, 0));
         self_terms(kind, cSL, cTrac, active, stream_);
         if (side != stream_) SPHSTK_HIP(hipStreamWaitEvent(stream_, ev_join_, 0));
-        launch_sheval_gather(geom_, d_trg_slot_off_.p, d_trg_nsrc_.p, evscratch_.p, f, in, out, cid, clop,
-                             overwrite && first, active, stream_);
+        launch_sheval_gather(geom_, d_trg_slot_off_.p, d_trg_nsrc_.p, evscratch_.p, f, S ? S->views : LevelViews{}, in,
+                             out, cid, clop, overwrite && first, active, stream_);
         if (S) levels_up(*S, out, active);
         cid = clop = 0.0;
         first = false;
@@ -1812,8 +1805,8 @@ void Operator::rigid_p2p(const double *force, const double *rho0, double *out, d
                      lists_rigid_.order.p, lists_rigid_.groups.p, lists_rigid_.iv.p, out, cTrac, 1, stream_);
     self_terms(0, 0.0, cTrac, nullptr, stream_);
     near_terms(0, 0.0, cTrac, nullptr, stream_);
-    launch_sheval_gather(geom_, d_trg_slot_off_.p, d_trg_nsrc_.p, evscratch_.p, FarSum{}, rho0, out, cId, 0.0, false,
-                         nullptr, stream_);
+    launch_sheval_gather(geom_, d_trg_slot_off_.p, d_trg_nsrc_.p, evscratch_.p, FarSum{}, LevelViews{}, rho0, out,
+                         cId, 0.0, false, nullptr, stream_);
     SPHSTK_HIP(hipGetLastError());
 }
 
@@ -1824,8 +1817,8 @@ void Operator::rigid_velocity(const double *rho, double inv_mu, double *vel) {
     analyse(nullptr, stream_);
     self_terms(1, 1.0, 0.0, nullptr, stream_);
     near_terms(1, 1.0, 0.0, nullptr, stream_);
-    launch_sheval_gather(geom_, d_trg_slot_off_.p, d_trg_nsrc_.p, evscratch_.p, FarSum{}, rho, u_ns_.p, 0.0, 0.0, true,
-                         nullptr, stream_);
+    launch_sheval_gather(geom_, d_trg_slot_off_.p, d_trg_nsrc_.p, evscratch_.p, FarSum{}, LevelViews{}, rho,
+                         u_ns_.p, 0.0, 0.0, true, nullptr, stream_);
     far_run(lists_rv_mid_, 1, 0, src64_.p, d_coords_.p, d_norms_.p, nullptr, chunks_.p, (int)chunks_.n,
             1.0 / (8.0 * kPi), u_ns_.p, nullptr);
     launch_rigid_avg(geom_, u_ns_.p, inv_mu, vel_ns_.p, stream_);

@@ -131,12 +131,6 @@ void build_far_lists(FarLists &L, int nsusp, const std::vector<int64_t> &susp_sp
                      const std::vector<int64_t> &toff, const std::vector<int64_t> &soff, const std::vector<Runs> &runs,
                      int tpl, int split, int64_t want_items, const std::vector<int64_t> *src_susp_off = nullptr);
 
-// One level of a multi-level far field: per-sphere grids of a lower order.
-struct FarLevel {
-    DevBuf<int64_t> d_off_by_sph; // first level point of each sphere
-    DevBuf<double> w;
-};
-
 // Device copies of one matrix per order in the layout of the transform GEMMs.
 struct GemmTables {
     DevBuf<double> d[kMaxOrder + 1];
@@ -181,7 +175,8 @@ struct LevelSet {
     int order[kMaxLevels];   // grid order of each level (capped by the sphere's order)
     bool fp64 = false;       // FP64 pair sums (else FP32)
     int tpl = 1;             // targets per lane of its work lists
-    std::vector<std::unique_ptr<FarLevel>> levels;
+    DevBuf<int64_t> off;              // per level: first level point of each sphere
+    DevBuf<double> w;                 // weights of the points of all levels
     FarLists all;                     // mid range, levels, source cells
     int mid_slots = 0;                // slots of the mid range (the fine grid's targets come first)
     DevBuf<float> src32, trg32;       // source and target records (FP32 set)
@@ -319,7 +314,7 @@ class Operator {
     void ensure_levels(LevelSet &S);
     void level_transforms(LevelSet &S);
     // grid of a sphere of order p on level l of a set, and the matrices between
-    // it and the fine grid
+    // it and the fine grid (grids of a lower order than the sphere's)
     const ShTables &level_grid(const LevelSet &S, int l, int p) const;
     const Resample &level_matrices(const LevelSet &S, int l, int p) const;
     void drop_fine_levels(LevelSet &S) const;

@@ -941,7 +941,7 @@ __global__ __launch_bounds__(64 * kSrcWaves) __attribute__((amdgpu_waves_per_eu(
 // each had a launch and a read-modify-write of the vector before.
 __global__ __launch_bounds__(256) void k_sheval_gather(DevGeom g, const int64_t *__restrict__ trg_slot_off,
                                                        const int *__restrict__ trg_nsrc, const double *__restrict__ scratch,
-                                                       FarSum far, const double *__restrict__ in,
+                                                       FarSum far, LevelViews L, const double *__restrict__ in,
                                                        double *__restrict__ out, double cId, double cLOP, int overwrite,
                                                        const int *__restrict__ active) {
     __shared__ double sh[8];
@@ -958,10 +958,16 @@ __global__ __launch_bounds__(256) void k_sheval_gather(DevGeom g, const int64_t 
     if (cLOP != 0.0) rigid_part(g, in, off, off + nT, R, sh, A, B);
     const int64_t base = trg_slot_off[T];
     const int ns = trg_nsrc[T];
+    const unsigned own = L.own[g.order[T]];
     for (int i = threadIdx.x; i < 3 * nT; i += blockDim.x) {
         const int64_t j = 3 * off + i;
         double s = 0.0;
         for (int k = 0; k < far.nslot; k++) s += far.part[k * far.stride + j];
+        for (int l = 0; own >> l; l++)
+            if (own >> l & 1) {
+                const double *part = L.part[l] + 3 * L.off[l][T] + i;
+                for (int k = 0; k < L.nslot[l]; k++) s += part[k * L.stride[l]];
+            }
         double v = 0.0;
         for (int k = 0; k < ns; k++) v += scratch[base + (int64_t)k * 3 * nT + i];
         s += v + cId * in[j];
@@ -1012,10 +1018,10 @@ void launch_sheval_items(const DevGeom &g, int mode, const double *rec, const Ev
 }
 
 void launch_sheval_gather(const DevGeom &g, const int64_t *trg_slot_off, const int *trg_nsrc, const double *scratch,
-                          const FarSum &far, const double *in, double *out, double cId, double cLOP, bool overwrite,
-                          const int *active, hipStream_t s) {
+                          const FarSum &far, const LevelViews &L, const double *in, double *out, double cId, double cLOP,
+                          bool overwrite, const int *active, hipStream_t s) {
     if (!g.nsph) return;
-    k_sheval_gather<<<dim3(g.nsph), dim3(256), 0, s>>>(g, trg_slot_off, trg_nsrc, scratch, far, in, out, cId, cLOP,
+    k_sheval_gather<<<dim3(g.nsph), dim3(256), 0, s>>>(g, trg_slot_off, trg_nsrc, scratch, far, L, in, out, cId, cLOP,
                                                       overwrite ? 1 : 0, active);
 }
 

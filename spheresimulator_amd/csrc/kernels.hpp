@@ -63,6 +63,9 @@ struct ShGemm {
 struct LevelViews {
     int nlev = 0;
     int first[kMaxOrder + 1][kMaxLevels + 1] = {};
+    // levels on which spheres of order p keep their own grid (bits): these have no
+    // stacked points; packing and gathering the fine grid serve them too
+    unsigned own[kMaxOrder + 1] = {};
     const int64_t *off[kMaxLevels] = {};
     const double *w[kMaxLevels] = {};
     void *src[kMaxLevels] = {};              // source records (force words written per apply)
@@ -101,10 +104,11 @@ void launch_equiv_forces(int ncell, int K, int Kc, const double *P, const double
                          const double *rho, const int *susp, const int *active, float *eq, hipStream_t s);
 
 // Transforms between grids and coefficients (transforms.hip).  pack_body: the
-// body-frame values bd (FP64) and/or bf (FP32) of `in`, and the force words of
-// the source records src64 / src32 (NULL: not wanted).
+// body-frame values bd (FP64) and, if wanted, bf (FP32) of `in`, and the force words
+// of the source records src64 / src32 (NULL: not wanted), on the fine grids and on
+// the levels of L that are a sphere's own grid.
 void launch_pack_body(const DevGeom &g, const double *in, double *bd, float *bf, double *src64, float *src32,
-                      int max_points, hipStream_t s);
+                      const LevelViews &L, int max_points, hipStream_t s);
 // coef: per sphere; cbody: the same as GEMM columns (per tile)
 void launch_analysis(const DevGeom &g, const ShGemm &M, const double *body, double *coef, double *cbody,
                      const int *active, hipStream_t s);
@@ -112,6 +116,18 @@ void launch_analysis(const DevGeom &g, const ShGemm &M, const double *body, doub
 // synthesis with per-degree blocks (a sphere's operator on its own surface)
 void launch_synthesis(const DevGeom &g, const ShGemm &M, const double *cbody, const int64_t *dst_off, int mul,
                       double coef, int rpow, double *out, const int *active, hipStream_t s);
+// Points of the levels of a set from their grids in the body frame: level l of order
+// p has the n points (x, y, z, weight) from tab + 4 first on, grids[l (kMaxOrder + 1) + p]
+// = (first, n).  Level l's points follow base[l] others in the set's coords, norms and
+// src64 (FP64) or trg32 and src32 (FP32); w: the weights of all levels in a row.
+struct LevelPoints {
+    const double *tab = nullptr;
+    const int2 *grids = nullptr;
+    int64_t base[kMaxLevels] = {};
+    double *w = nullptr, *coords = nullptr, *norms = nullptr, *src64 = nullptr;
+    float *trg32 = nullptr, *src32 = nullptr;
+};
+void launch_level_points(const DevGeom &g, const LevelPoints &P, const LevelViews &L, hipStream_t s);
 void launch_levels_down(const DevGeom &g, const ShGemm &M, bool fp64, const void *body, const LevelViews &L,
                         const int *active, hipStream_t s);
 void launch_pack_levels(const DevGeom &g, bool fp64, const LevelViews &L, void *body, int max_points, hipStream_t s);
@@ -154,11 +170,12 @@ struct FarSum {
 void launch_sheval_items(const DevGeom &g, int mode, const double *rec, const EvalItem *items, int nitems,
                          double *scratch, double cSL, double cTrac, const int *active, hipStream_t s,
                          const SrcItems *by_src = nullptr);
-// per-target gather: out (+)= far sum + the target's items + cId in + cLOP L[in]
-// (overwrite: out = ..., zero on inactive suspensions)
+// per-target gather: out (+)= far sum (with that of the levels of L that are a
+// sphere's own grid) + the target's items + cId in + cLOP L[in] (overwrite: out = ...,
+// zero on inactive suspensions)
 void launch_sheval_gather(const DevGeom &g, const int64_t *trg_slot_off, const int *trg_nsrc, const double *scratch,
-                          const FarSum &far, const double *in, double *out, double cId, double cLOP, bool overwrite,
-                          const int *active, hipStream_t s);
+                          const FarSum &far, const LevelViews &L, const double *in, double *out, double cId, double cLOP,
+                          bool overwrite, const int *active, hipStream_t s);
 void launch_identity(const DevGeom &g, const double *in, double *out, double cId, const int *active,
                      hipStream_t s);
 void launch_lop(const DevGeom &g, const double *in, double *out, double cLOP, const int *active, hipStream_t s);

@@ -54,10 +54,10 @@ __device__ __forceinline__ int64_t body_at(int col, int t) {
 // Grid values of every sphere, rotated to its body frame, as GEMM columns
 // (zero for absent spheres and padding columns), and the force words w f of the
 // far field's source records (whose positions were set at set-up).
-template <bool D, bool F>
+template <bool F>
 __global__ __launch_bounds__(256) void k_pack_body(DevGeom g, const double *__restrict__ in, double *__restrict__ bd,
                                                    float *__restrict__ bf, double *__restrict__ src64,
-                                                   float *__restrict__ src32) {
+                                                   float *__restrict__ src32, LevelViews L) {
     const SphTile Ti = g.tiles[blockIdx.y];
     const int n = (Ti.p + 1) * (2 * Ti.p + 2), cols = body_cols(n);
     const int e = blockIdx.x * blockDim.x + threadIdx.x, t = e & 15, k = e >> 4;
@@ -68,22 +68,67 @@ __global__ __launch_bounds__(256) void k_pack_body(DevGeom g, const double *__re
         const int64_t i = g.pt_off[S] + k;
         const double v[3] = {in[3 * i], in[3 * i + 1], in[3 * i + 2]};
         rotate(g.quat + 4 * S, -1.0, v, o);
-        if (src64) {
-            const double wi = g.w[i];
+        const double wi = g.w[i];
+        if (src64)
             for (int c = 0; c < 3; c++) src64[8 * i + 3 + c] = wi * v[c];
-        }
-        if (src32) {
-            const double wi = g.w[i];
+        if (src32)
             for (int c = 0; c < 3; c++) src32[8 * i + 3 + c] = (float)(wi * v[c]);
-        }
+        const unsigned own = L.own[Ti.p];
+        for (int l = 0; own >> l; l++)
+            if (own >> l & 1) {
+                const int64_t q = 8 * (L.off[l][S] + k) + 3;
+                if (src64)
+                    for (int c = 0; c < 3; c++) static_cast<double *>(L.src[l])[q + c] = wi * v[c];
+                if (src32)
+                    for (int c = 0; c < 3; c++) static_cast<float *>(L.src[l])[q + c] = (float)(wi * v[c]);
+            }
     }
     const int64_t base = g.body_off[blockIdx.y];
     for (int c = 0; c < 3; c++)
         if (3 * k + c < cols) {
             const int64_t a = base + body_at(3 * k + c, t);
-            if (D) bd[a] = o[c];
+            bd[a] = o[c];
             if (F) bf[a] = (float)o[c];
         }
+}
+
+// One workgroup per sphere and level; bound by its writes (232 bytes a point, FP64).
+// Points and records made on the host, one sphere after the other, and sent over took
+// most of a set's build: FP64 set of 48 suspensions of orders 6 to 16 (1.2e6 points)
+// 0.19 -> 0.06 s, of 1024 spheres p=12 0.068 -> 0.040 s, both with the identity
+// matrices of own-grid levels gone as well.
+template <bool FP64>
+__global__ __launch_bounds__(128) void k_level_points(DevGeom g, LevelPoints P, LevelViews L) {
+    const int S = blockIdx.x, l = blockIdx.y;
+    const int2 gr = P.grids[l * (kMaxOrder + 1) + g.order[S]];
+    const double R = g.rad[S];
+    const double q[4] = {g.quat[4 * S], g.quat[4 * S + 1], g.quat[4 * S + 2], g.quat[4 * S + 3]};
+    for (int k = threadIdx.x; k < gr.y; k += blockDim.x) {
+        const double *e = P.tab + 4 * ((int64_t)gr.x + k);
+        const int64_t i = P.base[l] + L.off[l][S] + k;
+        double nv[3];
+        rotate(q, 1.0, e, nv);
+        P.w[i - P.base[0]] = R * R * e[3];
+        for (int c = 0; c < 3; c++) {
+            const double x = g.pos[3 * S + c] + R * nv[c];
+            if (FP64) {
+                P.coords[3 * i + c] = x;
+                P.norms[3 * i + c] = nv[c];
+                P.src64[8 * i + c] = x;
+                P.src64[8 * i + 3 + c] = 0.0;
+            } else {
+                P.trg32[8 * i + c] = P.src32[8 * i + c] = (float)x;
+                P.trg32[8 * i + 3 + c] = (float)nv[c];
+                P.src32[8 * i + 3 + c] = 0.f;
+            }
+        }
+        for (int c = 6; c < 8; c++) {
+            if (FP64)
+                P.src64[8 * i + c] = 0.0;
+            else
+                P.trg32[8 * i + c] = P.src32[8 * i + c] = 0.f;
+        }
+    }
 }
 
 // The level fields of every sphere (each the sum of its far-field lists'
@@ -215,15 +260,22 @@ dim3 pack_grid(const DevGeom &g, int max_points) {
 } // namespace
 
 void launch_pack_body(const DevGeom &g, const double *in, double *bd, float *bf, double *src64, float *src32,
-                      int max_points, hipStream_t s) {
+                      const LevelViews &L, int max_points, hipStream_t s) {
     if (!g.nsph || !g.ntiles) return;
     const dim3 grid = pack_grid(g, max_points);
-    if (bd && bf)
-        k_pack_body<true, true><<<grid, dim3(256), 0, s>>>(g, in, bd, bf, src64, src32);
-    else if (bd)
-        k_pack_body<true, false><<<grid, dim3(256), 0, s>>>(g, in, bd, bf, src64, src32);
+    if (bf)
+        k_pack_body<true><<<grid, dim3(256), 0, s>>>(g, in, bd, bf, src64, src32, L);
     else
-        k_pack_body<false, true><<<grid, dim3(256), 0, s>>>(g, in, bd, bf, src64, src32);
+        k_pack_body<false><<<grid, dim3(256), 0, s>>>(g, in, bd, bf, src64, src32, L);
+}
+
+void launch_level_points(const DevGeom &g, const LevelPoints &P, const LevelViews &L, hipStream_t s) {
+    if (!g.nsph || !L.nlev) return;
+    const dim3 grid((unsigned)g.nsph, (unsigned)L.nlev);
+    if (P.coords)
+        k_level_points<true><<<grid, dim3(128), 0, s>>>(g, P, L);
+    else
+        k_level_points<false><<<grid, dim3(128), 0, s>>>(g, P, L);
 }
 
 void launch_analysis(const DevGeom &g, const ShGemm &M, const double *body, double *coef, double *cbody,
@@ -242,7 +294,7 @@ void launch_synthesis(const DevGeom &g, const ShGemm &M, const double *cbody, co
 
 void launch_levels_down(const DevGeom &g, const ShGemm &M, bool fp64, const void *body, const LevelViews &L,
                         const int *active, hipStream_t s) {
-    if (!g.nsph || !g.ntiles) return;
+    if (!g.nsph || !g.ntiles || !M.max_blk) return;
     const dim3 grid(M.max_blk, g.ntiles);
     if (fp64)
         k_sh_gemm<double, LEVEL_DOWN><<<grid, dim3(256), 0, s>>>(g, M, g.body_off, (const double *)body, L, SynthOut{},
@@ -253,7 +305,7 @@ void launch_levels_down(const DevGeom &g, const ShGemm &M, bool fp64, const void
 }
 
 void launch_pack_levels(const DevGeom &g, bool fp64, const LevelViews &L, void *body, int max_points, hipStream_t s) {
-    if (!g.nsph || !g.ntiles) return;
+    if (!g.nsph || !g.ntiles || !max_points) return;
     const dim3 grid = pack_grid(g, max_points);
     if (fp64)
         k_pack_levels<double><<<grid, dim3(256), 0, s>>>(g, L, (double *)body);
@@ -263,7 +315,7 @@ void launch_pack_levels(const DevGeom &g, bool fp64, const LevelViews &L, void *
 
 void launch_levels_up(const DevGeom &g, const ShGemm &M, bool fp64, const void *body, const LevelViews &L, double *out,
                       const int *active, hipStream_t s) {
-    if (!g.nsph || !g.ntiles) return;
+    if (!g.nsph || !g.ntiles || !M.max_blk) return;
     const dim3 grid(M.max_blk, g.ntiles);
     if (fp64)
         k_sh_gemm<double, LEVEL_UP><<<grid, dim3(256), 0, s>>>(g, M, L.body_off, (const double *)body, L, SynthOut{}, out,
