@@ -462,6 +462,7 @@ Operator::Operator(int nsusp, const int *counts, const double *pos, const double
             build_far_lists(lists_fine_, nsusp_, susp_sph_off_, pt_off_, pt_off_, runs_fine_, tpl, split, kWantItems);
         }
     }
+    lists_fine_.slots(); // with the handle, not in its first apply
     ls32_.tpl = ls64_.tpl = lsc_.tpl = tpl;
 
     src64_.alloc(std::max<int64_t>(8 * npts_, 8));
