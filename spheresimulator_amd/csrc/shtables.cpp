@@ -11,6 +11,7 @@
 // n(n+1) times that.  The analysis is the orthogonal projection in the grid's
 // quadrature inner product, which is exact for vector-SH degree <= p.
 #include "common.hpp"
+#include "pool.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -486,24 +487,13 @@ static std::unique_ptr<Resample> build_resample(int p, int pc, const ShTables &C
 }
 
 const Resample &resample_tables(int p, int pc) {
-    static std::mutex mu;
-    static std::map<std::pair<int, int>, std::unique_ptr<Resample>> cache;
-    std::lock_guard<std::mutex> lock(mu);
-    auto it = cache.find({p, pc});
-    if (it != cache.end()) return *it->second;
-    auto t = build_resample(p, pc, sh_tables(pc), pc == p);
-    const Resample &ref = *t;
-    cache[{p, pc}] = std::move(t);
-    return ref;
+    static Tables<std::pair<int, int>, Resample> kept;
+    return kept.get({p, pc}, [&] { return build_resample(p, pc, sh_tables(pc), pc == p); });
 }
 
 const Resample &level_resample(int p, int pc) {
-    static std::mutex mu;
-    static std::map<std::pair<int, int>, std::unique_ptr<Resample>> cache;
-    std::lock_guard<std::mutex> lock(mu);
-    auto &t = cache[{p, pc}];
-    if (!t) t = build_resample(p, pc, level_tables(pc), false, true);
-    return *t;
+    static Tables<std::pair<int, int>, Resample> kept;
+    return kept.get({p, pc}, [&] { return build_resample(p, pc, level_tables(pc), false, true); });
 }
 
 const ShTables &sh_tables(int p) {
