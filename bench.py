@@ -18,17 +18,17 @@ the final single layer and the rigid-body averages.
 * roofline: the mixed form's pair-sum kernel with the most time per timed
   solve, from HIP events the library records on its own stream around the
   launches of each apply: k_far_f64_lvl (the FP64 residual apply: mid range
-  and six levels) or k_far_f32 (per apply seven lists: mid range, four
-  levels, two source-cell lists; the coarse operator's applies and the FP32
-  operator's); the other is reported under "mixed".
+  and five levels) or k_far_f32 (mid range, four levels, five with the coarse
+  operator, and two source-cell lists per apply; the coarse operator's applies
+  and the FP32 operator's); the other is reported under "mixed".
 * cpu_baseline: the oracle's full operator apply (far, self and near terms)
   on a bounded sample of target spheres, scaled to a full FP64 solve with the
   FP64 apply count (kind "port", all host threads), labelled "extrapolated".
 * The 1024-sphere and batched workloads follow as extra keys when time allows.
 
-The driver runs `--steps 20 --warmup 5` under a time limit: when the first
-solve shows that the requested steps would not fit `--budget` seconds, the
-warmup is cut first and then the steps, and the line says so (`requested`).
+When the first solve shows that the requested steps would not fit `--budget`
+seconds, the warmup is cut first and then the steps, and the line says so
+(`requested`).
 """
 import argparse
 import json
@@ -267,7 +267,7 @@ def main():
     if f32 is not None:
         f32["coarse"] = far_roofline(stc, FP32_VALU_PEAK, "k_far_f32<traction>, coarse operator", 1)
         f32["inner"] = far_roofline(st32, FP32_VALU_PEAK, "k_far_f32<traction>, FP32 operator", 1)
-    f64 = far_roofline(st64ml, FP64_VALU_PEAK, "k_far_f64_lvl<traction>: the mid-range list and 6 level lists of "
+    f64 = far_roofline(st64ml, FP64_VALU_PEAK, "k_far_f64_lvl<traction>: the mid-range list and 5 level lists of "
                        "one FP64 residual apply in one launch", 1)
     out["roofline"], other = dominant(f32, f64, both, st64ml, cnt["steps"])
     if other is not None:

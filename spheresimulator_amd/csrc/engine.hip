@@ -25,8 +25,13 @@ namespace sphstk {
 namespace {
 
 constexpr int kMaxSupportedOrder = 20; // LDS of the expansion kernel bounds the order
-constexpr int64_t kChunk = 4096;  // most DOF per block of the segmented vector kernels
-constexpr int64_t kMinChunk = 512; // fewest, on problems that would not fill the GPU with kChunk
+// DOF per block of the segmented vector kernels: kMinChunk to kChunk, for
+// kWantChunks blocks.  FP64 solve of 64 spheres p=8 (3.1e4 unknowns) with at least
+// 256, 512, 1024 and 4096: 7.50, 7.45, 7.93 and 10.5 ms; 8 right-hand sides on 150
+// spheres p=10 (8.7e5) with 256, 1024 and 4096 blocks wanted: 130, 124.6, 123.8 ms;
+// mixed solve of 1024 spheres p=12 (1.04e6): 47.3, 46.3, 47.2 ms.
+constexpr int64_t kChunk = 4096;
+constexpr int64_t kMinChunk = 512;
 constexpr int64_t kWantChunks = 1024;
 constexpr int64_t kWantItems = 40000; // far-field work items wanted when a problem is small
 // most source slices of a target group: a slice is summed serially by one wave, a
@@ -34,9 +39,15 @@ constexpr int64_t kWantItems = 40000; // far-field work items wanted when a prob
 // order 8 (153 target groups): 0.292 ms an apply with 8, 0.259 with 16, 0.248 with
 // 32; a solve 7.31, 6.79 and 6.84 ms; 100 spheres mixed 9.37, 9.19 and 9.50 ms.
 constexpr int64_t kMaxSlices = 16;
-constexpr int64_t kMultiItems = 8192; // the same for several right-hand sides on one geometry
+// work items wanted for several right-hand sides on one geometry (a slice more is a
+// partial sum more for all of them).  8 on 150 spheres p=10: 157 ms with 2048, 145 with
+// 4096, 124.5 with 8192, 120.7 with 16384.
+constexpr int64_t kMultiItems = 8192;
 constexpr size_t kJoinIntervals = 65536; // host work lists: intervals up to which parts are joined for one upload
-constexpr int kSumsInBlock = 1024; // GMRES: most chunk partials of a segment that every block adds up itself
+// GMRES: most chunk partials of a segment that every block adds up itself instead of a
+// launch of its own.  FP64 solve of 64 spheres p=8 (61 partials) 7.45 against 8.57 ms
+// with the launch; mixed solve of 1024 spheres (1014 partials) 46.3 against 46.4 ms.
+constexpr int kSumsInBlock = 1024;
 constexpr int64_t kLookaheadDof = 300000; // GMRES below this many unknowns launches one iteration ahead
 constexpr double kTuneBudget = 3.0;    // seconds per autotuning pass (SPHSTK_FLAG_AUTOTUNE)
 
@@ -447,8 +458,6 @@ Operator::Operator(int nsusp, const int *counts, const double *pos, const double
             const std::vector<int64_t> so0(susp_sph_off_.begin(), susp_sph_off_.begin() + b0 + 1),
                 po0(pt_off_.begin(), pt_off_.begin() + s0 + 1);
             const std::vector<Runs> r0(runs_fine_.begin(), runs_fine_.begin() + s0);
-            // items for eight waves per SIMD: each slice adds a partial-sum pass
-            // over all copies
             const int64_t nb = std::max<int64_t>(1, pt_off_[s0] / (64 * kMultiTPL));
             const int slices = (int)std::max<int64_t>(1, std::min<int64_t>(32, (kMultiItems + nb - 1) / nb));
             build_far_lists(lists_fine_, b0, so0, po0, po0, r0, kMultiTPL, slices, kWantItems);
@@ -670,7 +679,7 @@ static void parallel_for(int n, const std::function<void(int, int)> &body, int c
 // FMM, cpp:332-348, :408-433, :641-690).  A group's source intervals are the
 // point ranges of its spheres' runs, with a per-lane mask where the group
 // spans spheres.  Each group's list is cut into `split` slices of nearly equal
-// length, one work item each, launched in order of decreasing work.
+// length, one work item each, launched by decreasing work (upload_far_lists).
 void append_far_lists(HostLists &H, int nsusp, const std::vector<int64_t> &susp_sph_off, const std::vector<int64_t> &toff,
                      const std::vector<int64_t> &soff, const std::vector<Runs> &runs, int tpl, int split,
                      int64_t want_items, const std::vector<int64_t> *src_susp_off, ListBase at) {
@@ -933,9 +942,9 @@ static std::vector<Chunk> make_chunks(int nsusp, const std::vector<int64_t> &sus
 // (R_S + R_T), a far pair (s >= 1.5) interacts
 //   s < 3        point to point on the fine grids ("mid"),
 //   3 <= s < 6   between grids of order p/2+1 (p < 10: p) (level 0),
-//   6 <= s < 11  between grids of order max(5, p/3+1)    (level 1),
-//   11 <= s < 18 between grids of order 4                (level 2),
-//   s >= 18      between grids of order 3                (level 3),
+//   6 <= s < 9   between grids of order max(5, p/3+1)    (level 1),
+//   9 <= s < 16  between grids of order 4                (level 2),
+//   s >= 16      between grids of order 3                (level 3),
 // (orders capped by p) through the degree-truncated density of the source
 // (Resample::down) with the target-grid field interpolated back to the fine grid
 // (Resample::up).  The field of degree-n density decays like (1/(2s))^(n+2) and
@@ -1756,10 +1765,10 @@ void Operator::ensure_centre() {
 // use): the FP32 and FP64 level sets and the final-velocity lists.  The FP64
 // set is first needed by the first refinement residual, after a whole inner
 // solve, so it is built on a host thread meanwhile: its construction is host
-// work, allocations and synchronous copies (no launches on the operator's
-// non-blocking stream), and nothing else reads ls64_ until
-// outer_levels_pay() has joined the thread (16384 spheres p=12: 3.1 s of the
-// 4.5 s set-up).
+// work, allocations, synchronous copies and, on the null stream, a few launches
+// that read the geometry and write the set's own buffers (none on the operator's
+// non-blocking stream); nothing else reads ls64_ until outer_levels_pay() has
+// joined the thread.
 void Operator::prepare_mixed(bool outer_levels, bool coarse) {
     if (nsph_ == 0) return;
     if (outer_levels && !ls64_.ready && !ls64_build_.valid()) {
@@ -1776,8 +1785,7 @@ void Operator::prepare_mixed(bool outer_levels, bool coarse) {
         }
         if (coarse && !ls32_.ready && !ls32_build_.valid()) {
             // with the coarse operator first, A32 is first needed after the
-            // first coarse GMRES: its set is built beside it the same way (its
-            // one launch, the target packing, writes only ls32_'s buffers)
+            // first coarse GMRES: its set is built beside it the same way
             const int dev = device_;
             ls32_build_ = std::async(std::launch::async, [this, dev] {
                 SPHSTK_HIP(hipSetDevice(dev));
@@ -2133,7 +2141,7 @@ void Mobility::seg_norms(const double *v, std::vector<double> &out) {
     Operator &A = *A_;
     const int B = A.nsusp();
     launch_seg_dot(v, v, A.chunks(), A.nchunks(), A.scratch_partial(), nullptr, A.stream());
-    launch_seg_reduce(A.scratch_partial(), A.seg_chunk_off(), B, scal_.p, 0, nullptr, A.stream());
+    launch_seg_reduce(A.scratch_partial(), A.seg_chunk_off(), B, scal_.p, nullptr, A.stream());
     out.resize(B);
     SPHSTK_HIP(hipMemcpyAsync(out.data(), scal_.p, sizeof(double) * B, hipMemcpyDeviceToHost, A.stream()));
     SPHSTK_HIP(hipStreamSynchronize(A.stream()));
@@ -2273,10 +2281,10 @@ void Mobility::gmres(const double *b, double *x, bool x_zero, double tol, int pr
                     launch_seg_mgs(W, vp, pp[cur ^ 1], sums, hp, Vi, pp[cur], sco, ch, nch, act_.p, st);
                     vp = Vi;
                     hp = Vi ? h_.p + size_t(pass * (m + 1) + i) * B : nv;
-                    if (!sums) launch_seg_reduce(pp[cur], sco, B, hp, 0, act_.p, st);
+                    if (!sums) launch_seg_reduce(pp[cur], sco, B, hp, act_.p, st);
                 }
             }
-            if (cgs2 && !sums) launch_seg_reduce(pp[cur], sco, B, nv, 0, act_.p, st);
+            if (cgs2 && !sums) launch_seg_reduce(pp[cur], sco, B, nv, act_.p, st);
             launch_seg_normalise(W, pp[cur], sums, nv, sco, ch, nch, act_.p, st);
             launch_gmres_givens(B, j, m, h_.p, cgs2 ? -1.0 : 1.0, d_H_.p, d_cs_.p, d_sn_.p, d_g_.p, d_bn_.p, tol,
                                 act_.p, d_kdim_.p, d_impok_.p, d_relres_.p, nact_host_ + (j & 1), st);

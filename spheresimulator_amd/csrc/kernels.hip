@@ -1091,12 +1091,10 @@ __device__ __forceinline__ double wave_total(const double *__restrict__ p, int n
 // One wave per segment.  One thread per segment read its partials one after the
 // other: 743 of them at 3000 spheres p=12, 55 us.
 __global__ __launch_bounds__(64) void k_seg_reduce(const double *__restrict__ partial, const int *__restrict__ off,
-                                                   double *__restrict__ out, int op, const int *__restrict__ active) {
+                                                   double *__restrict__ out, const int *__restrict__ active) {
     const int sgi = blockIdx.x;
     if (active && !active[sgi]) return;
-    double s = wave_total(partial + off[sgi], off[sgi + 1] - off[sgi]);
-    if (op == 1) s = (s > 0.0) ? 1.0 / sqrt(s) : 0.0;
-    if (op == 2) s = -s;
+    const double s = wave_total(partial + off[sgi], off[sgi + 1] - off[sgi]);
     if (threadIdx.x == 0) out[sgi] = s;
 }
 
@@ -1259,7 +1257,6 @@ __global__ __launch_bounds__(64) void k_seg_multi_reduce(const double *__restric
     if (threadIdx.x == 0) out[(int64_t)j * nseg + sgi] = op == 2 ? -s : s;
 }
 
-// out[i] += sum_k part[k*stride + i], k = 0..nslot-1, over the DOF chunks of active segments
 // ---------------------------------------------------------------------------
 // GMRES least-squares bookkeeping on the device (Belos GMRES, one Krylov space
 // per suspension): with it a restart cycle needs no host synchronisation.
@@ -1393,6 +1390,7 @@ void launch_gmres_backsub(int B, int m, const double *H, const double *g, const 
     if (B > 0) k_gmres_backsub<<<dim3((B + 255) / 256), dim3(256), 0, s>>>(B, m, H, g, kdim, cyc, coef);
 }
 
+// out[i] += sum_k part[k*stride + i], k = 0..nslot-1, over the DOF chunks of active segments
 __global__ __launch_bounds__(256) void k_slot_reduce(double *__restrict__ out, const double *__restrict__ part,
                                                      int nslot, int64_t stride, const Chunk *__restrict__ ch,
                                                      const int *__restrict__ active) {
@@ -1425,9 +1423,9 @@ void launch_seg_dot(const double *a, const double *b, const Chunk *chunks, int n
                     const int *active, hipStream_t s) {
     if (nchunks > 0) k_seg_dot<<<dim3(nchunks), dim3(256), 0, s>>>(a, b, chunks, partial, active);
 }
-void launch_seg_reduce(const double *partial, const int *off, int nseg, double *out, int op, const int *active,
+void launch_seg_reduce(const double *partial, const int *off, int nseg, double *out, const int *active,
                        hipStream_t s) {
-    if (nseg > 0) k_seg_reduce<<<dim3(nseg), dim3(64), 0, s>>>(partial, off, out, op, active);
+    if (nseg > 0) k_seg_reduce<<<dim3(nseg), dim3(64), 0, s>>>(partial, off, out, active);
 }
 void launch_seg_axpy(double *y, const double *x, const double *alpha, double sign, const Chunk *chunks, int nchunks,
                      const int *active, hipStream_t s) {

@@ -182,9 +182,9 @@ void launch_lop(const DevGeom &g, const double *in, double *out, double cLOP, co
 // segmented BLAS-1 over chunks (one segment per suspension)
 void launch_seg_dot(const double *a, const double *b, const Chunk *chunks, int nchunks, double *partial,
                     const int *active, hipStream_t s);
-// out[seg] = sum of partials of seg; op 0: sum, 1: 1/sqrt(sum) (0 if sum==0), 2: -sum
-void launch_seg_reduce(const double *partial, const int *seg_chunk_off, int nseg, double *out, int op,
-                       const int *active, hipStream_t s);
+// out[seg] = sum of partials of seg
+void launch_seg_reduce(const double *partial, const int *seg_chunk_off, int nseg, double *out, const int *active,
+                       hipStream_t s);
 // y += sign * alpha[seg] * x
 void launch_seg_axpy(double *y, const double *x, const double *alpha, double sign, const Chunk *chunks, int nchunks,
                      const int *active, hipStream_t s);

@@ -18,11 +18,10 @@ iterate x:
                 the velocities, the iteration count (30 + the second job's)
                 and the timing of both jobs.
 
-Run on the GPU box from the repository root, in two jobs:
-  python3 tests/golden/make_cfg5_fp64_reference.py --phase cycle1 --work gpurun_out/cfg5_ref
-  python3 tests/golden/make_cfg5_fp64_reference.py --phase finish --work gpurun_out/cfg5_ref
-The second job needs the first job's files in --work (gpurun_out/ comes back
-to the caller, who carries it into the second job); it writes
+Run from the repository root on a GPU, in two jobs:
+  python3 tests/golden/make_cfg5_fp64_reference.py --phase cycle1 --work cfg5_ref
+  python3 tests/golden/make_cfg5_fp64_reference.py --phase finish --work cfg5_ref
+The second job needs the first job's files in --work; it writes
 cfg5_fp64_reference.npz there, which is committed as tests/golden/.
 """
 import argparse
