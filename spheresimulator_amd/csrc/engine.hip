@@ -1333,11 +1333,9 @@ void Operator::ensure_levels(LevelSet &S) {
                     tab.push_back(t.w[q]);
                 }
             }
-    DevBuf<double> d_tab;
-    DevBuf<int2> d_grids;
-    d_tab.upload(tab);
-    d_grids.upload(grids);
-    P.tab = d_tab.p, P.grids = d_grids.p, P.w = S.w.p;
+    S.tab.upload(tab);
+    S.grids.upload(grids);
+    P.tab = S.tab.p, P.grids = S.grids.p, P.w = S.w.p;
     launch_level_points(geom_, P, V, st0);
     SPHSTK_HIP(hipGetLastError());
     SPHSTK_HIP(hipStreamSynchronize(st0));

@@ -177,6 +177,8 @@ struct LevelSet {
     int tpl = 1;             // targets per lane of its work lists
     DevBuf<int64_t> off;              // per level: first level point of each sphere
     DevBuf<double> w;                 // weights of the points of all levels
+    DevBuf<double> tab;               // the levels' grids in the body frame (LevelPoints; kept, since
+    DevBuf<int2> grids;               // freeing them would wait for the solve beside which a set is built)
     FarLists all;                     // mid range, levels, source cells
     int mid_slots = 0;                // slots of the mid range (the fine grid's targets come first)
     DevBuf<float> src32, trg32;       // source and target records (FP32 set)

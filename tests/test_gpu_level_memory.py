@@ -1,17 +1,23 @@
 """Device memory of the multi-level far field's work lists and partial sums."""
+import ctypes
+import gc
+
 import numpy as np
 import pytest
 
-torch = pytest.importorskip("torch")
 S = pytest.importorskip("spheresimulator_amd")
 
 pytestmark = pytest.mark.gpu
 
 
 def used():
-    torch.cuda.synchronize()
-    free, total = torch.cuda.mem_get_info()
-    return total - free
+    """Device memory in use, from the HIP runtime that libsphstk.so itself links."""
+    S.load()
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipDeviceSynchronize() == 0
+    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return total.value - free.value
 
 
 def test_coarse_set_holds_each_levels_own_partial_sums():
@@ -23,7 +29,7 @@ def test_coarse_set_holds_each_levels_own_partial_sums():
     records per point, intervals (48 bytes; about 5e6) and the matrices that is below
     1.1 GB; one slot count for all lists takes the 24 to 32 of the coarsest, 1.5 to 2 GB
     for the partial sums alone."""
-    torch.zeros(1, device="cuda")
+    gc.collect()  # handles of earlier tests
     n = 4096
     c = S.configs.make_suspension(n, 12, 11, vf=0.1, min_gap=0.2)
     op = S.SphereSTKSHOperator(c["pos"], c["radius"], c["quat"], c["order"], 0.5, 0.0, 1.0, 1.0)
