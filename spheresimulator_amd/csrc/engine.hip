@@ -1457,7 +1457,6 @@ void Operator::far_run(FarLists &L, int kind, int prec, const void *src, const d
                        const double *tnorms, const float *trg32, const Chunk *chunks, int nchunks, double coef,
                        double *out, const int *active) {
     if (L.pairs == 0.0) return; // e.g. a level that no sphere pair reaches
-    if (L.split > 1) L.slots();
     double *dst = L.split > 1 ? L.part.p : out;
     const int acc = L.split > 1 ? 0 : 1;
     launch_far(kind, prec, L.tpl, src, tcoords, tnorms, trg32, L.map, L.ngroups, L.order.p, L.groups.p, L.iv.p,
@@ -1747,6 +1746,7 @@ void Operator::ensure_centre() {
             rcen[t] = runs_of(excl[t], s0, s1, false);
         }
         build_far_lists(lists_rv_mid_, nsusp_, susp_sph_off_, pt_off_, pt_off_, rmid, lists_fine_.tpl, 0, kWantItems);
+        if (lists_rv_mid_.split > 1) lists_rv_mid_.slots();
         int64_t nb = 0;
         for (int b = 0; b < nsusp_; b++) nb += (susp_sph_off_[b + 1] - susp_sph_off_[b] + 63) / 64;
         const int split = (int)std::max<int64_t>(1, std::min<int64_t>(64, (kWantItems + nb - 1) / std::max<int64_t>(nb, 1)));
